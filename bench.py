@@ -167,8 +167,9 @@ def joint_impulses_fit(max_b, max_s, max_c, max_j):
 
 def kernel_name(scene, count):
     """The step kernel a batch launches (b3_engine_create): b3k_step<JI, true>
-    for worlds of at most two shapes; else b3k_step_shared<Masks, JL> when
-    the tiles fit one per CU, b3k_step<JI, false> when they do not."""
+    for worlds of at most two shapes; else b3k_step_quad<CR, JR> up to a
+    quarter tile per CU, b3k_step_shared<Masks, JL> when the tiles fit one
+    per CU, b3k_step<JI, false> when they do not."""
     import torch
     from puffysics_amd import scenes
     tiles = (count + 63) // 64
@@ -176,6 +177,8 @@ def kernel_name(scene, count):
     caps = scenes.SCENES[scene].caps
     if caps[1] <= 2:                 # one candidate pair: b3k_step<JI, true> at any batch size
         return "b3k_step<%s, true>" % ("true" if joint_impulses_fit(*caps) else "false")
+    if 4 * tiles <= cus:             # every benchmark family fits quad_layout
+        return "b3k_step_quad<2, %d>" % (1 if caps[3] <= 8 else 2)
     if tiles > cus:
         return "b3k_step<%s, false>" % ("true" if joint_impulses_fit(*caps) else "false")
     masks = 12 <= caps[1] <= 64
@@ -518,7 +521,7 @@ def _short(name):
 def _step_kernel(names):
     """The workload's step kernel: the launched kernel named b3k_step<JI> or
     b3k_step_shared<...>."""
-    cands = [n for n in names if _short(n).startswith("b3k_step<") or _short(n).startswith("b3k_step_shared<")]
+    cands = [n for n in names if _short(n).startswith(("b3k_step<", "b3k_step_shared<", "b3k_step_quad<"))]
     if len(set(cands)) != 1:
         raise SystemExit("expected one step kernel, found %s" % sorted(set(cands)))
     return cands[0]

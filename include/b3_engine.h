@@ -128,20 +128,24 @@ hipError_t b3_engine_device_view(const B3Engine* engine, void** tiles, size_t* w
  * hipErrorNotSupported while it is on. */
 #define B3_ENGINE_ART_CONTACTS 2u
 /* B3_ENGINE_ONE_WAVE_PER_TILE: no counterpart in the reference (a launch
- * choice).  A batch of at most one 64-world tile per CU normally runs with
- * eight waves per tile: they share the narrowphase (its pairs are
- * independent; four to seven waves collide, as many as have LDS rows for
- * their clip polygons), the contact sweeps and warm start (contacts on
- * disjoint dynamic bodies, level by level, keeping every body's updates in
- * contact order), the velocity and position updates, the joint geometry
- * and, when the joint rows fit in LDS, the joint passes (by joint levels),
- * while wave 0 does the rest; contact-bound worlds split each tile over
- * `parts` = 2 or 4 such workgroups when the CUs allow.  That allocates at
- * creation a staging buffer of 4 * tiles * parts * 64 * (1 + max(40 *
- * max_shapes * (max_shapes - 1) / 2, 2 * max_contacts)) bytes.  Worlds of at
- * most two shapes (one candidate pair) always step one wave per tile.  This
- * option launches one wave per tile as for larger batches.  Results are
- * identical either way. */
+ * choice).  A batch of at most a quarter of a 64-world tile per CU normally
+ * runs with four workgroups per tile, each of eight waves that give every
+ * world four lanes each (a contact or joint solve to four lanes, everything
+ * independent within a world spread over all 32).  A batch of at most one
+ * tile per CU runs with eight waves per tile, one lane of each to a world:
+ * they share the narrowphase (its pairs are independent; four to seven
+ * waves collide, as many as have LDS rows for their clip polygons), the
+ * contact sweeps and warm start (contacts on disjoint dynamic bodies, level
+ * by level, keeping every body's updates in contact order), the velocity
+ * and position updates, the joint geometry and, when the joint rows fit in
+ * LDS, the joint passes (by joint levels), while wave 0 does the rest;
+ * contact-bound worlds split each tile over `parts` = 2 or 4 such workgroups
+ * when the CUs allow.  Both allocate at creation a staging buffer of 4 *
+ * tiles * parts * 64 * (1 + max(40 * max_shapes * (max_shapes - 1) / 2, 2 *
+ * max_contacts)) bytes (parts 1 for the first).  Worlds of at most two
+ * shapes (one candidate pair) always step one wave per tile.  This option
+ * launches one wave per tile as for larger batches.  Results are identical
+ * either way. */
 #define B3_ENGINE_ONE_WAVE_PER_TILE 4u
 hipError_t b3_engine_set_options(B3Engine* engine, unsigned int options);
 

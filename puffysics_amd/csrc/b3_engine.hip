@@ -447,6 +447,7 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
         return err;
     }
     err = b3i_forces_init();
+    if (err == hipSuccess) err = b3i_quad_init();
     if (err != hipSuccess) {
         free(e);
         return err;
@@ -485,7 +486,20 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
          * contact) leave the tile's waves nothing to share; their one-wave
          * step keeps that contact's row for the step (b3k_step<JI, true>):
          * the hover at 4,096 worlds 0.0398 ms shared, 0.0383 ms one-wave. */
-        if (e->tiles <= cus && shared_lds <= kCuLdsBytes && g.max_s > 2) {
+        size_t quad_scratch = 0;
+        /* A quarter tile per workgroup fills the CUs at a quarter tile per
+         * CU: up to there each world of three shapes or more steps on a quad
+         * of lanes of each of eight waves (b3d_quad.h).  Measured at 4,096
+         * worlds (64 tiles), the shared step -> quads: stacks 241 -> 132 us,
+         * chains 398 -> 163, bin 713 -> 467, the arm 320 -> 144 (and at 300
+         * worlds 347 -> 143).  A second round of workgroups takes as long
+         * again: at 8,192 worlds the chains and the arm would gain (404 ->
+         * 316, 334 -> 267), the others lose (stacks 208 -> 258, bin 794 ->
+         * 867), and past that all lose.  Of two-shape worlds those with a
+         * contact gain (hover 37.5 -> 30.1 us) and those without lose to the
+         * barriers (a free sphere's step and task 23.9 -> 28.1). */
+        e->quad = g.max_s > 2 && 4 * e->tiles <= cus && b3i_quad_fit(g, &quad_scratch);
+        if (e->quad || (e->tiles <= cus && shared_lds <= kCuLdsBytes && g.max_s > 2)) {
             size_t max_cand = (size_t)g.max_s * (size_t)(g.max_s - 1) / 2;
             size_t stage_words = max_cand * kStageWords;
             if ((size_t)stage_sched_words(g) > stage_words) stage_words = (size_t)stage_sched_words(g);
@@ -493,7 +507,7 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
             e->lds_shared_bytes = shared_lds;
             e->shared_masks = shared_masks(g);
             e->joint_lds = joint_lds;
-            /* Contact-bound worlds step fewer than 64 to a workgroup when the
+            /* Without quads, contact-bound worlds step fewer than 64 to a workgroup when the
              * CUs allow: the narrowphase and the sweeps then take the union
              * of fewer worlds' code paths per step of their loops, on more
              * CUs.  Worlds of many shapes (whose candidate search uses the
@@ -503,7 +517,8 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
              * (16); the stacks 0.228 -> 0.218 (32) -> 0.223 (16); the hover
              * (4 contacts, 2 joints) 0.040 -> 0.041 and the chains (32, 8)
              * 0.394 -> 0.397 -> 0.443, which stay at 64. */
-            if (e->shared_masks && 4 * e->tiles <= cus) e->tile_parts = 4;
+            if (e->quad) e->tile_parts = 1;
+            else if (e->shared_masks && 4 * e->tiles <= cus) e->tile_parts = 4;
             else if (e->shared_masks && 2 * e->tiles <= cus) e->tile_parts = 2;
             else if (g.max_c > 4 * g.max_j && 2 * e->tiles <= cus) e->tile_parts = 2;
             err = hipMalloc((void**)&e->pair_stage,
@@ -514,7 +529,9 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
             }
         }
         /* per-step scratch: one per workgroup of a tile */
-        err = hipMalloc((void**)&e->scratch, (size_t)e->tiles * e->tile_parts * g.tile_scr_words * 4);
+        size_t scratch_words = (size_t)e->tile_parts * g.tile_scr_words;
+        if (e->quad && quad_scratch > scratch_words) scratch_words = quad_scratch;
+        err = hipMalloc((void**)&e->scratch, (size_t)e->tiles * scratch_words * 4);
         if (err != hipSuccess) {
             (void)b3_engine_destroy(e);
             return err;
@@ -623,6 +640,8 @@ hipError_t b3_batch_step_gpu(B3Engine* e, float dt, int substeps, const unsigned
     if (err != hipSuccess) return err;
     if (dt == 0.0f) return reset_mask ? b3_batch_restore_gpu(e, reset_mask, stream) : hipSuccess;
     if (e->options & B3_ENGINE_ART_CONTACTS) return b3i_step_art(e, dt, substeps, step_mask, reset_mask, stream);
+    if (e->quad && !(e->options & B3_ENGINE_ONE_WAVE_PER_TILE))
+        return b3i_step_quad(e, dt, substeps, step_mask, reset_mask, stream);
     if (e->pair_stage && !(e->options & B3_ENGINE_ONE_WAVE_PER_TILE)) {
         auto kernel = e->shared_masks ? (e->joint_lds ? b3k_step_shared<true, true> : b3k_step_shared<true, false>)
                                       : (e->joint_lds ? b3k_step_shared<false, true> : b3k_step_shared<false, false>);

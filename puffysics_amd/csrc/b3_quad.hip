@@ -1,0 +1,87 @@
+/*
+ * b3_quad.hip - the step on four lanes of each wave per world (b3d_quad.h)
+ * for batches that leave compute units idle at one lane per world.
+ */
+#include "b3d_quad.h"
+
+#include <hip/hip_runtime.h>
+
+#include "b3_engine.h"
+#include "b3_engine_internal.h"
+
+using namespace b3d;
+
+namespace {
+
+/* b3k_step on quads.  Bound by each world's chain of solves: at one lane a
+ * world a chain of eight hinges (4,096 worlds) took 391 us, 292 of them in
+ * 160 levels of joint solves at 1.83 us (a solve's ~400 instructions and
+ * ~90 row loads at ~5 cycles each, a wave alone on its SIMD); on quads with
+ * the rows in registers 163 us.  CR, JR: contacts and joints of a world
+ * that a wave keeps in registers. */
+template <int CR, int JR>
+__global__ __launch_bounds__(64 * kQuadWaves) void b3k_step_quad(uint32_t* live, const uint32_t* snap,
+        uint32_t* scratch, uint32_t* stage, size_t stage_tile_words, Geometry g, QuadLayout q, int count, float dt,
+        int substeps, const unsigned char* step_mask, const unsigned char* reset_mask, unsigned int opts) {
+    extern __shared__ float lds[];
+    int* wg = reinterpret_cast<int*>(lds);
+    int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63u);
+    int tile = (int)(blockIdx.x >> 2), part = (int)(blockIdx.x & 3u);
+    int col = lane >> 2, slot = part * kQuadCols + col;
+    if (reset_mask) {
+        uint64_t mine = ((1ull << kQuadCols) - 1) << (part * kQuadCols);
+        restore_tile(live, snap, g, count, reset_mask, tile, wave, kQuadWaves, mine);
+    }
+    int w = tile * 64 + slot;
+    bool stepping = w < count && (!step_mask || step_mask[w]);
+    /* every wave holds the same worlds, so the workgroup returns as a whole */
+    if (!(dt > 0.0f) || __ballot(stepping) == 0) return;
+    QLane Q;
+    Q.sub = lane & 3;
+    Q.wave = wave;
+    Q.worker = wave * 4 + Q.sub;
+    Q.q = q;
+    Q.lds = lds + kQuadWgWords + col;
+    uint32_t* tile_scratch = scratch + (size_t)tile * q.scratch_tile_words;
+    Q.recs = tile_scratch + (size_t)g.scr_words * kLanes + (size_t)slot * g.max_c * kQRecWords;
+    Q.st = PairStage{};
+    Q.st.p = stage + (size_t)tile * stage_tile_words + slot;
+    Q.L = lane_view(live, nullptr, nullptr, g, tile, slot, opts);
+    Q.L.scr = tile_scratch + slot;
+    Q.L.sq = reinterpret_cast<uint32_t*>(Q.lds);
+    Q.L.vel = Q.lds + q.y * kRow;
+    Q.L.active = stepping;
+    if (threadIdx.x < kQuadWgWords) wg[threadIdx.x] = 0;
+    for (int k = Q.worker; k <= hit_words(g); k += kQuadWorkers) lseti(Q, q.hits + k, 0);
+    __syncthreads();
+    quad_step<CR, JR>(Q, dt, substeps, wg);
+}
+
+/* Contacts of a world a wave keeps in registers. */
+constexpr int kKeptContacts = 2;
+
+}  // namespace
+
+bool b3i_quad_fit(const Geometry& g, size_t* scratch_tile_words) {
+    QuadLayout q;
+    if (!quad_layout(g, 2 * kQuadWaves, &q)) return false;
+    *scratch_tile_words = q.scratch_tile_words;
+    return true;
+}
+
+hipError_t b3i_quad_init() {
+    hipError_t err = b3i_lds_limit((const void*)b3k_step_quad<kKeptContacts, 1>);
+    if (err == hipSuccess) err = b3i_lds_limit((const void*)b3k_step_quad<kKeptContacts, 2>);
+    return err;
+}
+
+hipError_t b3i_step_quad(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
+        const unsigned char* reset_mask, hipStream_t stream) {
+    QuadLayout q;
+    if (!quad_layout(e->g, 2 * kQuadWaves, &q)) return hipErrorInvalidValue;
+    auto kernel = e->g.max_j <= kQuadWaves ? b3k_step_quad<kKeptContacts, 1> : b3k_step_quad<kKeptContacts, 2>;
+    size_t lds = ((size_t)kQuadWgWords + (size_t)q.words * kQuadCols) * sizeof(float);
+    kernel<<<e->tiles * 4, 64 * kQuadWaves, lds, stream>>>(e->live, e->snap, e->scratch, e->pair_stage,
+        e->stage_tile_words, e->g, q, e->count, dt, substeps, step_mask, reset_mask, e->options);
+    return hipGetLastError();
+}

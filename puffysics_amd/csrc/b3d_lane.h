@@ -46,7 +46,11 @@
 namespace b3d {
 
 constexpr int kLanes = B3D_LANES;
-constexpr int kVelWords = 7;
+constexpr int kRow = B3D_ROW;   /* stride of the LDS rows */
+/* Velocity row of a body: linear, angular, flags.  With four lanes to a
+ * world (B3D_QUAD) lane 0..2 of a quad reads a component and lane 3 a pad
+ * word, so both vectors take four words and the flags live elsewhere. */
+constexpr int kVelWords = B3D_QUAD ? 8 : 7, kVelAng = B3D_QUAD ? 4 : 3;
 
 /* ---- word offsets of the B3 structs ---- */
 #define B3D_W(T, f) ((int)(offsetof(T, f) / 4))
@@ -207,9 +211,10 @@ constexpr int SS_P = 0, SS_RADIUS = 3, SS_Q = 4, SS_HALF = 8, SS_TYPE = 11, SS_C
               SS_ROLLING = 23, kShapeRows = 6;
 constexpr int kBodyStatic = 1, kBodyDynamic = 2;   /* SS_BFLAGS bits */
 /* Loops over bodies, shapes and contacts run in chunks, every load of a
- * chunk issued before any of its results is used. */
-constexpr int kChunk = 4;
-constexpr int kShapeChunk = 4;
+ * chunk issued before any of its results is used (with as many workers to a
+ * world as B3D_QUAD gives, one item each covers most worlds). */
+constexpr int kChunk = B3D_QUAD ? 1 : 4;
+constexpr int kShapeChunk = B3D_QUAD ? 1 : 4;
 /* Per-step body records: the velocity increments of 09_step.inl:5-18 (all
  * their inputs are fixed for the step) and the damping factors (BS_*); the
  * delta pose, which the step keeps here and commits in finalize, and the
@@ -536,11 +541,13 @@ template <bool S>
 B3D_FN V3 q3s(const uint32_t* r, int k) { return v3(qfs<S>(r, k), qfs<S>(r, k + 1), qfs<S>(r, k + 2)); }
 
 /* ---- packed word rows (word k of a record at quad row k / 4, word row
- * k % 4 of it; slot s at column s) ---- */
-B3D_FN float rf(const uint32_t* r, int k) { return __builtin_bit_cast(float, r[(k >> 2) * kRowWords + (k & 3) * kLanes]); }
-B3D_FN uint32_t ru(const uint32_t* r, int k) { return r[(k >> 2) * kRowWords + (k & 3) * kLanes]; }
-B3D_FN void rsf(uint32_t* r, int k, float v) { r[(k >> 2) * kRowWords + (k & 3) * kLanes] = __builtin_bit_cast(uint32_t, v); }
-B3D_FN void rsu(uint32_t* r, int k, uint32_t v) { r[(k >> 2) * kRowWords + (k & 3) * kLanes] = v; }
+ * k % 4 of it; slot s at column s).  B3D_QUAD: the records are LDS rows,
+ * word k at row k. ---- */
+B3D_FN int row_word(int k) { return B3D_QUAD ? k * kRow : (k >> 2) * kRowWords + (k & 3) * kLanes; }
+B3D_FN float rf(const uint32_t* r, int k) { return __builtin_bit_cast(float, r[row_word(k)]); }
+B3D_FN uint32_t ru(const uint32_t* r, int k) { return r[row_word(k)]; }
+B3D_FN void rsf(uint32_t* r, int k, float v) { r[row_word(k)] = __builtin_bit_cast(uint32_t, v); }
+B3D_FN void rsu(uint32_t* r, int k, uint32_t v) { r[row_word(k)] = v; }
 B3D_FN V3 r3(const uint32_t* r, int k) { return v3(rf(r, k), rf(r, k + 1), rf(r, k + 2)); }
 B3D_FN void rs3(uint32_t* r, int k, V3 v) { rsf(r, k, v.x); rsf(r, k + 1, v.y); rsf(r, k + 2, v.z); }
 B3D_FN Q rq4(const uint32_t* r, int k) { return q4(rf(r, k), rf(r, k + 1), rf(r, k + 2), rf(r, k + 3)); }
@@ -556,12 +563,24 @@ B3D_FN int jw(const Lane& L, int j, int f) { return L.g.jo + j * kJointWords + f
 B3D_FN int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
 /* ---- body velocity rows ---- */
-B3D_FN V3 vlin(const Lane& L, int b) { const float* v = L.vel + b * kVelWords * kLanes; return v3(v[0], v[kLanes], v[2 * kLanes]); }
-B3D_FN V3 vang(const Lane& L, int b) { const float* v = L.vel + (b * kVelWords + 3) * kLanes; return v3(v[0], v[kLanes], v[2 * kLanes]); }
-B3D_FN void set_vlin(const Lane& L, int b, V3 x) { float* v = L.vel + b * kVelWords * kLanes; v[0] = x.x; v[kLanes] = x.y; v[2 * kLanes] = x.z; }
-B3D_FN void set_vang(const Lane& L, int b, V3 x) { float* v = L.vel + (b * kVelWords + 3) * kLanes; v[0] = x.x; v[kLanes] = x.y; v[2 * kLanes] = x.z; }
+B3D_FN V3 vlin(const Lane& L, int b) { const float* v = L.vel + b * kVelWords * kRow; return v3(v[0], v[kRow], v[2 * kRow]); }
+B3D_FN V3 vang(const Lane& L, int b) { const float* v = L.vel + (b * kVelWords + kVelAng) * kRow; return v3(v[0], v[kRow], v[2 * kRow]); }
+B3D_FN void set_vlin(const Lane& L, int b, V3 x) { float* v = L.vel + b * kVelWords * kRow; v[0] = x.x; v[kRow] = x.y; v[2 * kRow] = x.z; }
+B3D_FN void set_vang(const Lane& L, int b, V3 x) { float* v = L.vel + (b * kVelWords + kVelAng) * kRow; v[0] = x.x; v[kRow] = x.y; v[2 * kRow] = x.z; }
+#if B3D_QUAD
+/* LDS rows of a world past its velocities: the bodies' flags, delta-pose
+ * and increment records (kDeltaRows, kBodyRows quads of words each); then,
+ * while contacts are generated, the shape records are where L.sq points. */
+B3D_FN int quad_flags_word(const Geometry& g) { return g.max_b * kVelWords; }
+B3D_FN int quad_delta_word(const Geometry& g) { return g.max_b * (kVelWords + 1); }
+B3D_FN int quad_body_word(const Geometry& g) { return g.max_b * (kVelWords + 1 + 4 * kDeltaRows); }
+B3D_FN int quad_body_rows(const Geometry& g) { return g.max_b * (kVelWords + 1 + 4 * kDeltaRows + 4 * kBodyRows); }
+B3D_FN float* vel_flags(const Lane& L, int b) { return L.vel + (quad_flags_word(L.g) + b) * kRow; }
+#else
+B3D_FN float* vel_flags(const Lane& L, int b) { return L.vel + (b * kVelWords + 6) * kRow; }
+#endif
 B3D_FN int is_dyn_flag(const Lane& L, int b) {
-    return (__builtin_bit_cast(uint32_t, L.vel[(b * kVelWords + 6) * kLanes]) & kFlagDynamic) != 0;
+    return (__builtin_bit_cast(uint32_t, *vel_flags(L, b)) & kFlagDynamic) != 0;
 }
 
 B3D_FN int body_count(const Lane& L) { return L.counted ? L.nb : clampi(ldi(L.w, H_BODY_COUNT), 0, L.g.max_b); }
@@ -588,8 +607,8 @@ B3D_FN void count_contacts(Lane& L) {
 B3D_FN void vel_store(const Lane& L, int first = 0, int stride = 1) {
     int nb = body_count(L);
     for (int b = first; b < nb; b += stride) {
-        const float* v = L.vel + b * kVelWords * kLanes;
-        for (int c = 0; c < 6; c++) stf(L.w, bw(L, b, B_LIN_VEL + c), v[c * kLanes]);
+        const float* v = L.vel + b * kVelWords * kRow;
+        for (int c = 0; c < 6; c++) stf(L.w, bw(L, b, B_LIN_VEL + c), v[(c < 3 ? c : kVelAng + c - 3) * kRow]);
     }
 }
 
@@ -631,6 +650,7 @@ B3D_FN void shape_aabb(const Posed& P, V3* lo, V3* hi) {
 }
 
 B3D_FN uint32_t* shape_rec(const Lane& L, int s) {
+    if (B3D_QUAD) return L.sq + s * 4 * kShapeRows * kRow;
     return L.sq + (size_t)(L.g.q_shape + s * kShapeRows) * kRowWords + L.sslot;
 }
 B3D_FN uint32_t* old_rec(const Lane& L, int k) { return L.scr + (L.g.scr_old + k * kOldWords) * kLanes; }
@@ -781,9 +801,15 @@ B3D_FN V3 jimp_ld3(const Lane& L, int j, int world_word) {
 }
 
 B3D_FN uint32_t* body_rec(const Lane& L, int b) {
+#if B3D_QUAD
+    return (uint32_t*)L.vel + (quad_body_word(L.g) + b * 4 * kBodyRows) * kRow;
+#endif
     return L.sq + (size_t)(L.g.q_body + b * kBodyRows) * kRowWords + L.sslot;
 }
 B3D_FN uint32_t* delta_rec(const Lane& L, int b) {
+#if B3D_QUAD
+    return (uint32_t*)L.vel + (quad_delta_word(L.g) + b * 4 * kDeltaRows) * kRow;
+#endif
     return L.sq + (size_t)(L.g.q_delta + b * kDeltaRows) * kRowWords + L.sslot;
 }
 B3D_FN uint32_t pair_key(int a, int b) { return a < b ? ((uint32_t)a << 16) | (uint32_t)b : ((uint32_t)b << 16) | (uint32_t)a; }
@@ -860,14 +886,14 @@ B3D_FN void shape_pass(const Lane& L, int ns, float* bounds, int first = 0, int 
             rsf(r, SS_FRICTION, mat[k][0]);
             rsf(r, SS_RESTITUTION, mat[k][1]);
             rsf(r, SS_ROLLING, mat[k][2]);
-            float* bd = bounds + s * 6 * kLanes;
+            float* bd = bounds + s * 6 * kRow;
             V3 l = sub(lo, pad), h = add(hi, pad);
             bd[0] = l.x;
-            bd[kLanes] = l.y;
-            bd[2 * kLanes] = l.z;
-            bd[3 * kLanes] = h.x;
-            bd[4 * kLanes] = h.y;
-            bd[5 * kLanes] = h.z;
+            bd[kRow] = l.y;
+            bd[2 * kRow] = l.z;
+            bd[3 * kRow] = h.x;
+            bd[4 * kRow] = h.y;
+            bd[5 * kRow] = h.z;
         }
     }
 }
@@ -1022,7 +1048,7 @@ struct NewContact {
  * turn). */
 struct Box6 { float lx, ly, lz, hx, hy, hz; };
 B3D_FN Box6 box_load(const float* b) {
-    return Box6{b[0], b[kLanes], b[2 * kLanes], b[3 * kLanes], b[4 * kLanes], b[5 * kLanes]};
+    return Box6{b[0], b[kRow], b[2 * kRow], b[3 * kRow], b[4 * kRow], b[5 * kRow]};
 }
 B3D_FN bool box_overlap(const Box6& a, const Box6& b) {
     return (a.lx <= b.hx) & (a.hx >= b.lx) & (a.ly <= b.hy) & (a.hy >= b.ly) & (a.lz <= b.hz) & (a.hz >= b.lz);
@@ -1307,12 +1333,11 @@ B3D_FN void pair_share(const Lane& L, const PairStage& S, bool masks, int ncand,
     }
 }
 
-/* Contact cc of the step from candidate pair (i, j)'s manifold m: its
- * anchors and base separations, the warm start from the matching old
- * contact, the world's contact row and the head for prepare_contacts
- * (08:140-170, b3_contact_from_mani 08:5-39).  Returns the CF_* flags. */
-B3D_FN int write_new_contact(const Lane& L, int cc, int i, int j, const PairShape& A, const PairShape& B,
-        const Mani& m, int sorted, int match, const OldWarm& orec, int old_n) {
+/* The contact of candidate pair (i, j) from its manifold m: its anchors and
+ * base separations, and the warm start from the matching old contact
+ * (08:140-170, b3_contact_from_mani 08:5-39). */
+B3D_FN NewContact new_contact(const Lane& L, int i, int j, const PairShape& A, const PairShape& B, const Mani& m,
+        int sorted, int match, const OldWarm& orec, int old_n) {
     NewContact nc;
     nc.count = m.count;
     nc.normal = m.normal;
@@ -1344,6 +1369,13 @@ B3D_FN int write_new_contact(const Lane& L, int cc, int i, int j, const PairShap
             }
         }
     }
+    return nc;
+}
+
+/* Contact cc of the step to the world's contact row.  Returns the CF_*
+ * flags. */
+B3D_FN int store_new_contact(const Lane& L, int cc, int i, int j, const PairShape& A, const PairShape& B,
+        const NewContact& nc) {
     uint32_t* w = L.w;
     sti(w, cw(L, cc, C_SHAPE_A), i);
     sti(w, cw(L, cc, C_SHAPE_B), j);
@@ -1371,13 +1403,22 @@ B3D_FN int write_new_contact(const Lane& L, int cc, int i, int j, const PairShap
     int info = (A.bflags & kBodyDynamic ? CF_DYN_A : 0) | (B.bflags & kBodyDynamic ? CF_DYN_B : 0)
         | (!((A.bflags & B.bflags) & kBodyDynamic) ? CF_STATIC : 0) | (restitution != 0.0f ? CF_RESTITUTION : 0)
         | (!(rolling <= 0.0f) ? CF_ROLLING : 0);
-    uint32_t* hd = chead_rec(L, cc);
-    sti(hd, CH_AB, A.body | (B.body << 16));
-    sti(hd, CH_INFO, nc.count | (info << 8));
     stf(w, cw(L, cc, C_TWIST_IMPULSE), nc.twist);
     stf(w, cw(L, cc, C_FRICTION_IMPULSE), nc.fi.x);
     stf(w, cw(L, cc, C_FRICTION_IMPULSE + 1), nc.fi.y);
     st3(w, cw(L, cc, C_ROLLING_IMPULSE), nc.roll);
+    return info;
+}
+
+/* Contact cc of the step from candidate pair (i, j)'s manifold: the world's
+ * contact row and the head for prepare_contacts.  Returns the CF_* flags. */
+B3D_FN int write_new_contact(const Lane& L, int cc, int i, int j, const PairShape& A, const PairShape& B,
+        const Mani& m, int sorted, int match, const OldWarm& orec, int old_n) {
+    NewContact nc = new_contact(L, i, j, A, B, m, sorted, match, orec, old_n);
+    int info = store_new_contact(L, cc, i, j, A, B, nc);
+    uint32_t* hd = chead_rec(L, cc);
+    sti(hd, CH_AB, A.body | (B.body << 16));
+    sti(hd, CH_INFO, nc.count | (info << 8));
     return info;
 }
 
@@ -1696,11 +1737,101 @@ B3D_FN int tile_levels(const Lane& L) {
     return m;
 }
 
-constexpr int kPrepChunk = 2;
+/* The prepared values of one contact (b3_prepare_one_contact, 08:234-291);
+ * the per-point values are zero past its count. */
+struct ContactPrep {
+    float rel_vel[kMaxManifold], nmass[kMaxManifold], lever[kMaxManifold], base_sep[kMaxManifold], ni[kMaxManifold];
+    V3 center_a, center_b;
+    M2 tmass;
+    float twist_mass;
+};
+B3D_FN ContactPrep contact_prep(int pc, V3 n, V3 t1, const V3* ra, const V3* rb, const float* bs, const float* ni,
+        float ma, float mb, M3 ia, M3 ib, int need_rv, V3 va, V3 wa, V3 vb, V3 wb) {
+    const float inv_tau = 1.0f / kSpeculative;
+    ContactPrep o;
+    /* tangent2 = tangent1 x normal as written by b3_contact_from_mani */
+    V3 t2 = cross(t1, n);
+    V3 center_a = zero3(), center_b = zero3();
+    float wsum = 0.0f;
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        o.rel_vel[p] = 0.0f;
+        o.nmass[p] = 0.0f;
+        o.base_sep[p] = 0.0f;
+        o.ni[p] = 0.0f;
+        if (p >= pc) continue;
+        V3 rap = ra[p], rbp = rb[p];
+        V3 rn_a = cross(rap, n);
+        V3 rn_b = cross(rbp, n);
+        float kn = ma + mb + dot(rn_a, mv(ia, rn_a)) + dot(rn_b, mv(ib, rn_b));
+        o.nmass[p] = kn > 0.0f ? 1.0f / kn : 0.0f;
+        if (need_rv) {
+            V3 vra = add(va, cross(wa, rap));
+            V3 vrb = add(vb, cross(wb, rbp));
+            o.rel_vel[p] = dot(n, sub(vrb, vra));
+        }
+        float sep = bs[p] + dot(sub(rbp, rap), n);
+        float weight = clampf(2.0f - sep * inv_tau, kMinFrictionW, 1.0f);
+        center_a = madd(center_a, weight, rap);
+        center_b = madd(center_b, weight, rbp);
+        wsum += weight;
+        o.base_sep[p] = bs[p];
+        o.ni[p] = ni[p];
+    }
+    float invw = wsum > 0.0f ? 1.0f / wsum : 0.0f;
+    center_a = scale(center_a, invw);
+    center_b = scale(center_b, invw);
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        o.lever[p] = 0.0f;
+        if (p < pc) o.lever[p] = len(sub(ra[p], center_a));
+    }
+    V3 rt_a1 = cross(center_a, t1);
+    V3 rt_a2 = cross(center_a, t2);
+    V3 rt_b1 = cross(center_b, t1);
+    V3 rt_b2 = cross(center_b, t2);
+    M2 k2;
+    k2.cx.x = ma + mb + dot(rt_a1, mv(ia, rt_a1)) + dot(rt_b1, mv(ib, rt_b1));
+    k2.cy.y = ma + mb + dot(rt_a2, mv(ia, rt_a2)) + dot(rt_b2, mv(ib, rt_b2));
+    k2.cx.y = dot(rt_a1, mv(ia, rt_a2)) + dot(rt_b1, mv(ib, rt_b2));
+    k2.cy.x = k2.cx.y;
+    o.tmass = inv2(k2);
+    float kt = dot(n, mv(madd3(ia, ib), n));
+    o.twist_mass = kt > 0.0f ? 1.0f / kt : 0.0f;
+    o.center_a = center_a;
+    o.center_b = center_b;
+    return o;
+}
+/* kKeepSolverFields: the prepared values to the world's contact row. */
+B3D_FN void keep_solver_fields(const Lane& L, int c, int pc, const ContactPrep& p, float ma, float mb, M3 ia, M3 ib,
+        Soft soft) {
+    uint32_t* w = L.w;
+#pragma unroll
+    for (int q = 0; q < kMaxManifold; q++) {
+        if (q >= pc) continue;
+        stf(w, pw(L, c, q, P_NORMAL_MASS), p.nmass[q]);
+        stf(w, pw(L, c, q, P_REL_VEL), p.rel_vel[q]);
+        stf(w, pw(L, c, q, P_LEVER), p.lever[q]);
+    }
+    st3(w, cw(L, c, C_CENTER_A), p.center_a);
+    st3(w, cw(L, c, C_CENTER_B), p.center_b);
+    stf(w, cw(L, c, C_TWIST_MASS), p.twist_mass);
+    stf(w, cw(L, c, C_TANGENT_MASS), p.tmass.cx.x);
+    stf(w, cw(L, c, C_TANGENT_MASS + 1), p.tmass.cx.y);
+    stf(w, cw(L, c, C_TANGENT_MASS + 2), p.tmass.cy.x);
+    stf(w, cw(L, c, C_TANGENT_MASS + 3), p.tmass.cy.y);
+    stm3(w, cw(L, c, C_ROLLING_MASS), inv3(madd3(ia, ib)));
+    stf(w, cw(L, c, C_INV_MASS_A), ma);
+    stf(w, cw(L, c, C_INV_MASS_B), mb);
+    stm3(w, cw(L, c, C_INV_I_A), ia);
+    stm3(w, cw(L, c, C_INV_I_B), ib);
+    stsoft(w, cw(L, c, C_SOFTNESS), soft);
+}
+
+constexpr int kPrepChunk = B3D_QUAD ? 1 : 2;
 B3D_FN int prepare_contacts(const Lane& L, Soft cs, Soft ss, int first = 0, int stride = 1) {
     uint32_t* w = L.w;
     int cc = contact_count_word(L);
-    const float inv_tau = 1.0f / kSpeculative;
     const int keep = (L.opts & kKeepSolverFields) != 0;
     /* a shared tile prepares its contacts in parallel (chunks first,
      * first + stride, ... per wave) and warm-starts them afterwards, level
@@ -1790,97 +1921,35 @@ B3D_FN int prepare_contacts(const Lane& L, Soft cs, Soft ss, int first = 0, int 
                 vb = vlin(L, b[k]);
                 wb = vang(L, b[k]);
             }
-            /* tangent2 = tangent1 x normal as written by b3_contact_from_mani */
+            ContactPrep o = contact_prep(pc[k], n[k], t1[k], ra[k], rb[k], bs[k], ni[k], ma, mb, ia, ib, need_rv, va,
+                wa, vb, wb);
             V3 t2 = cross(t1[k], n[k]);
-            V3 center_a = zero3(), center_b = zero3();
-            float wsum = 0.0f;
-            float rel_vel[kMaxManifold], nmass[kMaxManifold], bsp[kMaxManifold],
-                nip[kMaxManifold];
-#pragma unroll
-            for (int p = 0; p < kMaxManifold; p++) {
-                rel_vel[p] = 0.0f;
-                nmass[p] = 0.0f;
-                bsp[p] = 0.0f;
-                nip[p] = 0.0f;
-                if (p >= pc[k]) continue;
-                V3 rap = ra[k][p], rbp = rb[k][p];
-                V3 rn_a = cross(rap, n[k]);
-                V3 rn_b = cross(rbp, n[k]);
-                float kn = ma + mb + dot(rn_a, mv(ia, rn_a)) + dot(rn_b, mv(ib, rn_b));
-                nmass[p] = kn > 0.0f ? 1.0f / kn : 0.0f;
-                if (need_rv) {
-                    V3 vra = add(va, cross(wa, rap));
-                    V3 vrb = add(vb, cross(wb, rbp));
-                    rel_vel[p] = dot(n[k], sub(vrb, vra));
-                }
-                float sep = bs[k][p] + dot(sub(rbp, rap), n[k]);
-                float weight = clampf(2.0f - sep * inv_tau, kMinFrictionW, 1.0f);
-                center_a = madd(center_a, weight, rap);
-                center_b = madd(center_b, weight, rbp);
-                wsum += weight;
-                bsp[p] = bs[k][p];
-                nip[p] = ni[k][p];
-            }
-            float invw = wsum > 0.0f ? 1.0f / wsum : 0.0f;
-            center_a = scale(center_a, invw);
-            center_b = scale(center_b, invw);
+            V3 center_a = o.center_a, center_b = o.center_b;
 #pragma unroll
             for (int p = 0; p < kMaxManifold; p++) {
                 if (p >= pc[k]) continue;
-                float lever = len(sub(ra[k][p], center_a));
                 uint32_t* pr = prec(L, c, p, pslot[k][p]);
                 qs3(pr, PR_RA, ra[k][p]);
-                qsf(pr, PR_NMASS, nmass[p]);
+                qsf(pr, PR_NMASS, o.nmass[p]);
                 qs3(pr, PR_RB, rb[k][p]);
-                qsf(pr, PR_LEVER, lever);
-                if (L.opts & kKeepSolverFields) {
-                    stf(w, pw(L, c, p, P_NORMAL_MASS), nmass[p]);
-                    stf(w, pw(L, c, p, P_REL_VEL), rel_vel[p]);
-                    stf(w, pw(L, c, p, P_LEVER), lever);
-                }
+                qsf(pr, PR_LEVER, o.lever[p]);
             }
-            V3 rt_a1 = cross(center_a, t1[k]);
-            V3 rt_a2 = cross(center_a, t2);
-            V3 rt_b1 = cross(center_b, t1[k]);
-            V3 rt_b2 = cross(center_b, t2);
-            M2 k2;
-            k2.cx.x = ma + mb + dot(rt_a1, mv(ia, rt_a1)) + dot(rt_b1, mv(ib, rt_b1));
-            k2.cy.y = ma + mb + dot(rt_a2, mv(ia, rt_a2)) + dot(rt_b2, mv(ib, rt_b2));
-            k2.cx.y = dot(rt_a1, mv(ia, rt_a2)) + dot(rt_b1, mv(ib, rt_b2));
-            k2.cy.x = k2.cx.y;
-            M2 tmass = inv2(k2);
-            M3 isum = madd3(ia, ib);
-            float kt = dot(n[k], mv(isum, n[k]));
-            float twist_mass = kt > 0.0f ? 1.0f / kt : 0.0f;
-            if (L.opts & kKeepSolverFields) {
-                st3(w, cw(L, c, C_CENTER_A), center_a);
-                st3(w, cw(L, c, C_CENTER_B), center_b);
-                stf(w, cw(L, c, C_TWIST_MASS), twist_mass);
-                stf(w, cw(L, c, C_TANGENT_MASS), tmass.cx.x);
-                stf(w, cw(L, c, C_TANGENT_MASS + 1), tmass.cx.y);
-                stf(w, cw(L, c, C_TANGENT_MASS + 2), tmass.cy.x);
-                stf(w, cw(L, c, C_TANGENT_MASS + 3), tmass.cy.y);
-                stm3(w, cw(L, c, C_ROLLING_MASS), inv3(isum));
-                stf(w, cw(L, c, C_INV_MASS_A), ma);
-                stf(w, cw(L, c, C_INV_MASS_B), mb);
-                stm3(w, cw(L, c, C_INV_I_A), ia);
-                stm3(w, cw(L, c, C_INV_I_B), ib);
-                stsoft(w, cw(L, c, C_SOFTNESS), (fl[k] & CF_STATIC) ? ss : cs);
-            }
+            if (L.opts & kKeepSolverFields)
+                keep_solver_fields(L, c, pc[k], o, ma, mb, ia, ib, (fl[k] & CF_STATIC) ? ss : cs);
             /* the packed record */
             qsu(r, R_AB, (uint32_t)(a[k] | (b[k] << 16)));
             qsu(r, R_INFO, (uint32_t)(pc[k] | ((fl[k] | fixed[k]) << 8)));
             qsf(r, R_FRICTION, fric[k]);
-            qsf(r, R_TWIST_MASS, twist_mass);
+            qsf(r, R_TWIST_MASS, o.twist_mass);
             qs3(r, R_N, n[k]);
             qsf(r, R_ROLLING, roll_c[k]);
             rec_store_masses(r, fl[k], ma, ia, mb, ib);
             qs3(r, R_T1, t1[k]);
-            qsf(r, R_TM_XX, tmass.cx.x);
+            qsf(r, R_TM_XX, o.tmass.cx.x);
             qs3(r, R_CA, center_a);
-            qsf(r, R_TM_XY, tmass.cx.y);
+            qsf(r, R_TM_XY, o.tmass.cx.y);
             qs3(r, R_CB, center_b);
-            qsf(r, R_TM_YY, tmass.cy.y);
+            qsf(r, R_TM_YY, o.tmass.cy.y);
             qsf(r, R_FI, fi[k].x);
             qsf(r, R_FI + 1, fi[k].y);
             qsf(r, R_TWIST, tw[k]);
@@ -1888,21 +1957,21 @@ B3D_FN int prepare_contacts(const Lane& L, Soft cs, Soft ss, int first = 0, int 
             qs3(r, R_ROLL, roll[k]);
             if (fl[k] & CF_RESTITUTION) {
 #pragma unroll
-                for (int p = 0; p < kMaxManifold; p++) qsf(r, R_REL_VEL + p, rel_vel[p]);
+                for (int p = 0; p < kMaxManifold; p++) qsf(r, R_REL_VEL + p, o.rel_vel[p]);
             }
 #pragma unroll
             for (int p = 0; p < kMaxManifold; p++) {
-                qsf(r, R_BASE_SEP + p, bsp[p]);
+                qsf(r, R_BASE_SEP + p, o.base_sep[p]);
             }
 #pragma unroll
             for (int p = 0; p < 2; p++) {
-                qsf(r, R_NI + 2 * p, nip[p]);
+                qsf(r, R_NI + 2 * p, o.ni[p]);
                 qsf(r, R_TN + 2 * p, 0.0f);
             }
             if (pc[k] > 2) {
 #pragma unroll
                 for (int p = 2; p < kMaxManifold; p++) {
-                    qsf(r, R_NI + 2 * p, nip[p]);
+                    qsf(r, R_NI + 2 * p, o.ni[p]);
                     qsf(r, R_TN + 2 * p, 0.0f);
                 }
             }
@@ -1911,7 +1980,7 @@ B3D_FN int prepare_contacts(const Lane& L, Soft cs, Soft ss, int first = 0, int 
 #pragma unroll
                 for (int p = 0; p < kMaxManifold; p++) {
                     if (p >= pc[k]) continue;
-                    V3 P = scale(n[k], nip[p]);
+                    V3 P = scale(n[k], o.ni[p]);
                     apply_impulse(L, a[k], ma, ia, ra[k][p], P, -1.0f);
                     apply_impulse(L, b[k], mb, ib, rb[k][p], P, 1.0f);
                 }
@@ -2240,6 +2309,48 @@ B3D_FN void joint_geometry(const Lane& L, int first = 0, int stride = 1);
  * are computed by each solve from the bodies' delta poses. */
 B3D_FN void delta_geometry(const Lane& L) { joint_geometry(L); }
 
+/* What a joint's rows need from its bodies' delta poses (see JS_*). */
+struct JGeo { V3 ra, rb, psep, px, py, cv; M3 pki; float kxx, kxy, kyy, kinv, relx, rely, tw; };
+B3D_FN JGeo joint_geo(int info, Q dqa, Q dqb, V3 dpa, V3 dpb, Q fqa, Q fqb, V3 fpa, V3 fpb, V3 dcen, float ma,
+        float mb, M3 ia, M3 ib) {
+    JGeo o;
+    Q qa = qmul(dqa, fqa);
+    Q qb = qmul(dqb, fqb);
+    if (qdot(qa, qb) < 0.0f) qb = qneg(qb);
+    Q rel = qinv_mul(qa, qb);
+    o.ra = rot(dqa, fpa);
+    o.rb = rot(dqb, fpb);
+    o.psep = add(add(sub(dpb, dpa), sub(o.rb, o.ra)), dcen);
+    /* the point rows' matrix as b3_solve3 inverts it in every solve
+     * (06:241-255, 03_math.inl:343-345) */
+    o.pki = inv3(point_k(ma, mb, ia, ib, o.ra, o.rb));
+    int fixed = info & JF_FIXED;
+    if (info & JF_WELD) {
+        if (fixed) return o;
+        Q sq = rel;
+        if (rel.s < 0.0f) sq = qneg(rel);
+        Q diff = q4(-sq.v.x, -sq.v.y, -sq.v.z, 1.0f - sq.s);
+        o.cv = neg(rot(qa, scale(qmul(diff, qconj(sq)).v, 2.0f)));
+        return o;
+    }
+    int need_twist = (info & (JF_SPRING | JF_MOTOR | JF_LIMIT)) && !fixed;
+    o.tw = need_twist ? twist(rel) : 0.0f;
+    o.relx = rel.v.x;
+    o.rely = rel.v.y;
+    if (!fixed) {
+        hinge_perps(qa, rel, &o.px, &o.py);
+        /* the perpendicular rows' 2x2 matrix and b3_solve2's reciprocal
+         * determinant (06:600-626, 03_math.inl:347-359) */
+        M3 isum = madd3(ia, ib);
+        o.kxx = dot(o.px, mv(isum, o.px));
+        o.kyy = dot(o.py, mv(isum, o.py));
+        o.kxy = dot(o.px, mv(isum, o.py));
+        float det = o.kxx * o.kyy - o.kxy * o.kxy;
+        o.kinv = det <= 1.0e-12f ? __builtin_nanf("") : 1.0f / det;
+    }
+    return o;
+}
+
 /* The joint rows' delta-pose geometry, joints first, first + stride, ...
  * (a shared tile's waves split them). */
 B3D_FN void joint_geometry(const Lane& L, int first, int stride) {
@@ -2294,50 +2405,30 @@ B3D_FN void joint_geometry(const Lane& L, int first, int stride) {
             int j = j0 + k * stride;
             if (j >= nj) continue;
             uint32_t* r = joint_rec(L, j);
-            Q qa = qmul(dqa[k], fqa[k]);
-            Q qb = qmul(dqb[k], fqb[k]);
-            if (qdot(qa, qb) < 0.0f) qb = qneg(qb);
-            Q rel = qinv_mul(qa, qb);
-            V3 ra = rot(dqa[k], fpa[k]);
-            V3 rb = rot(dqb[k], fpb[k]);
-            st3(r, JS_RA, ra);
-            st3(r, JS_RB, rb);
-            st3(r, JS_PSEP, add(add(sub(dpb[k], dpa[k]), sub(rb, ra)), dcen[k]));
-            /* the point rows' matrix as b3_solve3 inverts it in every solve
-             * (06:241-255, 03_math.inl:343-345) */
-            stm3(r, JS_PKI, inv3(point_k(ma[k], mb[k], ia[k], ib[k], ra, rb)));
             int fixed = info[k] & JF_FIXED;
+            JGeo o = joint_geo(info[k], dqa[k], dqb[k], dpa[k], dpb[k], fqa[k], fqb[k], fpa[k], fpb[k], dcen[k], ma[k],
+                mb[k], ia[k], ib[k]);
+            st3(r, JS_RA, o.ra);
+            st3(r, JS_RB, o.rb);
+            st3(r, JS_PSEP, o.psep);
+            stm3(r, JS_PKI, o.pki);
             if (info[k] & JF_WELD) {
-                if (fixed) continue;
-                Q sq = rel;
-                if (rel.s < 0.0f) sq = qneg(rel);
-                Q diff = q4(-sq.v.x, -sq.v.y, -sq.v.z, 1.0f - sq.s);
-                st3(r, JS_CV, neg(rot(qa, scale(qmul(diff, qconj(sq)).v, 2.0f))));
+                if (!fixed) st3(r, JS_CV, o.cv);
                 continue;
             }
-            int need_twist = (info[k] & (JF_SPRING | JF_MOTOR | JF_LIMIT)) && !fixed;
-            stf(r, JS_TW, need_twist ? twist(rel) : 0.0f);
-            stf(r, JS_RELX, rel.v.x);
-            stf(r, JS_RELY, rel.v.y);
+            stf(r, JS_TW, o.tw);
+            stf(r, JS_RELX, o.relx);
+            stf(r, JS_RELY, o.rely);
             if (!fixed) {
-                V3 px, py;
-                hinge_perps(qa, rel, &px, &py);
-                st3(r, JS_PX, px);
-                st3(r, JS_PY, py);
-                /* the perpendicular rows' 2x2 matrix and b3_solve2's
-                 * reciprocal determinant (06:600-626, 03_math.inl:347-359) */
-                M3 isum = madd3(ia[k], ib[k]);
-                float kxx = dot(px, mv(isum, px));
-                float kyy = dot(py, mv(isum, py));
-                float kxy = dot(px, mv(isum, py));
-                float det = kxx * kyy - kxy * kxy;
-                stf(r, JS_KXX, kxx);
-                stf(r, JS_KXY, kxy);
-                stf(r, JS_KYY, kyy);
-                stf(r, JS_KINV, det <= 1.0e-12f ? __builtin_nanf("") : 1.0f / det);
+                st3(r, JS_PX, o.px);
+                st3(r, JS_PY, o.py);
+                stf(r, JS_KXX, o.kxx);
+                stf(r, JS_KXY, o.kxy);
+                stf(r, JS_KYY, o.kyy);
+                stf(r, JS_KINV, o.kinv);
                 /* the solve's latest hinge rows are part of the joint state */
-                st3(w, jw(L, j, J_PERP_X), px);
-                st3(w, jw(L, j, J_PERP_Y), py);
+                st3(w, jw(L, j, J_PERP_X), o.px);
+                st3(w, jw(L, j, J_PERP_Y), o.py);
             }
         }
     }
@@ -3272,7 +3363,6 @@ B3D_FN int jlevel_next(const Lane& L, int i, int* lev, int mine) {
 
 /* A row's delta-state geometry from the scratch record (every field, in
  * one batch of loads), and the rest of the row from its LDS row. */
-struct JGeo { V3 ra, rb, psep, px, py, cv; M3 pki; float kxx, kxy, kyy, kinv, relx, rely, tw; };
 B3D_FN JGeo jgeo_load(const Lane& L, int j) {
     const uint32_t* g = joint_rec(L, j);
     JGeo o;
@@ -3613,10 +3703,10 @@ B3D_FN void body_prepass(const Lane& L, float h, int first = 0, int stride = 1) 
         for (int k = 0; k < kChunk; k++) {
             int b = b0 + k;
             if (b >= nb) continue;
-            float* row = L.vel + b * kVelWords * kLanes;
+            float* row = L.vel + b * kVelWords * kRow;
 #pragma unroll
-            for (int c = 0; c < 6; c++) row[c * kLanes] = vel[k][c];
-            row[6 * kLanes] = __builtin_bit_cast(float, flags[k]);
+            for (int c = 0; c < 6; c++) row[(c < 3 ? c : kVelAng + c - 3) * kRow] = vel[k][c];
+            *vel_flags(L, b) = __builtin_bit_cast(float, flags[k]);
             uint32_t* r = body_rec(L, b);
             uint32_t* d = delta_rec(L, b);
             int kind = (int)(flags[k] & 0xffu) | (type[k] == kDynamic ? kKindDynamic : 0)

@@ -36,6 +36,15 @@
 #ifndef B3D_LANES
 #define B3D_LANES 64
 #endif
+/* Stride between consecutive words of one world in LDS rows: a tile's 64
+ * lanes, or the worlds of one workgroup where a workgroup steps a part of a
+ * tile with several lanes to a world (B3D_QUAD, b3d_quad.h). */
+#ifndef B3D_QUAD
+#define B3D_QUAD 0
+#endif
+#ifndef B3D_ROW
+#define B3D_ROW B3D_LANES
+#endif
 
 namespace b3d {
 

@@ -1,0 +1,1184 @@
+/*
+ * b3d_quad.h - one world's step on four lanes of each of a workgroup's
+ * waves, for batches that leave most of the chip idle at one lane a world.
+ *
+ * A workgroup of kQuadWaves waves steps kQuadCols = 16 worlds, a quarter of
+ * a 64-world tile: lanes 4c .. 4c + 3 of every wave belong to world c, so a
+ * world has 4 * kQuadWaves = 32 lanes ("workers").  Two ways of using them:
+ *   - what is independent within a world (shapes, candidate pairs, contact
+ *     preparation, body updates, joint geometry) goes one item to a worker,
+ *     through the same scalar functions as the other steps (b3d_lane.h with
+ *     LDS rows of B3D_ROW = 16 words and the per-step records in LDS);
+ *   - what is a chain (the Gauss-Seidel solves, whose order is part of the
+ *     result) goes one solve to a quad of lanes: lane 0..2 of the quad holds
+ *     component x, y, z of every vector, lane 3 the scalars that ride along,
+ *     and products across components use DPP operands.
+ * Why: a chain's time is its instruction count (a dependent fp32 operation
+ * issues every ~5 cycles, whatever the other lanes or a second wave of the
+ * SIMD do), and a vector operation on a quad is one instruction where one
+ * lane needs three (a dot product 4 for 5, a cross product 5 for 9, a
+ * matrix-vector product 5 for 15).  Every component is computed by the same
+ * operations in the same order as in the scalar code, so the bits are the
+ * same.
+ *
+ * Each wave owns contacts and joints for the whole step: joint j is wave
+ * j mod kQuadWaves', contact number i in level order wave i mod
+ * kQuadWaves', and the owner keeps its rows in registers over all sweeps
+ * (the first CR contacts and JR joints of a wave; further contacts are
+ * loaded from their records for each solve).  The velocities are in LDS;
+ * levels of contacts and of joint solves on disjoint dynamic bodies
+ * (b3d_lane.h) go in turn with a workgroup barrier after each, which costs
+ * ~50 cycles.
+ *
+ * Device only.  Include before any other header of the engine.
+ */
+#ifndef PUFFYSICS_AMD_B3D_QUAD_H
+#define PUFFYSICS_AMD_B3D_QUAD_H
+
+#define B3D_QUAD 1
+#define B3D_ROW 16
+#include "b3d_lane.h"
+
+namespace b3d {
+
+#define B3Q_FN static __device__ inline __attribute__((always_inline))
+
+/* ---- quads: component arithmetic on DPP operands ---- */
+template <int P>
+B3Q_FN float qperm(float x) {
+    return __builtin_bit_cast(float,
+        __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), P, 0xf, 0xf, true));
+}
+/* lane P's value in all four lanes */
+template <int P>
+B3Q_FN float qbc(float x) { return qperm<P * 0x55>(x); }
+B3Q_FN float qnext(float x) { return qperm<1 | 2 << 2 | 0 << 4 | 3 << 6>(x); }   /* y z x */
+B3Q_FN float qprev(float x) { return qperm<2 | 0 << 2 | 1 << 4 | 3 << 6>(x); }   /* z x y */
+B3Q_FN float qdot3(float a, float b) {
+    float t = a * b;
+    return qbc<0>(t) + qbc<1>(t) + qbc<2>(t);
+}
+B3Q_FN float qcross(float a, float b) { return qnext(a) * qprev(b) - qprev(a) * qnext(b); }
+/* a lane's row of a matrix: its component of the three columns */
+struct QM { float x, y, z; };
+B3Q_FN float qmv(QM m, float v) { return m.x * qbc<0>(v) + m.y * qbc<1>(v) + m.z * qbc<2>(v); }
+/* rot (03_math.inl) by the unit quaternion q (lane 3: s) */
+B3Q_FN float qrot(float q, float v) {
+    float t = qcross(q, v) * 2.0f;
+    return v + (t * qbc<3>(q) + qcross(q, t));
+}
+
+/* ---- the workgroup's LDS, per world, in words (rows of B3D_ROW) ----
+ * Region X, while contacts are generated: the shape records, the candidates'
+ * hit bits and the old-contacts-unsorted flag, the joint keys; afterwards
+ * the contact levels, the joint levels and the joints' geometry.  Past it,
+ * the new contacts' heads.  Region Y, while contacts are generated: shape
+ * bounds, overlap masks, old contact keys and the colliding workers' clip
+ * rows; afterwards the bodies' rows (quad_body_rows). */
+constexpr int kQuadCols = B3D_ROW, kQuadWaves = 8, kQuadWorkers = 4 * kQuadWaves;
+constexpr int kQuadLdsWords = 160 * 1024 / 4 / kQuadCols;
+/* words of the workgroup (not per world) at the start of LDS */
+constexpr int WG_LEVELS = 0, WG_JLEVELS = 1, WG_JOINTS = 2, WG_REST = 3, kQuadWgWords = 16;
+/* joint geometry rows (struct JGeo) */
+constexpr int JG_TW = 0, JG_RELX = 1, JG_RELY = 2, JG_KXX = 3, JG_KXY = 4, JG_KYY = 5, JG_KINV = 6, JG_PX = 7,
+              JG_PY = 10, JG_RA = 13, JG_RB = 16, JG_PSEP = 19, JG_CV = 22, JG_PKI = 25, kJGWords = 35;
+/* contact head: body a | body b << 8 | points << 16 | CF_* flags << 20 */
+struct QuadLayout {
+    int hits, jkeys;                    /* X, contact generation (the shape records are at 0) */
+    int last, pos, level, order;        /* X, contact levels */
+    int jlast, jlev, jgeo;              /* X, joints */
+    int heads;
+    int y;                              /* region Y: the bodies' rows */
+    int bounds, masks, keys, clip, cw;  /* Y, contact generation; cw workers collide */
+    int words;                          /* in all, per world */
+    size_t scratch_tile_words;          /* HBM, per tile: the per-lane words, then the contact records */
+};
+/* contact records in HBM, world after world, contact after contact */
+constexpr int kQRecQuads = 26, kQRecWords = 4 * kQRecQuads;
+enum { QR_N, QR_T1, QR_CA, QR_CB, QR_IA, QR_IB = QR_IA + 3, QR_ROLL = QR_IB + 3, QR_FI, QR_NMASS, QR_NI, QR_TN, QR_LEVER,
+       QR_SEP, QR_RV, QR_RA, QR_RB = QR_RA + 4 };
+static_assert(QR_RB + 4 == kQRecQuads, "contact record quads");
+
+/* The layout of a capacity set; false when it does not fit. */
+B3D_FN bool quad_layout(const Geometry& g, int max_joints, QuadLayout* q) {
+    if (g.max_s > 64 || g.max_b > 255 || g.max_c > 1023 || g.max_j > max_joints) return false;
+    int hw = hit_words(g);
+    q->hits = 4 * kShapeRows * g.max_s;
+    q->jkeys = q->hits + hw + 1;
+    int xa = q->jkeys + g.max_j;
+    q->last = 0;
+    q->pos = q->last + g.max_b;
+    q->level = q->pos + g.max_c + 2;
+    q->order = q->level + g.max_c;
+    q->jlast = q->order + g.max_c;
+    q->jlev = q->jlast + g.max_b;
+    q->jgeo = q->jlev + g.max_j;
+    int xb = q->jgeo + kJGWords * g.max_j;
+    q->heads = xa > xb ? xa : xb;
+    q->y = q->heads + g.max_c;
+    q->bounds = q->y;
+    q->masks = q->bounds + 6 * g.max_s;
+    q->keys = q->masks + 2 * g.max_s;
+    q->clip = q->keys + g.max_c;
+    int most = kQuadLdsWords - kQuadWgWords / kQuadCols, room = most - q->clip;
+    int rows = q->y + quad_body_rows(g);
+    int cand = g.max_s * (g.max_s - 1) / 2;
+    q->cw = room / kClipWords;
+    if (q->cw > kQuadWorkers) q->cw = kQuadWorkers;
+    if (q->cw > cand) q->cw = cand < 1 ? 1 : cand;
+    if (q->cw < 4 && q->cw < cand) return false;
+    int gen = q->clip + q->cw * kClipWords;
+    q->words = gen > rows ? gen : rows;
+    q->scratch_tile_words = (size_t)g.scr_words * kLanes + (size_t)kLanes * g.max_c * kQRecWords;
+    return q->words <= most;
+}
+
+/* One lane's view: its world (L, rows in LDS), its place in the quad and
+ * among the world's workers. */
+struct QLane {
+    Lane L;
+    float* lds;        /* LDS rows + world column */
+    uint32_t* recs;    /* the world's contact records */
+    PairStage st;      /* the tile's manifold stage */
+    int sub, wave, worker;
+    QuadLayout q;
+};
+B3Q_FN float* lrow(const QLane& Q, int word) { return Q.lds + word * kRow; }
+B3Q_FN int lgeti(const QLane& Q, int word) { return __builtin_bit_cast(int, Q.lds[word * kRow]); }
+B3Q_FN void lseti(const QLane& Q, int word, int v) { Q.lds[word * kRow] = __builtin_bit_cast(float, v); }
+
+/* ---- contact generation ---- */
+
+/* The old contacts' keys, their pairs' order and warm data, the shape
+ * records and bounds, and the joint keys (find_contacts' opening): one item
+ * to a worker. */
+B3Q_FN void quad_open(const QLane& Q, int old_n, int ns, int nj) {
+    const Lane& L = Q.L;
+    for (int k = Q.worker; k < old_n; k += kQuadWorkers) {
+        int sa = ldi(L.w, cw(L, k, C_SHAPE_A)), sb = ldi(L.w, cw(L, k, C_SHAPE_B));
+        int pk = k > 0 ? k - 1 : 0;
+        int pa = ldi(L.w, cw(L, pk, C_SHAPE_A)), pb = ldi(L.w, cw(L, pk, C_SHAPE_B));
+        uint32_t key = shape_key(sa, sb);
+        lseti(Q, Q.q.keys + k, (int)key);
+        uint32_t* o = old_rec(L, k);
+        sti(o, O_SHAPE_A, sa);
+        sti(o, O_SHAPE_B, sb);
+        if (k > 0 && !(shape_key(pa, pb) < key && (uint32_t)sa < 65536u && (uint32_t)sb < 65536u))
+            lseti(Q, Q.q.hits + hit_words(L.g), 1);
+    }
+    old_warm_copy(L, old_n, Q.worker, kQuadWorkers);
+    shape_pass(L, ns, lrow(Q, Q.q.bounds), Q.worker, kQuadWorkers);
+    for (int j = Q.worker; j < nj; j += kQuadWorkers) {
+        uint32_t key = 0xffffffffu;
+        if (!ldi(L.w, jw(L, j, J_COLLIDE_CONNECTED)))
+            key = pair_key(ldi(L.w, jw(L, j, J_BODY_A)), ldi(L.w, jw(L, j, J_BODY_B)));
+        lseti(Q, Q.q.jkeys + j, (int)key);
+    }
+}
+
+B3Q_FN uint64_t quad_mask(const QLane& Q, int i) {
+    return (uint64_t)(uint32_t)lgeti(Q, Q.q.masks + 2 * i) | ((uint64_t)(uint32_t)lgeti(Q, Q.q.masks + 2 * i + 1) << 32);
+}
+/* Bound-overlap masks, a row of pairs (i, j > i) to a worker. */
+B3Q_FN void quad_overlaps(const QLane& Q, int ns) {
+    const float* bounds = lrow(Q, Q.q.bounds);
+    for (int i = Q.worker; i < ns; i += kQuadWorkers) {
+        Box6 bi = box_load(bounds + i * 6 * kRow);
+        uint64_t m = 0;
+        for (int j0 = i + 1; j0 < ns; j0 += 4) {
+            Box6 bj[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (j0 + k < ns) bj[k] = box_load(bounds + (j0 + k) * 6 * kRow);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (j0 + k < ns && box_overlap(bi, bj[k])) m |= 1ull << (j0 + k);
+        }
+        lseti(Q, Q.q.masks + 2 * i, (int)(uint32_t)m);
+        lseti(Q, Q.q.masks + 2 * i + 1, (int)(uint32_t)(m >> 32));
+    }
+}
+
+/* This worker's share of the narrowphase: candidates worker, worker + cw,
+ * ... in (i, j) order, their manifolds to the stage (pair_share). */
+B3Q_FN void quad_collide(const QLane& Q, int ns, int nj, int old_n) {
+    const Lane& L = Q.L;
+    if (Q.worker >= Q.q.cw) return;
+    bool sorted = lgeti(Q, Q.q.hits + hit_words(L.g)) == 0;
+    int t = Q.worker, acc = 0;
+    float* clip = lrow(Q, Q.q.clip + Q.worker * kClipWords);
+    for (int i = 0; i < ns; i++) {
+        uint64_t m = quad_mask(Q, i);
+        int c = __builtin_popcountll(m);
+        for (; t < acc + c; t += Q.q.cw) {
+            uint64_t mm = m;
+            for (int k = t - acc; k > 0; k--) mm &= mm - 1;
+            int j = __builtin_ctzll(mm);
+            PairShape A, B;
+            pshape_load(L, i, &A);
+            pshape_load(L, j, &B);
+            uint32_t bkey = pair_key(A.body, B.body);
+            int joined = 0;
+            for (int k = 0; k < nj; k++) joined |= (uint32_t)lgeti(Q, Q.q.jkeys + k) == bkey;
+            Mani mf;
+            mf.count = 0;
+            if (!(A.body == B.body || (A.bflags & B.bflags & kBodyStatic) || (A.cat & B.mask) == 0
+                    || (B.cat & A.mask) == 0 || joined))
+                collide_pair(&mf, A.P, B.P, clip);
+            if (mf.count > 0) {
+                /* the old contact of the same pair (the merge of the sorted lists) */
+                uint32_t key = shape_key(i, j);
+                int match = -1;
+                if (sorted) {
+                    int lo = 0, hi = old_n;
+                    while (lo < hi) {
+                        int mid = (lo + hi) >> 1;
+                        if ((uint32_t)lgeti(Q, Q.q.keys + mid) < key) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    if (lo < old_n && (uint32_t)lgeti(Q, Q.q.keys + lo) == key) match = lo;
+                }
+                mani_store(Q.st, L.lane, t, mf, key, match);
+                lds_or(lrow(Q, Q.q.hits + (t >> 5)), 1u << (t & 31));
+            }
+        }
+        acc += c;
+    }
+}
+
+B3Q_FN Quad quad_of(V3 v, float s) {
+    return Quad{__builtin_bit_cast(uint32_t, v.x), __builtin_bit_cast(uint32_t, v.y),
+        __builtin_bit_cast(uint32_t, v.z), __builtin_bit_cast(uint32_t, s)};
+}
+B3Q_FN uint32_t* qrec(const QLane& Q, int c) { return Q.recs + (size_t)c * kQRecWords; }
+
+/* New contact k of the world: the candidate with the k-th manifold, written
+ * to the world's row (write_new_contact) and prepared (contact_prep,
+ * b3_prepare_one_contact) into its record, with its head in LDS.  Returns
+ * its CF_* flags. */
+B3Q_FN int quad_contact(const QLane& Q, int k, int t, int old_n, bool sorted, Soft cs, Soft ss) {
+    const Lane& L = Q.L;
+    uint32_t* w = L.w;
+    Mani m;
+    uint32_t key;
+    int match;
+    mani_load(Q.st, L.lane, t, &m, &key, &match);
+    int i = (int)(key >> 16), j = (int)(key & 0xffffu);
+    PairShape A, B;
+    pshape_load(L, i, &A);
+    pshape_load(L, j, &B);
+    OldWarm orec;
+    if (sorted && match >= 0) old_load(L, match, &orec);
+    /* zero unless the body is dynamic (08:236-241) */
+    float ma = 0.0f, mb = 0.0f;
+    M3 ia = m3zero(), ib = m3zero();
+    if (A.bflags & kBodyDynamic) {
+        ma = ldf(w, bw(L, A.body, B_INV_MASS));
+        ia = ldm3(w, bw(L, A.body, B_INV_I_WORLD));
+    }
+    if (B.bflags & kBodyDynamic) {
+        mb = ldf(w, bw(L, B.body, B_INV_MASS));
+        ib = ldm3(w, bw(L, B.body, B_INV_I_WORLD));
+    }
+    NewContact nc = new_contact(L, i, j, A, B, m, sorted, match, orec, old_n);
+    int info = store_new_contact(L, k, i, j, A, B, nc);
+    const int keep = (L.opts & kKeepSolverFields) != 0;
+    const int need_rv = keep || (info & CF_RESTITUTION);
+    V3 va = zero3(), wa = zero3(), vb = zero3(), wb = zero3();
+    if (need_rv) {
+        /* the bodies' velocities of the start of the step */
+        va = ld3(w, bw(L, A.body, B_LIN_VEL));
+        wa = ld3(w, bw(L, A.body, B_ANG_VEL));
+        vb = ld3(w, bw(L, B.body, B_LIN_VEL));
+        wb = ld3(w, bw(L, B.body, B_ANG_VEL));
+    }
+    ContactPrep p = contact_prep(nc.count, nc.normal, nc.t1, nc.r_a, nc.r_b, nc.base_sep, nc.ni, ma, mb, ia, ib,
+        need_rv, va, wa, vb, wb);
+    if (keep) keep_solver_fields(L, k, nc.count, p, ma, mb, ia, ib, (info & CF_STATIC) ? ss : cs);
+    Quad* r = reinterpret_cast<Quad*>(qrec(Q, k));
+    float friction = sqrtf(A.friction * B.friction);
+    float restitution = A.restitution > B.restitution ? A.restitution : B.restitution;
+    float rolling = maxf(A.rolling, B.rolling);
+    r[QR_N] = quad_of(nc.normal, friction);
+    r[QR_T1] = quad_of(nc.t1, p.twist_mass);
+    r[QR_CA] = quad_of(p.center_a, rolling);
+    r[QR_CB] = quad_of(p.center_b, restitution);
+    r[QR_IA] = quad_of(ia.cx, ma);
+    r[QR_IA + 1] = quad_of(ia.cy, p.tmass.cx.x);
+    r[QR_IA + 2] = quad_of(ia.cz, p.tmass.cx.y);
+    r[QR_IB] = quad_of(ib.cx, mb);
+    r[QR_IB + 1] = quad_of(ib.cy, p.tmass.cy.y);
+    r[QR_IB + 2] = quad_of(ib.cz, 0.0f);
+    r[QR_ROLL] = quad_of(nc.roll, nc.twist);
+    r[QR_FI] = quad_of(v3(nc.fi.x, nc.fi.y, 0.0f), 0.0f);
+    r[QR_NMASS] = quad_of(v3(p.nmass[0], p.nmass[1], p.nmass[2]), p.nmass[3]);
+    r[QR_NI] = quad_of(v3(p.ni[0], p.ni[1], p.ni[2]), p.ni[3]);
+    r[QR_TN] = quad_of(zero3(), 0.0f);
+    r[QR_LEVER] = quad_of(v3(p.lever[0], p.lever[1], p.lever[2]), p.lever[3]);
+    r[QR_SEP] = quad_of(v3(p.base_sep[0], p.base_sep[1], p.base_sep[2]), p.base_sep[3]);
+    r[QR_RV] = quad_of(v3(p.rel_vel[0], p.rel_vel[1], p.rel_vel[2]), p.rel_vel[3]);
+#pragma unroll
+    for (int q = 0; q < kMaxManifold; q++) {
+        if (q >= nc.count) continue;
+        r[QR_RA + q] = quad_of(nc.r_a[q], 0.0f);
+        r[QR_RB + q] = quad_of(nc.r_b[q], 0.0f);
+    }
+    lseti(Q, Q.q.heads + k, A.body | (B.body << 8) | (nc.count << 16) | (info << 20));
+    return info;
+}
+
+/* The world's new contacts, one to a worker at a time, and its header
+ * counts (append_share, find_pairs).  Returns the contact count. */
+B3Q_FN int quad_append(const QLane& Q, int old_n, Soft cs, Soft ss, int* wg) {
+    const Lane& L = Q.L;
+    int total = 0, hw = hit_words(L.g);
+    for (int k = 0; k < hw; k++) total += __builtin_popcount((uint32_t)lgeti(Q, Q.q.hits + k));
+    int cc = total < L.g.max_c ? total : L.g.max_c;
+    bool sorted = lgeti(Q, Q.q.hits + hw) == 0;
+    int acc = 0, word = 0, flags = 0;
+    for (int k = Q.worker; k < cc; k += kQuadWorkers) {
+        uint32_t bits = (uint32_t)lgeti(Q, Q.q.hits + word);
+        while (acc + __builtin_popcount(bits) <= k) {
+            acc += __builtin_popcount(bits);
+            word++;
+            bits = (uint32_t)lgeti(Q, Q.q.hits + word);
+        }
+        for (int r = k - acc; r > 0; r--) bits &= bits - 1;
+        flags |= quad_contact(Q, k, word * 32 + __builtin_ctz(bits), old_n, sorted, cs, ss);
+    }
+    if (flags & CF_RESTITUTION) atomicOr(wg + WG_REST, 1);
+    if (Q.worker == 0) {
+        sti(L.w, H_CONTACT_COUNT, cc);
+        sti(L.w, H_CONTACT_OVERFLOW, ldi(L.w, H_CONTACT_OVERFLOW) | (total > L.g.max_c ? 1 : 0));
+        sti(L.w, H_CONTACTS_DROPPED, ldi(L.w, H_CONTACTS_DROPPED) + (total - cc));
+    }
+    return cc;
+}
+
+/* The contacts' levels (sched_build) and their order by level: entry i is
+ * contact | level << 10.  One worker of the world. */
+B3Q_FN void quad_levels(const QLane& Q, int cc, int nb, int* wg) {
+    for (int b = 0; b < nb; b++) lseti(Q, Q.q.last + b, 0);
+    for (int lev = 0; lev <= cc; lev++) lseti(Q, Q.q.pos + lev, 0);
+    int nlev = 0;
+    for (int c0 = 0; c0 < cc; c0 += kSchedChunk) {
+        int hd[kSchedChunk];
+#pragma unroll
+        for (int k = 0; k < kSchedChunk; k++)
+            if (c0 + k < cc) hd[k] = lgeti(Q, Q.q.heads + c0 + k);
+#pragma unroll
+        for (int k = 0; k < kSchedChunk; k++) {
+            int c = c0 + k;
+            if (c >= cc) continue;
+            int a = hd[k] & 255, b = (hd[k] >> 8) & 255, fl = hd[k] >> 20;
+            int la = (fl & CF_DYN_A) ? lgeti(Q, Q.q.last + a) : 0;
+            int lb = (fl & CF_DYN_B) ? lgeti(Q, Q.q.last + b) : 0;
+            int lev = (la > lb ? la : lb) + 1;
+            if (fl & CF_DYN_A) lseti(Q, Q.q.last + a, lev);
+            if (fl & CF_DYN_B) lseti(Q, Q.q.last + b, lev);
+            lseti(Q, Q.q.level + c, lev);
+            lseti(Q, Q.q.pos + lev, lgeti(Q, Q.q.pos + lev) + 1);
+            if (lev > nlev) nlev = lev;
+        }
+    }
+    int run = 0;
+    for (int lev = 1; lev <= nlev; lev++) {
+        int n = lgeti(Q, Q.q.pos + lev);
+        lseti(Q, Q.q.pos + lev, run);
+        run += n;
+    }
+    for (int c = 0; c < cc; c++) {
+        int lev = lgeti(Q, Q.q.level + c);
+        int at = lgeti(Q, Q.q.pos + lev);
+        lseti(Q, Q.q.pos + lev, at + 1);
+        lseti(Q, Q.q.order + at, c | (lev << 10));
+    }
+    atomicMax(wg + WG_LEVELS, nlev);
+}
+
+/* The joint solves' levels (joint_levels_scan): of joint j in the pass's
+ * two iterations, at jlev + j (first | second << 8).  One worker. */
+B3Q_FN void quad_joint_levels(const QLane& Q, int nj, int nb, int* wg) {
+    const Lane& L = Q.L;
+    for (int b = 0; b < nb; b++) lseti(Q, Q.q.jlast + b, 0);
+    int nlev = 0;
+    for (int it = 0; it < kJointIters; it++) {
+        for (int j = 0; j < nj; j++) {
+            uint32_t ab = ldu(joint_rec(L, j), JS_AB);
+            int a = (int)(ab & 0xffffu), b = (int)(ab >> 16);
+            bool da = is_dyn_flag(L, a), db = is_dyn_flag(L, b);
+            int la = da ? lgeti(Q, Q.q.jlast + a) : 0;
+            int lb = db ? lgeti(Q, Q.q.jlast + b) : 0;
+            int lev = (la > lb ? la : lb) + 1;
+            if (da) lseti(Q, Q.q.jlast + a, lev);
+            if (db) lseti(Q, Q.q.jlast + b, lev);
+            lseti(Q, Q.q.jlev + j, it == 0 ? lev : lgeti(Q, Q.q.jlev + j) | (lev << 8));
+            if (lev > nlev) nlev = lev;
+        }
+    }
+    atomicMax(wg + WG_JLEVELS, nlev);
+    atomicMax(wg + WG_JOINTS, nj);
+}
+
+/* The joints' delta-pose geometry to their LDS rows, joints first, first +
+ * stride, ... */
+B3Q_FN void quad_joint_geometry(const QLane& Q, int nj, int first, int stride) {
+    const Lane& L = Q.L;
+    const uint32_t* w = L.w;
+    for (int j = first; j < nj; j += stride) {
+        uint32_t ab = ldu(joint_rec(L, j), JS_AB);
+        int info = ldi(joint_rec(L, j), JS_INFO);
+        b3d::Q fqa = ldq(w, jw(L, j, J_FRAME_Q_A)), fqb = ldq(w, jw(L, j, J_FRAME_Q_B));
+        V3 fpa = ld3(w, jw(L, j, J_FRAME_P_A)), fpb = ld3(w, jw(L, j, J_FRAME_P_B));
+        V3 dcen = ld3(w, jw(L, j, J_DELTA_CENTER));
+        float ma = ldf(w, jw(L, j, J_INV_MASS_A)), mb = ldf(w, jw(L, j, J_INV_MASS_B));
+        M3 ia = ldm3(w, jw(L, j, J_INV_I_A)), ib = ldm3(w, jw(L, j, J_INV_I_B));
+        const uint32_t* da = delta_rec(L, (int)(ab & 0xffffu));
+        const uint32_t* db = delta_rec(L, (int)(ab >> 16));
+        JGeo o = joint_geo(info, rq4(da, BD_DQ), rq4(db, BD_DQ), r3(da, BD_DP), r3(db, BD_DP), fqa, fqb, fpa, fpb, dcen,
+            ma, mb, ia, ib);
+        float* g = lrow(Q, Q.q.jgeo + j * kJGWords);
+        auto put = [g](int k, float v) { g[k * kRow] = v; };
+        auto put3 = [put](int k, V3 v) { put(k, v.x); put(k + 1, v.y); put(k + 2, v.z); };
+        put3(JG_RA, o.ra);
+        put3(JG_RB, o.rb);
+        put3(JG_PSEP, o.psep);
+        put3(JG_PKI, o.pki.cx);
+        put3(JG_PKI + 3, o.pki.cy);
+        put3(JG_PKI + 6, o.pki.cz);
+        bool fixed = (info & JF_FIXED) != 0;
+        if (info & JF_WELD) {
+            if (!fixed) put3(JG_CV, o.cv);
+            continue;
+        }
+        put(JG_TW, o.tw);
+        put(JG_RELX, o.relx);
+        put(JG_RELY, o.rely);
+        if (fixed) continue;
+        put3(JG_PX, o.px);
+        put3(JG_PY, o.py);
+        put(JG_KXX, o.kxx);
+        put(JG_KXY, o.kxy);
+        put(JG_KYY, o.kyy);
+        put(JG_KINV, o.kinv);
+    }
+}
+
+/* ---- contact rows on quads ---- */
+
+/* A contact's row in a quad's registers: each float is one quad of the
+ * record, lane 3 holding the scalar that rides along (QR_*): friction with
+ * n, twist mass with t1, rolling with ca, restitution with cb, the inverse
+ * masses and the tangent mass with the inertia columns, the twist impulse
+ * with roll.  Of the per-point values (nmass, ni, tn, lever, sep) lane p
+ * holds point p's. */
+struct CQ {
+    int c, lev, fl;        /* contact (-1: none), its level, CF_* flags | points << 8; the bodies' velocity rows */
+    int va, vb;
+    float n, t1, ca, cb, roll, fi, nmass, ni, tn, lever, sep;
+    QM ia, ib;
+    float ra[kMaxManifold], rb[kMaxManifold];
+};
+constexpr int kQDynA = 1 << 16, kQDynB = 1 << 17;   /* CQ::fl, JQ::info: the body's velocity is written */
+
+B3Q_FN float qload(const uint32_t* r, int quad) { return __builtin_bit_cast(float, r[4 * quad]); }
+/* Velocity rows: this lane's component (lane 3: a pad word). */
+B3Q_FN int qvel_row(int b) { return b * kVelWords * kRow; }
+B3Q_FN float* qvel(const QLane& Q) { return Q.L.vel + Q.sub * kRow; }
+
+/* This lane's part of the row of order entry e (contact | level << 10),
+ * with its separations at the bodies' delta poses (08_contacts.inl:
+ * 331-333). */
+B3Q_FN void cq_deltas(const QLane& Q, const CQ& r, float* dpa, float* dqa, float* dpb, float* dqb) {
+    int d = Q.q.y + quad_delta_word(Q.L.g) + Q.sub;
+    int a = r.va / (kVelWords * kRow), b = r.vb / (kVelWords * kRow);
+    const float* da = lrow(Q, d + a * 4 * kDeltaRows);
+    const float* db = lrow(Q, d + b * 4 * kDeltaRows);
+    *dpa = da[BD_DP * kRow];
+    *dqa = da[BD_DQ * kRow];
+    *dpb = db[BD_DP * kRow];
+    *dqb = db[BD_DQ * kRow];
+}
+B3Q_FN float cq_separations(const QLane& Q, const CQ& r, float base) {
+    float dpa, dqa, dpb, dqb;
+    cq_deltas(Q, r, &dpa, &dqa, &dpb, &dqb);
+    float dp = dpb - dpa, sep = 0.0f;
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        if (p >= ((r.fl >> 8) & 255)) continue;
+        float ds = dp + (qrot(dqb, r.rb[p]) - qrot(dqa, r.ra[p]));
+        float s = qdot3(ds, r.n);
+        sep = Q.sub == p ? s : sep;
+    }
+    return sep + base;
+}
+B3Q_FN void cq_load(const QLane& Q, int e, CQ* r) {
+    int c = e & 1023;
+    int hd = lgeti(Q, Q.q.heads + c);
+    const uint32_t* rc = qrec(Q, c) + Q.sub;
+    int a = hd & 255, b = (hd >> 8) & 255;
+    r->c = c;
+    r->lev = e >> 10;
+    r->fl = (hd >> 20) | (((hd >> 16) & 15) << 8) | (is_dyn_flag(Q.L, a) ? kQDynA : 0)
+        | (is_dyn_flag(Q.L, b) ? kQDynB : 0);
+    r->va = qvel_row(a);
+    r->vb = qvel_row(b);
+    r->n = qload(rc, QR_N);
+    r->t1 = qload(rc, QR_T1);
+    r->ca = qload(rc, QR_CA);
+    r->cb = qload(rc, QR_CB);
+    r->roll = qload(rc, QR_ROLL);
+    r->fi = qload(rc, QR_FI);
+    r->nmass = qload(rc, QR_NMASS);
+    r->ni = qload(rc, QR_NI);
+    r->tn = qload(rc, QR_TN);
+    r->lever = qload(rc, QR_LEVER);
+    r->ia = QM{qload(rc, QR_IA), qload(rc, QR_IA + 1), qload(rc, QR_IA + 2)};
+    r->ib = QM{qload(rc, QR_IB), qload(rc, QR_IB + 1), qload(rc, QR_IB + 2)};
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        r->ra[p] = 0.0f;
+        r->rb[p] = 0.0f;
+        if (p >= ((r->fl >> 8) & 255)) continue;
+        r->ra[p] = qload(rc, QR_RA + p);
+        r->rb[p] = qload(rc, QR_RB + p);
+    }
+}
+/* The base separations a row's separations add (kept in the record). */
+B3Q_FN float cq_base(const QLane& Q, const CQ& r) { return qload(qrec(Q, r.c) + Q.sub, QR_SEP); }
+/* The row's impulses back to the record. */
+B3Q_FN void cq_store(const QLane& Q, const CQ& r) {
+    uint32_t* rc = qrec(Q, r.c) + Q.sub;
+    rc[4 * QR_NI] = __builtin_bit_cast(uint32_t, r.ni);
+    rc[4 * QR_TN] = __builtin_bit_cast(uint32_t, r.tn);
+    rc[4 * QR_FI] = __builtin_bit_cast(uint32_t, r.fi);
+    rc[4 * QR_ROLL] = __builtin_bit_cast(uint32_t, r.roll);
+}
+
+/* A row's bodies' velocities: read, and written back where dynamic. */
+struct QVel { float va, wa, vb, wb; };
+B3Q_FN QVel qvel_load(const QLane& Q, int va, int vb) {
+    const float* v = qvel(Q);
+    return QVel{v[va], v[va + kVelAng * kRow], v[vb], v[vb + kVelAng * kRow]};
+}
+B3Q_FN void qvel_store(const QLane& Q, int va, int vb, int fl, QVel x) {
+    float* v = qvel(Q);
+    if (fl & kQDynA) {
+        v[va] = x.va;
+        v[va + kVelAng * kRow] = x.wa;
+    }
+    if (fl & kQDynB) {
+        v[vb] = x.vb;
+        v[vb + kVelAng * kRow] = x.wb;
+    }
+}
+/* Impulse P at levers ra and rb on the bodies (b after a, opposite). */
+B3Q_FN void qimpulse(QVel* x, float ma, QM ia, float mb, QM ib, float ra, float rb, float P) {
+    x->va = x->va - ma * P;
+    x->wa = x->wa - qmv(ia, qcross(ra, P));
+    x->vb = x->vb + mb * P;
+    x->wb = x->wb + qmv(ib, qcross(rb, P));
+}
+
+/* The contact's warm start (08:194-232). */
+B3Q_FN void cq_warm(const QLane& Q, const CQ& r) {
+    QVel x = qvel_load(Q, r.va, r.vb);
+    float ma = qbc<3>(r.ia.x), mb = qbc<3>(r.ib.x);
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        if (p >= ((r.fl >> 8) & 255)) continue;
+        float ni = p == 0 ? qbc<0>(r.ni) : (p == 1 ? qbc<1>(r.ni) : (p == 2 ? qbc<2>(r.ni) : qbc<3>(r.ni)));
+        qimpulse(&x, ma, r.ia, mb, r.ib, r.ra[p], r.rb[p], r.n * ni);
+    }
+    float t2 = qcross(r.t1, r.n);
+    float f = r.t1 * qbc<0>(r.fi) + t2 * qbc<1>(r.fi);
+    qimpulse(&x, ma, r.ia, mb, r.ib, r.ca, r.cb, f);
+    float tr = r.n * qbc<3>(r.roll) + r.roll;
+    x.wa = x.wa - qmv(r.ia, tr);
+    x.wb = x.wb + qmv(r.ib, tr);
+    qvel_store(Q, r.va, r.vb, r.fl, x);
+}
+
+/* Rolling resistance (07_packed.inl:24-45) on quads. */
+B3Q_FN void cq_rolling(const CQ& r, float t2, float rolling, float total_n, float* impulse, QVel* x) {
+    QM is = QM{r.ia.x + r.ib.x, r.ia.y + r.ib.y, r.ia.z + r.ib.z};
+    M2 k;
+    float it2 = qmv(is, t2);
+    k.cx.x = qdot3(r.t1, qmv(is, r.t1));
+    k.cy.y = qdot3(t2, it2);
+    k.cx.y = qdot3(r.t1, it2);
+    k.cy.x = k.cx.y;
+    float wr = x->wb - x->wa;
+    V2 rhs;
+    rhs.x = qdot3(wr, r.t1);
+    rhs.y = qdot3(wr, t2);
+    V2 d = mv2(inv2(k), rhs);
+    float next = *impulse - (r.t1 * d.x + t2 * d.y);
+    float limit = rolling * total_n;
+    float l2 = qdot3(next, next);
+    if (l2 > limit * limit && l2 > 0.0f) next = next * rsqrt_scale(limit, l2);
+    float delta = next - *impulse;
+    *impulse = next;
+    x->wa = x->wa - qmv(r.ia, delta);
+    x->wb = x->wb + qmv(r.ib, delta);
+}
+
+/* One contact's solve, b3_solve_one_contact (08:315-413), as crow_solve. */
+template <bool Relax>
+B3Q_FN void cq_solve(const QLane& Q, CQ& r, float inv_h, float contact_speed, Soft cs, Soft ss) {
+    QVel x = qvel_load(Q, r.va, r.vb);
+    float ma = qbc<3>(r.ia.x), mb = qbc<3>(r.ib.x);
+    /* each lane the coefficients of its own point */
+    float vbias = 0.0f, mscale = 1.0f, iscale = 0.0f;
+    if (!Relax) {
+        bool st = (r.fl & CF_STATIC) != 0;
+        float ms = st ? ss.mass_scale : cs.mass_scale;
+        vbias = maxf(ms * (st ? ss.bias_rate : cs.bias_rate) * r.sep, -contact_speed);
+        mscale = ms;
+        iscale = st ? ss.impulse_scale : cs.impulse_scale;
+    }
+    if (r.sep > 0.0f) {
+        vbias = r.sep * inv_h;
+        mscale = 1.0f;
+        iscale = 0.0f;
+    }
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        if (p >= ((r.fl >> 8) & 255)) continue;
+        float vra = x.va + qcross(x.wa, r.ra[p]);
+        float vrb = x.vb + qcross(x.wb, r.rb[p]);
+        float vn = qdot3(vrb - vra, r.n);
+        float dimp = -r.nmass * (mscale * vn + vbias) - iscale * r.ni;
+        float nimp = maxf(r.ni + dimp, 0.0f);
+        dimp = nimp - r.ni;
+        r.ni = Q.sub == p ? nimp : r.ni;
+        r.tn = Q.sub == p ? r.tn + nimp : r.tn;
+        dimp = p == 0 ? qbc<0>(dimp) : (p == 1 ? qbc<1>(dimp) : (p == 2 ? qbc<2>(dimp) : qbc<3>(dimp)));
+        qimpulse(&x, ma, r.ia, mb, r.ib, r.ra[p], r.rb[p], r.n * dimp);
+    }
+    if (Relax) {
+        /* sums over the points, in point order */
+        float lev = r.lever * r.ni;
+        int pc = (r.fl >> 8) & 255;
+        float total_n = 0.0f, twist_lim = 0.0f;
+        if (pc > 0) {
+            total_n = total_n + qbc<0>(r.ni);
+            twist_lim = twist_lim + qbc<0>(lev);
+        }
+        if (pc > 1) {
+            total_n = total_n + qbc<1>(r.ni);
+            twist_lim = twist_lim + qbc<1>(lev);
+        }
+        if (pc > 2) {
+            total_n = total_n + qbc<2>(r.ni);
+            twist_lim = twist_lim + qbc<2>(lev);
+        }
+        if (pc > 3) {
+            total_n = total_n + qbc<3>(r.ni);
+            twist_lim = twist_lim + qbc<3>(lev);
+        }
+        float friction = qbc<3>(r.n), twist_imp = qbc<3>(r.roll);
+        float twist_s = qdot3(r.n, x.wb - x.wa);
+        float max_t = friction * twist_lim;
+        float dtw = -qbc<3>(r.t1) * twist_s;
+        float new_t = clampf(twist_imp + dtw, -max_t, max_t);
+        dtw = new_t - twist_imp;
+        float tw = r.n * dtw;
+        x.wa = x.wa - qmv(r.ia, tw);
+        x.wb = x.wb + qmv(r.ib, tw);
+
+        float t2 = qcross(r.t1, r.n);
+        float vr = (x.vb + qcross(x.wb, r.cb)) - (x.va + qcross(x.wa, r.ca));
+        V2 vt;
+        vt.x = qdot3(vr, r.t1);
+        vt.y = qdot3(vr, t2);
+        M2 tm;
+        tm.cx.x = qbc<3>(r.ia.y);
+        tm.cx.y = qbc<3>(r.ia.z);
+        tm.cy.x = tm.cx.y;
+        tm.cy.y = qbc<3>(r.ib.y);
+        V2 tmv = mv2(tm, vt);
+        float fx = qbc<0>(r.fi), fy = qbc<1>(r.fi);
+        V2 ni;
+        ni.x = fx - tmv.x;
+        ni.y = fy - tmv.y;
+        float max_f = friction * total_n;
+        float fl2 = ni.x * ni.x + ni.y * ni.y;
+        if (fl2 > max_f * max_f && fl2 > 0.0f) {
+            float sc = rsqrt_scale(max_f, fl2);
+            ni.x *= sc;
+            ni.y *= sc;
+        }
+        r.fi = Q.sub == 0 ? ni.x : ni.y;
+        float P = r.t1 * (ni.x - fx) + t2 * (ni.y - fy);
+        qimpulse(&x, ma, r.ia, mb, r.ib, r.ca, r.cb, P);
+        float roll = r.roll;
+        if (r.fl & CF_ROLLING) cq_rolling(r, t2, qbc<3>(r.ca), total_n, &roll, &x);
+        r.roll = Q.sub == 3 ? new_t : roll;
+    }
+    qvel_store(Q, r.va, r.vb, r.fl, x);
+}
+
+/* b3_apply_restitution for one contact (08:439-480). */
+B3Q_FN void cq_restitution(const QLane& Q, CQ& r, float threshold) {
+    if (!(r.fl & CF_RESTITUTION)) return;
+    QVel x = qvel_load(Q, r.va, r.vb);
+    float ma = qbc<3>(r.ia.x), mb = qbc<3>(r.ib.x), e = qbc<3>(r.cb);
+    float rv = qload(qrec(Q, r.c) + Q.sub, QR_RV);
+    /* each lane its own point's test: 1 when the point is left alone */
+    float skip = rv > -threshold || r.tn == 0.0f ? 1.0f : 0.0f;
+#pragma unroll
+    for (int p = 0; p < kMaxManifold; p++) {
+        if (p >= ((r.fl >> 8) & 255)) continue;
+        float s = p == 0 ? qbc<0>(skip) : (p == 1 ? qbc<1>(skip) : (p == 2 ? qbc<2>(skip) : qbc<3>(skip)));
+        if (s != 0.0f) continue;
+        float vra = x.va + qcross(x.wa, r.ra[p]);
+        float vrb = x.vb + qcross(x.wb, r.rb[p]);
+        float vn = qdot3(vrb - vra, r.n);
+        float imp = -r.nmass * (vn + e * rv);
+        float nimp = maxf(r.ni + imp, 0.0f);
+        imp = nimp - r.ni;
+        r.ni = Q.sub == p ? nimp : r.ni;
+        imp = p == 0 ? qbc<0>(imp) : (p == 1 ? qbc<1>(imp) : (p == 2 ? qbc<2>(imp) : qbc<3>(imp)));
+        qimpulse(&x, ma, r.ia, mb, r.ib, r.ra[p], r.rb[p], r.n * imp);
+    }
+    qvel_store(Q, r.va, r.vb, r.fl, x);
+}
+
+/* The accumulated impulses of a row to the world's contact (contact_writeback). */
+B3Q_FN void cq_writeback(const QLane& Q, const CQ& r) {
+    const Lane& L = Q.L;
+    uint32_t* w = L.w;
+    if (Q.sub < ((r.fl >> 8) & 255)) {
+        stf(w, pw(L, r.c, Q.sub, P_NORMAL_IMPULSE), r.ni);
+        stf(w, pw(L, r.c, Q.sub, P_TOTAL_NORMAL), r.tn);
+    }
+    if (Q.sub < 2) stf(w, cw(L, r.c, C_FRICTION_IMPULSE + Q.sub), r.fi);
+    if (Q.sub == 3) stf(w, cw(L, r.c, C_TWIST_IMPULSE), r.roll);
+    else if (r.fl & CF_ROLLING) stf(w, cw(L, r.c, C_ROLLING_IMPULSE + Q.sub), r.roll);
+}
+
+/* ---- joint rows on quads ---- */
+
+/* A joint's row in a quad's registers.  Scalars are the same in all four
+ * lanes.  A weld's fields share the hinge's: axis the accumulated angular
+ * impulse, ia_ax, ib_ax, px the angular mass columns, py the angular error;
+ * axial, maxt the linear and angular hertz, (target, ss.x, ss.y) the linear
+ * and (ss.z, speed, lower) the angular spring. */
+struct JQ {
+    int j, lev, info;      /* joint (-1: none), its two levels (quad_joint_levels), JF_* | kQDyn* */
+    int va, vb;
+    float ma, mb;
+    QM ia, ib;
+    Soft soft;
+    float lin_imp, ra, rb, psep;
+    QM pki;
+    float axis, ia_ax, ib_ax, px, py;
+    float axial, maxt, target, speed, lower, upper;
+    QM ss;                 /* the spring's softness */
+    float spring_imp, motor_imp, lower_imp, upper_imp, perp_x, perp_y;
+    float kxx, kxy, kyy, kinv, tw, relx, rely;
+};
+/* The row's delta-pose geometry (quad_joint_geometry). */
+B3Q_FN void jq_geometry(const QLane& Q, JQ* r) {
+    const float* g = lrow(Q, Q.q.jgeo + r->j * kJGWords);
+    const float* v = g + Q.sub * kRow;
+    r->ra = v[JG_RA * kRow];
+    r->rb = v[JG_RB * kRow];
+    r->psep = v[JG_PSEP * kRow];
+    r->pki = QM{v[JG_PKI * kRow], v[(JG_PKI + 3) * kRow], v[(JG_PKI + 6) * kRow]};
+    if (r->info & JF_WELD) {
+        r->py = v[JG_CV * kRow];
+        return;
+    }
+    r->px = v[JG_PX * kRow];
+    r->py = v[JG_PY * kRow];
+    r->kxx = g[JG_KXX * kRow];
+    r->kxy = g[JG_KXY * kRow];
+    r->kyy = g[JG_KYY * kRow];
+    r->kinv = g[JG_KINV * kRow];
+    r->tw = g[JG_TW * kRow];
+    r->relx = g[JG_RELX * kRow];
+    r->rely = g[JG_RELY * kRow];
+}
+B3Q_FN void jq_load(const QLane& Q, int j, JQ* r) {
+    const Lane& L = Q.L;
+    const uint32_t* w = L.w;
+    const uint32_t* rec = joint_rec(L, j);
+    int k = Q.sub < 3 ? Q.sub : 2;     /* lane 3 reads what lane 2 does */
+    auto v = [w, k, &L, j](int f) { return ldf(w, jw(L, j, f + k)); };
+    auto s = [w, &L, j](int f) { return ldf(w, jw(L, j, f)); };
+    uint32_t ab = ldu(rec, JS_AB);
+    int a = (int)(ab & 0xffffu), b = (int)(ab >> 16);
+    r->j = j;
+    r->lev = lgeti(Q, Q.q.jlev + j);
+    r->info = ldi(rec, JS_INFO) | (is_dyn_flag(L, a) ? kQDynA : 0) | (is_dyn_flag(L, b) ? kQDynB : 0);
+    r->va = qvel_row(a);
+    r->vb = qvel_row(b);
+    r->ma = s(J_INV_MASS_A);
+    r->mb = s(J_INV_MASS_B);
+    r->ia = QM{v(J_INV_I_A), v(J_INV_I_A + 3), v(J_INV_I_A + 6)};
+    r->ib = QM{v(J_INV_I_B), v(J_INV_I_B + 3), v(J_INV_I_B + 6)};
+    r->soft = ldsoft(w, jw(L, j, J_SOFTNESS));
+    r->lin_imp = v(J_LINEAR_IMPULSE);
+    r->kxx = r->kxy = r->kyy = r->kinv = r->tw = r->relx = r->rely = 0.0f;
+    r->spring_imp = r->motor_imp = r->lower_imp = r->upper_imp = r->perp_x = r->perp_y = r->upper = 0.0f;
+    if (r->info & JF_WELD) {
+        r->axis = v(J_ANGULAR_IMPULSE);
+        r->ia_ax = v(J_ANGULAR_MASS);
+        r->ib_ax = v(J_ANGULAR_MASS + 3);
+        r->px = v(J_ANGULAR_MASS + 6);
+        r->axial = s(J_LINEAR_HERTZ);
+        r->maxt = s(J_ANGULAR_HERTZ);
+        r->target = s(J_LINEAR_SPRING);
+        r->ss.x = s(J_LINEAR_SPRING + 1);
+        r->ss.y = s(J_LINEAR_SPRING + 2);
+        r->ss.z = s(J_ANGULAR_SPRING);
+        r->speed = s(J_ANGULAR_SPRING + 1);
+        r->lower = s(J_ANGULAR_SPRING + 2);
+    } else {
+        r->axis = v(J_ROTATION_AXIS);
+        r->ia_ax = ldf(rec, JS_IAX + k);
+        r->ib_ax = ldf(rec, JS_IBX + k);
+        r->axial = s(J_AXIAL_MASS);
+        r->maxt = s(J_MAX_MOTOR_TORQUE);
+        r->target = s(J_TARGET_ANGLE);
+        r->ss = QM{s(J_SPRING_SOFTNESS), s(J_SPRING_SOFTNESS + 1), s(J_SPRING_SOFTNESS + 2)};
+        r->speed = s(J_MOTOR_SPEED);
+        r->lower = s(J_LOWER_ANGLE);
+        r->upper = s(J_UPPER_ANGLE);
+        r->spring_imp = s(J_SPRING_IMPULSE);
+        r->motor_imp = s(J_MOTOR_IMPULSE);
+        r->lower_imp = s(J_LOWER_IMPULSE);
+        r->upper_imp = s(J_UPPER_IMPULSE);
+        r->perp_x = s(J_PERP_IMPULSE);
+        r->perp_y = s(J_PERP_IMPULSE + 1);
+    }
+    jq_geometry(Q, r);
+}
+
+/* The joint's warm start (b3_warm_start_joints, 06:204-239), at the start of
+ * the step: the anchors at the initial delta poses, the hinge rows as
+ * b3_prepare_joints left them in the world. */
+B3Q_FN void jq_warm(const QLane& Q, const JQ& r) {
+    const Lane& L = Q.L;
+    int k = Q.sub < 3 ? Q.sub : 2;
+    float ang;
+    if (ldi(L.w, jw(L, r.j, J_TYPE)) != kJointRevolute) {
+        ang = ldf(L.w, jw(L, r.j, J_ANGULAR_IMPULSE + k));
+    } else {
+        float axial = r.spring_imp + r.motor_imp + r.lower_imp - r.upper_imp;
+        float px = ldf(L.w, jw(L, r.j, J_PERP_X + k)), py = ldf(L.w, jw(L, r.j, J_PERP_Y + k));
+        ang = px * r.perp_x + py * r.perp_y;
+        ang = ang + axial * r.axis;
+    }
+    QVel x = qvel_load(Q, r.va, r.vb);
+    x.va = x.va - r.ma * r.lin_imp;
+    x.wa = x.wa - qmv(r.ia, qcross(r.ra, r.lin_imp) + ang);
+    x.vb = x.vb + r.mb * r.lin_imp;
+    x.wb = x.wb + qmv(r.ib, qcross(r.rb, r.lin_imp) + ang);
+    qvel_store(Q, r.va, r.vb, r.info, x);
+}
+
+/* One joint's solve: b3_solve_revolute (06:436-642) or b3_solve_weld
+ * (06:285-332), as solve_revolute and solve_weld. */
+template <bool Bias>
+B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
+    QVel x = qvel_load(Q, r.va, r.vb);
+    const bool fixed = (r.info & JF_FIXED) != 0;
+    Soft psoft = r.soft;
+    bool pbias = Bias;
+    if (r.info & JF_WELD) {
+        if (!fixed) {
+            float bias = 0.0f, mscale = 1.0f, iscale = 0.0f;
+            if (Bias || r.maxt > 0.0f) {
+                bias = r.py * r.ss.z;
+                mscale = r.speed;
+                iscale = r.lower;
+            }
+            float cdot = x.wb - x.wa;
+            float impulse = qmv(QM{r.ia_ax, r.ib_ax, r.px}, cdot + bias) * -mscale - iscale * r.axis;
+            r.axis = r.axis + impulse;
+            x.wa = x.wa - qmv(r.ia, impulse);
+            x.wb = x.wb + qmv(r.ib, impulse);
+        }
+        pbias = Bias || r.axial > 0.0f;
+        psoft.bias_rate = r.target;
+        psoft.mass_scale = r.ss.x;
+        psoft.impulse_scale = r.ss.y;
+    } else if (!fixed) {
+        if (r.info & JF_SPRING) {
+            float bias = r.ss.x * (r.tw - r.target);
+            float cdot = qdot3(x.wb - x.wa, r.axis);
+            float old = r.spring_imp;
+            float dimp = -r.ss.y * r.axial * (cdot + bias) - r.ss.z * old;
+            float nimp = old + dimp;
+            if (r.maxt > 0.0f) {
+                float maxp = r.maxt * h;
+                nimp = clampf(nimp, -maxp, maxp);
+            }
+            dimp = nimp - old;
+            r.spring_imp = nimp;
+            x.wa = x.wa - dimp * r.ia_ax;
+            x.wb = x.wb + dimp * r.ib_ax;
+        }
+        if (r.info & JF_MOTOR) {
+            bool blocked = false;
+            if (r.info & JF_LIMIT) {
+                if (r.tw >= r.upper - 0.01f && r.speed > 0.0f) blocked = true;
+                if (r.tw <= r.lower + 0.01f && r.speed < 0.0f) blocked = true;
+            }
+            if (blocked) {
+                r.motor_imp = 0.0f;
+            } else {
+                float old = r.motor_imp;
+                float cdot = qdot3(x.wb - x.wa, r.axis) - r.speed;
+                float dimp = -r.axial * cdot;
+                float nimp = old + dimp;
+                float maxp = r.maxt * h;
+                nimp = clampf(nimp, -maxp, maxp);
+                dimp = nimp - old;
+                r.motor_imp = nimp;
+                x.wa = x.wa - dimp * r.ia_ax;
+                x.wb = x.wb + dimp * r.ib_ax;
+            }
+        }
+        if (r.info & JF_LIMIT) {
+            float old = r.lower_imp;
+            float lo = limit_impulse(r.tw - r.lower, qdot3(x.wb - x.wa, r.axis), inv_h, Bias, r.soft, r.axial, old);
+            r.lower_imp = lo;
+            float dimp = lo - old;
+            x.wa = x.wa - dimp * r.ia_ax;
+            x.wb = x.wb + dimp * r.ib_ax;
+            old = r.upper_imp;
+            float up = limit_impulse(r.upper - r.tw, qdot3(x.wa - x.wb, r.axis), inv_h, Bias, r.soft, r.axial, old);
+            r.upper_imp = up;
+            dimp = up - old;
+            x.wa = x.wa + dimp * r.ia_ax;
+            x.wb = x.wb - dimp * r.ib_ax;
+        }
+        V2 bias;
+        bias.x = 0.0f;
+        bias.y = 0.0f;
+        float mscale = 1.0f, iscale = 0.0f;
+        if (Bias) {
+            bias.x = r.soft.bias_rate * r.relx;
+            bias.y = r.soft.bias_rate * r.rely;
+            mscale = r.soft.mass_scale;
+            iscale = r.soft.impulse_scale;
+        }
+        float wrel = x.wb - x.wa;
+        V2 rhs;
+        rhs.x = qdot3(wrel, r.px) + bias.x;
+        rhs.y = qdot3(wrel, r.py) + bias.y;
+        V2 sol;
+        sol.x = 0.0f;
+        sol.y = 0.0f;
+        if (r.kinv == r.kinv) {
+            sol.x = r.kinv * (r.kyy * rhs.x - r.kxy * rhs.y);
+            sol.y = r.kinv * (-r.kxy * rhs.x + r.kxx * rhs.y);
+        }
+        V2 dimp;
+        dimp.x = -mscale * sol.x - iscale * r.perp_x;
+        dimp.y = -mscale * sol.y - iscale * r.perp_y;
+        r.perp_x = r.perp_x + dimp.x;
+        r.perp_y = r.perp_y + dimp.y;
+        float ang = r.px * dimp.x + r.py * dimp.y;
+        x.wa = x.wa - qmv(r.ia, ang);
+        x.wb = x.wb + qmv(r.ib, ang);
+    }
+    /* the point rows (06:257-282) */
+    float cdot = (x.vb + qcross(x.wb, r.rb)) - (x.va + qcross(x.wa, r.ra));
+    float bias = 0.0f, mscale = 1.0f, iscale = 0.0f;
+    if (pbias) {
+        bias = r.psep * psoft.bias_rate;
+        mscale = psoft.mass_scale;
+        iscale = psoft.impulse_scale;
+    }
+    float impulse = qmv(r.pki, cdot + bias) * -mscale - iscale * r.lin_imp;
+    r.lin_imp = r.lin_imp + impulse;
+    qimpulse(&x, r.ma, r.ia, r.mb, r.ib, r.ra, r.rb, impulse);
+    qvel_store(Q, r.va, r.vb, r.info, x);
+}
+
+/* A row's impulses, and a hinge's latest perpendicular rows, to the world
+ * (joint_writeback, joint_geometry). */
+B3Q_FN void jq_writeback(const QLane& Q, const JQ& r) {
+    const Lane& L = Q.L;
+    uint32_t* w = L.w;
+    auto put3 = [w, &L, &r, &Q](int f, float x) { if (Q.sub < 3) stf(w, jw(L, r.j, f + Q.sub), x); };
+    auto put = [w, &L, &r, &Q](int f, float x) { if (Q.sub == 0) stf(w, jw(L, r.j, f), x); };
+    put3(J_LINEAR_IMPULSE, r.lin_imp);
+    if (r.info & JF_FIXED) return;
+    if (r.info & JF_WELD) {
+        put3(J_ANGULAR_IMPULSE, r.axis);
+        return;
+    }
+    put3(J_PERP_X, r.px);
+    put3(J_PERP_Y, r.py);
+    put(J_PERP_IMPULSE, r.perp_x);
+    put(J_PERP_IMPULSE + 1, r.perp_y);
+    if (r.info & JF_SPRING) put(J_SPRING_IMPULSE, r.spring_imp);
+    if (r.info & JF_MOTOR) put(J_MOTOR_IMPULSE, r.motor_imp);
+    if (r.info & JF_LIMIT) {
+        put(J_LOWER_IMPULSE, r.lower_imp);
+        put(J_UPPER_IMPULSE, r.upper_imp);
+    }
+}
+
+/* ---- the step ---- */
+
+/* The wave's contacts of one level: those in registers whose level it is,
+ * then those past them in the order (pointer *at), loaded and stored. */
+template <int CR, class Solve>
+B3Q_FN void quad_level(const QLane& Q, CQ (&row)[CR], int cc, int lev, int* at, Solve solve) {
+#pragma unroll
+    for (int i = 0; i < CR; i++)
+        if (row[i].lev == lev) solve(row[i]);
+    while (*at < cc) {
+        int e = lgeti(Q, Q.q.order + *at);
+        if ((e >> 10) != lev) break;
+        CQ r;
+        cq_load(Q, e, &r);
+        r.sep = cq_separations(Q, r, cq_base(Q, r));
+        solve(r);
+        cq_store(Q, r);
+        *at += kQuadWaves;
+    }
+}
+
+/* One b3_step (09_step.inl:148-264, default configuration) of the
+ * workgroup's worlds.  Every thread runs it and meets every barrier; lanes
+ * of worlds that do not step (L.active false) have no items.  `wg`: the
+ * workgroup's words, zero at entry, as are the hit bits; a barrier has
+ * passed since. */
+template <int CR, int JR>
+B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
+    Lane& L = Q.L;
+    const bool act = L.active;
+    int subs = substeps < 1 ? 1 : substeps;
+    float h = dt / (float)subs;
+    float inv_dt = 1.0f / dt;
+    float inv_h = (float)subs * inv_dt;
+    float hertz = minf(ldf(L.w, H_CONTACT_HERTZ), 0.25f * inv_h);
+    float damping = ldf(L.w, H_CONTACT_DAMPING);
+    Soft cs = make_soft(hertz, damping, h);
+    Soft ss = make_soft(2.0f * hertz, 0.5f * damping, h);
+    float contact_speed = ldf(L.w, H_CONTACT_SPEED);
+    float rest_threshold = ldf(L.w, H_RESTITUTION_THRESHOLD);
+    int old_n = act ? clampi(ldi(L.w, H_CONTACT_COUNT), 0, L.g.max_c) : 0;
+    int ns = act ? clampi(ldi(L.w, H_SHAPE_COUNT), 0, L.g.max_s) : 0;
+    count_bodies_and_joints(L);
+    const int nb = L.nb, nj = L.nj;
+
+    quad_open(Q, old_n, ns, nj);
+    B3D_BARRIER();
+    quad_overlaps(Q, ns);
+    B3D_BARRIER();
+    quad_collide(Q, ns, nj, old_n);
+    B3D_BARRIER();
+    int cc = 0;
+    if (act) {
+        cc = quad_append(Q, old_n, cs, ss, wg);
+        body_prepass(L, h, Q.worker, kQuadWorkers);
+        prepare_joints(L, h, Q.worker, kQuadWorkers);
+    }
+    B3D_BARRIER();
+    if (act) {
+        if (Q.worker == 0) quad_levels(Q, cc, nb, wg);
+        if (Q.worker == 4) quad_joint_levels(Q, nj, nb, wg);
+        if (Q.worker >= 8) quad_joint_geometry(Q, nj, Q.worker - 8, kQuadWorkers - 8);
+    }
+    B3D_BARRIER();
+    const int nlev = __builtin_amdgcn_readfirstlane(wg[WG_LEVELS]);
+    const int njlev = __builtin_amdgcn_readfirstlane(wg[WG_JLEVELS]);
+    const int njmax = __builtin_amdgcn_readfirstlane(wg[WG_JOINTS]);
+    const bool rest = __builtin_amdgcn_readfirstlane(wg[WG_REST]) != 0;
+    CQ row[CR];
+    float base[CR];
+#pragma unroll
+    for (int i = 0; i < CR; i++) {
+        int at = i * kQuadWaves + Q.wave;
+        row[i].c = -1;
+        row[i].lev = 0;
+        if (at < cc) {
+            cq_load(Q, lgeti(Q, Q.q.order + at), &row[i]);
+            base[i] = cq_base(Q, row[i]);
+        }
+    }
+    JQ joint[JR];
+#pragma unroll
+    for (int i = 0; i < JR; i++) {
+        int j = i * kQuadWaves + Q.wave;
+        joint[i].j = -1;
+        joint[i].lev = 0;
+        if (j < nj) jq_load(Q, j, &joint[i]);
+    }
+    const int past = CR * kQuadWaves + Q.wave;   /* the wave's first contact not in registers */
+    auto levels = [&](auto solve) {
+        int at = past;
+        for (int lev = 1; lev <= nlev; lev++) {
+            quad_level<CR>(Q, row, cc, lev, &at, solve);
+            B3D_BARRIER();
+        }
+    };
+    auto joint_levels = [&](auto solve) {
+        for (int lev = 1; lev <= njlev; lev++) {
+#pragma unroll
+            for (int i = 0; i < JR; i++)
+                if ((joint[i].lev & 255) == lev || (joint[i].lev >> 8) == lev) solve(joint[i]);
+            B3D_BARRIER();
+        }
+    };
+    auto separations = [&]() {
+#pragma unroll
+        for (int i = 0; i < CR; i++)
+            if (row[i].lev > 0) row[i].sep = cq_separations(Q, row[i], base[i]);
+    };
+    separations();
+    levels([&](CQ& r) { cq_warm(Q, r); });
+    for (int j = 0; j < njmax; j++) {
+#pragma unroll
+        for (int i = 0; i < JR; i++)
+            if (joint[i].j == j) jq_warm(Q, joint[i]);
+        B3D_BARRIER();
+    }
+    for (int s = 0; s < subs; s++) {
+        if (act) integrate_velocities(L, Q.worker, kQuadWorkers);
+        B3D_BARRIER();
+        levels([&](CQ& r) { cq_solve<false>(Q, r, inv_h, contact_speed, cs, ss); });
+        joint_levels([&](JQ& r) { jq_solve<true>(Q, r, h, inv_h); });
+        if (act) integrate_positions(L, h, inv_dt, Q.worker, kQuadWorkers);
+        B3D_BARRIER();
+        if (njmax > 0) {
+            quad_joint_geometry(Q, nj, Q.worker, kQuadWorkers);
+            B3D_BARRIER();
+#pragma unroll
+            for (int i = 0; i < JR; i++)
+                if (joint[i].j >= 0) jq_geometry(Q, &joint[i]);
+        }
+        separations();
+        levels([&](CQ& r) { cq_solve<true>(Q, r, inv_h, contact_speed, cs, ss); });
+        joint_levels([&](JQ& r) { jq_solve<false>(Q, r, h, inv_h); });
+        if (rest) levels([&](CQ& r) { cq_restitution(Q, r, rest_threshold); });
+    }
+#pragma unroll
+    for (int i = 0; i < CR; i++)
+        if (row[i].lev > 0) cq_writeback(Q, row[i]);
+    for (int at = past; at < cc; at += kQuadWaves) {
+        CQ r;
+        cq_load(Q, lgeti(Q, Q.q.order + at), &r);
+        cq_writeback(Q, r);
+    }
+#pragma unroll
+    for (int i = 0; i < JR; i++)
+        if (joint[i].j >= 0) jq_writeback(Q, joint[i]);
+    if (act) {
+        finalize(L, Q.worker, kQuadWorkers);
+        vel_store(L, Q.worker, kQuadWorkers);
+    }
+}
+
+}  // namespace b3d
+
+#endif
