@@ -167,9 +167,9 @@ def joint_impulses_fit(max_b, max_s, max_c, max_j):
 
 def kernel_name(scene, count):
     """The step kernel a batch launches (b3_engine_create): b3k_step<JI, true>
-    for worlds of at most two shapes; else b3k_step_quad<CR, JR> up to a
-    quarter tile per CU, b3k_step_shared<Masks, JL> when the tiles fit one
-    per CU, b3k_step<JI, false> when they do not."""
+    for worlds of at most two shapes; else b3k_step_quad<W, CR, JR> up to a
+    quarter (W = 8) or half a tile (4) per CU, b3k_step_shared<Masks, JL>
+    when the tiles fit one per CU, b3k_step<JI, false> when they do not."""
     import torch
     from puffysics_amd import scenes
     tiles = (count + 63) // 64
@@ -177,8 +177,10 @@ def kernel_name(scene, count):
     caps = scenes.SCENES[scene].caps
     if caps[1] <= 2:                 # one candidate pair: b3k_step<JI, true> at any batch size
         return "b3k_step<%s, true>" % ("true" if joint_impulses_fit(*caps) else "false")
-    if 4 * tiles <= cus:             # every benchmark family fits quad_layout
-        return "b3k_step_quad<2, %d>" % (1 if caps[3] <= 8 else 2)
+    if 4 * tiles <= cus:             # every benchmark family fits quad_layout at eight waves
+        return "b3k_step_quad<8, 2, %d>" % (1 if caps[3] <= 8 else 2)
+    if 2 * tiles <= cus and caps[1] <= 32:
+        return "b3k_step_quad<4, %s>" % ("3, 1" if caps[3] <= 4 else "2, 2" if caps[3] <= 8 else "1, 4")
     if tiles > cus:
         return "b3k_step<%s, false>" % ("true" if joint_impulses_fit(*caps) else "false")
     masks = 12 <= caps[1] <= 64

@@ -128,10 +128,10 @@ hipError_t b3_engine_device_view(const B3Engine* engine, void** tiles, size_t* w
  * hipErrorNotSupported while it is on. */
 #define B3_ENGINE_ART_CONTACTS 2u
 /* B3_ENGINE_ONE_WAVE_PER_TILE: no counterpart in the reference (a launch
- * choice).  A batch of at most a quarter of a 64-world tile per CU normally
- * runs with four workgroups per tile, each of eight waves that give every
- * world four lanes each (a contact or joint solve to four lanes, everything
- * independent within a world spread over all 32).  A batch of at most one
+ * choice).  A batch of at most a quarter (half) of a 64-world tile per CU
+ * normally runs with four workgroups per tile, each of eight (four) waves
+ * that give every world four lanes each (a contact or joint solve to four
+ * lanes, everything independent within a world spread over all of them).  A batch of at most one
  * tile per CU runs with eight waves per tile, one lane of each to a world:
  * they share the narrowphase (its pairs are independent; four to seven
  * waves collide, as many as have LDS rows for their clip polygons), the

@@ -489,17 +489,23 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
         size_t quad_scratch = 0;
         /* A quarter tile per workgroup fills the CUs at a quarter tile per
          * CU: up to there each world of three shapes or more steps on a quad
-         * of lanes of each of eight waves (b3d_quad.h).  Measured at 4,096
-         * worlds (64 tiles), the shared step -> quads: stacks 241 -> 132 us,
-         * chains 398 -> 163, bin 713 -> 467, the arm 320 -> 144 (and at 300
-         * worlds 347 -> 143).  A second round of workgroups takes as long
-         * again: at 8,192 worlds the chains and the arm would gain (404 ->
-         * 316, 334 -> 267), the others lose (stacks 208 -> 258, bin 794 ->
-         * 867), and past that all lose.  Of two-shape worlds those with a
-         * contact gain (hover 37.5 -> 30.1 us) and those without lose to the
-         * barriers (a free sphere's step and task 23.9 -> 28.1). */
-        e->quad = g.max_s > 2 && 4 * e->tiles <= cus && b3i_quad_fit(g, &quad_scratch);
-        if (e->quad || (e->tiles <= cus && shared_lds <= kCuLdsBytes && g.max_s > 2)) {
+         * of lanes of each of eight waves (b3d_quad.h), and up to half a tile
+         * per CU, two workgroups to a CU, of four waves (where their LDS
+         * fits: not the bin).  Measured, the shared step -> quads, us: at
+         * 4,096 worlds (64 tiles) stacks 207 -> 91, chains 395 -> 153, bin
+         * 686 -> 395, the arm 320 -> 131 (at 300 worlds 313 -> 117); at
+         * 8,192 stacks 211 -> 132, chains 405 -> 210, the arm 336 -> 225.
+         * With more workgroups than the CUs hold at once the shared step
+         * wins: at 16,384 worlds stacks 234 against 243, the arm 398
+         * against 442 (chains 430 against 408).  Of two-shape worlds those
+         * with a contact gain (hover 34.9 -> 26.3 at 4,096) and those without
+         * lose to the barriers (a free sphere's step and task 23.9 -> 28.1). */
+        e->quad_waves = 0;
+        if (g.max_s > 2) {
+            if (4 * e->tiles <= cus && b3i_quad_fit(g, 8, &quad_scratch)) e->quad_waves = 8;
+            else if (4 * e->tiles <= 2 * cus && b3i_quad_fit(g, 4, &quad_scratch)) e->quad_waves = 4;
+        }
+        if (e->quad_waves || (e->tiles <= cus && shared_lds <= kCuLdsBytes && g.max_s > 2)) {
             size_t max_cand = (size_t)g.max_s * (size_t)(g.max_s - 1) / 2;
             size_t stage_words = max_cand * kStageWords;
             if ((size_t)stage_sched_words(g) > stage_words) stage_words = (size_t)stage_sched_words(g);
@@ -517,7 +523,7 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
              * (16); the stacks 0.228 -> 0.218 (32) -> 0.223 (16); the hover
              * (4 contacts, 2 joints) 0.040 -> 0.041 and the chains (32, 8)
              * 0.394 -> 0.397 -> 0.443, which stay at 64. */
-            if (e->quad) e->tile_parts = 1;
+            if (e->quad_waves) e->tile_parts = 1;
             else if (e->shared_masks && 4 * e->tiles <= cus) e->tile_parts = 4;
             else if (e->shared_masks && 2 * e->tiles <= cus) e->tile_parts = 2;
             else if (g.max_c > 4 * g.max_j && 2 * e->tiles <= cus) e->tile_parts = 2;
@@ -530,7 +536,7 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
         }
         /* per-step scratch: one per workgroup of a tile */
         size_t scratch_words = (size_t)e->tile_parts * g.tile_scr_words;
-        if (e->quad && quad_scratch > scratch_words) scratch_words = quad_scratch;
+        if (e->quad_waves && quad_scratch > scratch_words) scratch_words = quad_scratch;
         err = hipMalloc((void**)&e->scratch, (size_t)e->tiles * scratch_words * 4);
         if (err != hipSuccess) {
             (void)b3_engine_destroy(e);
@@ -640,7 +646,7 @@ hipError_t b3_batch_step_gpu(B3Engine* e, float dt, int substeps, const unsigned
     if (err != hipSuccess) return err;
     if (dt == 0.0f) return reset_mask ? b3_batch_restore_gpu(e, reset_mask, stream) : hipSuccess;
     if (e->options & B3_ENGINE_ART_CONTACTS) return b3i_step_art(e, dt, substeps, step_mask, reset_mask, stream);
-    if (e->quad && !(e->options & B3_ENGINE_ONE_WAVE_PER_TILE))
+    if (e->quad_waves && !(e->options & B3_ENGINE_ONE_WAVE_PER_TILE))
         return b3i_step_quad(e, dt, substeps, step_mask, reset_mask, stream);
     if (e->pair_stage && !(e->options & B3_ENGINE_ONE_WAVE_PER_TILE)) {
         auto kernel = e->shared_masks ? (e->joint_lds ? b3k_step_shared<true, true> : b3k_step_shared<true, false>)

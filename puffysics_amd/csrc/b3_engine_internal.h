@@ -30,7 +30,8 @@ struct B3Engine {
     bool joint_lds;          /* ... and keep the joint rows in LDS (b3d::joint_rows_fit) */
     int tile_parts;          /* workgroups per tile of the shared step (1, 2 or 4), each with its own
                                 scratch and stage */
-    bool quad;               /* the step on quads of lanes (b3d_quad.h), a quarter tile to a workgroup */
+    int quad_waves;          /* the step on quads of lanes (b3d_quad.h), a quarter tile to a workgroup of so
+                                many waves; 0: another step */
     bool joint_impulses_lds; /* the one-wave step keeps the joint impulses in LDS (b3d::ji_fit) */
 };
 
@@ -56,10 +57,10 @@ hipError_t b3i_art_init(B3Engine* e);
 hipError_t b3i_step_art(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
     const unsigned char* reset_mask, hipStream_t stream);
 
-/* The step on quads (b3_quad.hip): whether it takes worlds of geometry g,
- * with the scratch words it needs per tile; its set-up on the current
+/* The step on quads (b3_quad.hip): whether it takes worlds of geometry g in
+ * workgroups of `waves` waves, with the scratch words it needs per tile; its set-up on the current
  * device; its launch. */
-bool b3i_quad_fit(const b3d::Geometry& g, size_t* scratch_tile_words);
+bool b3i_quad_fit(const b3d::Geometry& g, int waves, size_t* scratch_tile_words);
 hipError_t b3i_quad_init();
 hipError_t b3i_step_quad(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
     const unsigned char* reset_mask, hipStream_t stream);

@@ -17,10 +17,10 @@ namespace {
  * world a chain of eight hinges (4,096 worlds) took 391 us, 292 of them in
  * 160 levels of joint solves at 1.83 us (a solve's ~400 instructions and
  * ~90 row loads at ~5 cycles each, a wave alone on its SIMD); on quads with
- * the rows in registers 163 us.  CR, JR: contacts and joints of a world
- * that a wave keeps in registers. */
-template <int CR, int JR>
-__global__ __launch_bounds__(64 * kQuadWaves) void b3k_step_quad(uint32_t* live, const uint32_t* snap,
+ * the rows in registers 163 us.  W: waves of the workgroup; CR, JR: contacts
+ * and joints of a world that a wave keeps in registers. */
+template <int W, int CR, int JR>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) void b3k_step_quad(uint32_t* live, const uint32_t* snap,
         uint32_t* scratch, uint32_t* stage, size_t stage_tile_words, Geometry g, QuadLayout q, int count, float dt,
         int substeps, const unsigned char* step_mask, const unsigned char* reset_mask, unsigned int opts) {
     extern __shared__ float lds[];
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(64 * kQuadWaves) void b3k_step_quad(uint32_t* live,
     int col = lane >> 2, slot = part * kQuadCols + col;
     if (reset_mask) {
         uint64_t mine = ((1ull << kQuadCols) - 1) << (part * kQuadCols);
-        restore_tile(live, snap, g, count, reset_mask, tile, wave, kQuadWaves, mine);
+        restore_tile(live, snap, g, count, reset_mask, tile, wave, W, mine);
     }
     int w = tile * 64 + slot;
     bool stepping = w < count && (!step_mask || step_mask[w]);
@@ -40,6 +40,8 @@ __global__ __launch_bounds__(64 * kQuadWaves) void b3k_step_quad(uint32_t* live,
     Q.sub = lane & 3;
     Q.wave = wave;
     Q.worker = wave * 4 + Q.sub;
+    Q.waves = W;
+    Q.workers = 4 * W;
     Q.q = q;
     Q.lds = lds + kQuadWgWords + col;
     uint32_t* tile_scratch = scratch + (size_t)tile * q.scratch_tile_words;
@@ -52,36 +54,45 @@ __global__ __launch_bounds__(64 * kQuadWaves) void b3k_step_quad(uint32_t* live,
     Q.L.vel = Q.lds + q.y * kRow;
     Q.L.active = stepping;
     if (threadIdx.x < kQuadWgWords) wg[threadIdx.x] = 0;
-    for (int k = Q.worker; k <= hit_words(g); k += kQuadWorkers) lseti(Q, q.hits + k, 0);
+    for (int k = Q.worker; k <= hit_words(g); k += 4 * W) lseti(Q, q.hits + k, 0);
     __syncthreads();
     quad_step<CR, JR>(Q, dt, substeps, wg);
 }
 
-/* Contacts of a world a wave keeps in registers. */
-constexpr int kKeptContacts = 2;
+using QuadKernel = void (*)(uint32_t*, const uint32_t*, uint32_t*, uint32_t*, size_t, Geometry, QuadLayout, int, float,
+    int, const unsigned char*, const unsigned char*, unsigned int);
+QuadKernel quad_kernel(int waves, int max_j) {
+    if (waves == 8) return max_j <= 8 ? b3k_step_quad<8, 2, 1> : b3k_step_quad<8, 2, 2>;
+    return max_j <= 4 ? b3k_step_quad<4, 3, 1> : (max_j <= 8 ? b3k_step_quad<4, 2, 2> : b3k_step_quad<4, 1, 4>);
+}
+
+size_t quad_lds_bytes(int waves) { return kCuLdsBytes * waves / 8; }
 
 }  // namespace
 
-bool b3i_quad_fit(const Geometry& g, size_t* scratch_tile_words) {
+bool b3i_quad_fit(const Geometry& g, int waves, size_t* scratch_tile_words) {
     QuadLayout q;
-    if (!quad_layout(g, 2 * kQuadWaves, &q)) return false;
+    if (!quad_layout(g, waves, quad_lds_bytes(waves), &q)) return false;
     *scratch_tile_words = q.scratch_tile_words;
     return true;
 }
 
 hipError_t b3i_quad_init() {
-    hipError_t err = b3i_lds_limit((const void*)b3k_step_quad<kKeptContacts, 1>);
-    if (err == hipSuccess) err = b3i_lds_limit((const void*)b3k_step_quad<kKeptContacts, 2>);
-    return err;
+    for (int waves = 4; waves <= 8; waves += 4)
+        for (int max_j = 4; max_j <= 16; max_j += 4) {
+            hipError_t err = b3i_lds_limit((const void*)quad_kernel(waves, max_j));
+            if (err != hipSuccess) return err;
+        }
+    return hipSuccess;
 }
 
 hipError_t b3i_step_quad(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
         const unsigned char* reset_mask, hipStream_t stream) {
     QuadLayout q;
-    if (!quad_layout(e->g, 2 * kQuadWaves, &q)) return hipErrorInvalidValue;
-    auto kernel = e->g.max_j <= kQuadWaves ? b3k_step_quad<kKeptContacts, 1> : b3k_step_quad<kKeptContacts, 2>;
+    if (!quad_layout(e->g, e->quad_waves, quad_lds_bytes(e->quad_waves), &q)) return hipErrorInvalidValue;
+    QuadKernel kernel = quad_kernel(e->quad_waves, e->g.max_j);
     size_t lds = ((size_t)kQuadWgWords + (size_t)q.words * kQuadCols) * sizeof(float);
-    kernel<<<e->tiles * 4, 64 * kQuadWaves, lds, stream>>>(e->live, e->snap, e->scratch, e->pair_stage,
+    kernel<<<e->tiles * 4, 64 * e->quad_waves, lds, stream>>>(e->live, e->snap, e->scratch, e->pair_stage,
         e->stage_tile_words, e->g, q, e->count, dt, substeps, step_mask, reset_mask, e->options);
     return hipGetLastError();
 }

@@ -2,9 +2,9 @@
  * b3d_quad.h - one world's step on four lanes of each of a workgroup's
  * waves, for batches that leave most of the chip idle at one lane a world.
  *
- * A workgroup of kQuadWaves waves steps kQuadCols = 16 worlds, a quarter of
+ * A workgroup of W (8 or 4) waves steps kQuadCols = 16 worlds, a quarter of
  * a 64-world tile: lanes 4c .. 4c + 3 of every wave belong to world c, so a
- * world has 4 * kQuadWaves = 32 lanes ("workers").  Two ways of using them:
+ * world has 4 W lanes ("workers").  Two ways of using them:
  *   - what is independent within a world (shapes, candidate pairs, contact
  *     preparation, body updates, joint geometry) goes one item to a worker,
  *     through the same scalar functions as the other steps (b3d_lane.h with
@@ -22,8 +22,7 @@
  * same.
  *
  * Each wave owns contacts and joints for the whole step: joint j is wave
- * j mod kQuadWaves', contact number i in level order wave i mod
- * kQuadWaves', and the owner keeps its rows in registers over all sweeps
+ * j mod W's, contact number i in level order wave i mod W's, and the owner keeps its rows in registers over all sweeps
  * (the first CR contacts and JR joints of a wave; further contacts are
  * loaded from their records for each solve).  The velocities are in LDS;
  * levels of contacts and of joint solves on disjoint dynamic bodies
@@ -75,21 +74,25 @@ B3Q_FN float qrot(float q, float v) {
  * the new contacts' heads.  Region Y, while contacts are generated: shape
  * bounds, overlap masks, old contact keys and the colliding workers' clip
  * rows; afterwards the bodies' rows (quad_body_rows). */
-constexpr int kQuadCols = B3D_ROW, kQuadWaves = 8, kQuadWorkers = 4 * kQuadWaves;
-constexpr int kQuadLdsWords = 160 * 1024 / 4 / kQuadCols;
+constexpr int kQuadCols = B3D_ROW;
 /* words of the workgroup (not per world) at the start of LDS */
 constexpr int WG_LEVELS = 0, WG_JLEVELS = 1, WG_JOINTS = 2, WG_REST = 3, kQuadWgWords = 16;
-/* joint geometry rows (struct JGeo) */
-constexpr int JG_TW = 0, JG_RELX = 1, JG_RELY = 2, JG_KXX = 3, JG_KXY = 4, JG_KYY = 5, JG_KINV = 6, JG_PX = 7,
-              JG_PY = 10, JG_RA = 13, JG_RB = 16, JG_PSEP = 19, JG_CV = 22, JG_PKI = 25, kJGWords = 35;
+/* joint geometry quads (struct JGeo): a vector and a scalar each; a weld's
+ * angular error is in JG_PY */
+enum { JG_RA_TW, JG_RB_RELX, JG_PSEP_RELY, JG_PX_KXX, JG_PY_KXY, JG_K0_KYY, JG_K1_KINV, JG_K2, kJGQuads };
+constexpr int kJGWords = 4 * kJGQuads;
+/* what a joint's geometry reads besides the delta poses, fixed for the step */
+constexpr int JC_AB = 0, JC_INFO = 1, JC_QA = 2, JC_QB = 6, JC_PA = 10, JC_PB = 13, JC_DC = 16, JC_MA = 19, JC_MB = 20,
+              JC_IA = 21, JC_IB = 30, kJCWords = 39;
 /* contact head: body a | body b << 8 | points << 16 | CF_* flags << 20 */
 struct QuadLayout {
     int hits, jkeys;                    /* X, contact generation (the shape records are at 0) */
     int last, pos, level, order;        /* X, contact levels */
-    int jlast, jlev, jgeo;              /* X, joints */
+    int jlast, jlev, jgeo, jconst;      /* X, joints */
     int heads;
     int y;                              /* region Y: the bodies' rows */
     int bounds, masks, keys, clip, cw;  /* Y, contact generation; cw workers collide */
+    int waves;                          /* of the workgroup */
     int words;                          /* in all, per world */
     size_t scratch_tile_words;          /* HBM, per tile: the per-lane words, then the contact records */
 };
@@ -99,9 +102,11 @@ enum { QR_N, QR_T1, QR_CA, QR_CB, QR_IA, QR_IB = QR_IA + 3, QR_ROLL = QR_IB + 3,
        QR_SEP, QR_RV, QR_RA, QR_RB = QR_RA + 4 };
 static_assert(QR_RB + 4 == kQRecQuads, "contact record quads");
 
-/* The layout of a capacity set; false when it does not fit. */
-B3D_FN bool quad_layout(const Geometry& g, int max_joints, QuadLayout* q) {
-    if (g.max_s > 64 || g.max_b > 255 || g.max_c > 1023 || g.max_j > max_joints) return false;
+/* The layout of a capacity set for workgroups of `waves` waves with
+ * lds_bytes of LDS; false when it does not fit. */
+B3D_FN bool quad_layout(const Geometry& g, int waves, size_t lds_bytes, QuadLayout* q) {
+    if (g.max_s > 64 || g.max_b > 255 || g.max_c > 1023 || g.max_j > 16) return false;
+    q->waves = waves;
     int hw = hit_words(g);
     q->hits = 4 * kShapeRows * g.max_s;
     q->jkeys = q->hits + hw + 1;
@@ -113,18 +118,19 @@ B3D_FN bool quad_layout(const Geometry& g, int max_joints, QuadLayout* q) {
     q->jlast = q->order + g.max_c;
     q->jlev = q->jlast + g.max_b;
     q->jgeo = q->jlev + g.max_j;
-    int xb = q->jgeo + kJGWords * g.max_j;
+    q->jconst = q->jgeo + kJGWords * g.max_j;
+    int xb = q->jconst + kJCWords * g.max_j;
     q->heads = xa > xb ? xa : xb;
     q->y = q->heads + g.max_c;
     q->bounds = q->y;
     q->masks = q->bounds + 6 * g.max_s;
     q->keys = q->masks + 2 * g.max_s;
     q->clip = q->keys + g.max_c;
-    int most = kQuadLdsWords - kQuadWgWords / kQuadCols, room = most - q->clip;
+    int most = (int)(lds_bytes / 4 - kQuadWgWords) / kQuadCols, room = most - q->clip;
     int rows = q->y + quad_body_rows(g);
     int cand = g.max_s * (g.max_s - 1) / 2;
     q->cw = room / kClipWords;
-    if (q->cw > kQuadWorkers) q->cw = kQuadWorkers;
+    if (q->cw > 4 * waves) q->cw = 4 * waves;
     if (q->cw > cand) q->cw = cand < 1 ? 1 : cand;
     if (q->cw < 4 && q->cw < cand) return false;
     int gen = q->clip + q->cw * kClipWords;
@@ -141,6 +147,7 @@ struct QLane {
     uint32_t* recs;    /* the world's contact records */
     PairStage st;      /* the tile's manifold stage */
     int sub, wave, worker;
+    int waves, workers;   /* compile-time constants once inlined */
     QuadLayout q;
 };
 B3Q_FN float* lrow(const QLane& Q, int word) { return Q.lds + word * kRow; }
@@ -154,7 +161,7 @@ B3Q_FN void lseti(const QLane& Q, int word, int v) { Q.lds[word * kRow] = __buil
  * to a worker. */
 B3Q_FN void quad_open(const QLane& Q, int old_n, int ns, int nj) {
     const Lane& L = Q.L;
-    for (int k = Q.worker; k < old_n; k += kQuadWorkers) {
+    for (int k = Q.worker; k < old_n; k += Q.workers) {
         int sa = ldi(L.w, cw(L, k, C_SHAPE_A)), sb = ldi(L.w, cw(L, k, C_SHAPE_B));
         int pk = k > 0 ? k - 1 : 0;
         int pa = ldi(L.w, cw(L, pk, C_SHAPE_A)), pb = ldi(L.w, cw(L, pk, C_SHAPE_B));
@@ -166,9 +173,9 @@ B3Q_FN void quad_open(const QLane& Q, int old_n, int ns, int nj) {
         if (k > 0 && !(shape_key(pa, pb) < key && (uint32_t)sa < 65536u && (uint32_t)sb < 65536u))
             lseti(Q, Q.q.hits + hit_words(L.g), 1);
     }
-    old_warm_copy(L, old_n, Q.worker, kQuadWorkers);
-    shape_pass(L, ns, lrow(Q, Q.q.bounds), Q.worker, kQuadWorkers);
-    for (int j = Q.worker; j < nj; j += kQuadWorkers) {
+    old_warm_copy(L, old_n, Q.worker, Q.workers);
+    shape_pass(L, ns, lrow(Q, Q.q.bounds), Q.worker, Q.workers);
+    for (int j = Q.worker; j < nj; j += Q.workers) {
         uint32_t key = 0xffffffffu;
         if (!ldi(L.w, jw(L, j, J_COLLIDE_CONNECTED)))
             key = pair_key(ldi(L.w, jw(L, j, J_BODY_A)), ldi(L.w, jw(L, j, J_BODY_B)));
@@ -182,7 +189,7 @@ B3Q_FN uint64_t quad_mask(const QLane& Q, int i) {
 /* Bound-overlap masks, a row of pairs (i, j > i) to a worker. */
 B3Q_FN void quad_overlaps(const QLane& Q, int ns) {
     const float* bounds = lrow(Q, Q.q.bounds);
-    for (int i = Q.worker; i < ns; i += kQuadWorkers) {
+    for (int i = Q.worker; i < ns; i += Q.workers) {
         Box6 bi = box_load(bounds + i * 6 * kRow);
         uint64_t m = 0;
         for (int j0 = i + 1; j0 < ns; j0 += 4) {
@@ -200,49 +207,56 @@ B3Q_FN void quad_overlaps(const QLane& Q, int ns) {
 }
 
 /* This worker's share of the narrowphase: candidates worker, worker + cw,
- * ... in (i, j) order, their manifolds to the stage (pair_share). */
+ * ... in (i, j) order, their manifolds to the stage (pair_share).  The pair
+ * is looked up first and collided outside that loop: the workers' pairs are
+ * in different rows of the masks, and a collision inside the walk would run
+ * once per row. */
 B3Q_FN void quad_collide(const QLane& Q, int ns, int nj, int old_n) {
     const Lane& L = Q.L;
     if (Q.worker >= Q.q.cw) return;
     bool sorted = lgeti(Q, Q.q.hits + hit_words(L.g)) == 0;
-    int t = Q.worker, acc = 0;
+    int acc = 0, i = 0;
+    uint64_t m = ns > 0 ? quad_mask(Q, 0) : 0;
     float* clip = lrow(Q, Q.q.clip + Q.worker * kClipWords);
-    for (int i = 0; i < ns; i++) {
-        uint64_t m = quad_mask(Q, i);
+    for (int t = Q.worker;; t += Q.q.cw) {
         int c = __builtin_popcountll(m);
-        for (; t < acc + c; t += Q.q.cw) {
-            uint64_t mm = m;
-            for (int k = t - acc; k > 0; k--) mm &= mm - 1;
-            int j = __builtin_ctzll(mm);
-            PairShape A, B;
-            pshape_load(L, i, &A);
-            pshape_load(L, j, &B);
-            uint32_t bkey = pair_key(A.body, B.body);
-            int joined = 0;
-            for (int k = 0; k < nj; k++) joined |= (uint32_t)lgeti(Q, Q.q.jkeys + k) == bkey;
-            Mani mf;
-            mf.count = 0;
-            if (!(A.body == B.body || (A.bflags & B.bflags & kBodyStatic) || (A.cat & B.mask) == 0
-                    || (B.cat & A.mask) == 0 || joined))
-                collide_pair(&mf, A.P, B.P, clip);
-            if (mf.count > 0) {
-                /* the old contact of the same pair (the merge of the sorted lists) */
-                uint32_t key = shape_key(i, j);
-                int match = -1;
-                if (sorted) {
-                    int lo = 0, hi = old_n;
-                    while (lo < hi) {
-                        int mid = (lo + hi) >> 1;
-                        if ((uint32_t)lgeti(Q, Q.q.keys + mid) < key) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    if (lo < old_n && (uint32_t)lgeti(Q, Q.q.keys + lo) == key) match = lo;
-                }
-                mani_store(Q.st, L.lane, t, mf, key, match);
-                lds_or(lrow(Q, Q.q.hits + (t >> 5)), 1u << (t & 31));
-            }
+        while (i < ns && t >= acc + c) {
+            acc += c;
+            i++;
+            m = i < ns ? quad_mask(Q, i) : 0;
+            c = __builtin_popcountll(m);
         }
-        acc += c;
+        if (i >= ns) break;
+        uint64_t mm = m;
+        for (int k = t - acc; k > 0; k--) mm &= mm - 1;
+        int j = __builtin_ctzll(mm);
+        PairShape A, B;
+        pshape_load(L, i, &A);
+        pshape_load(L, j, &B);
+        uint32_t bkey = pair_key(A.body, B.body);
+        int joined = 0;
+        for (int k = 0; k < nj; k++) joined |= (uint32_t)lgeti(Q, Q.q.jkeys + k) == bkey;
+        Mani mf;
+        mf.count = 0;
+        if (!(A.body == B.body || (A.bflags & B.bflags & kBodyStatic) || (A.cat & B.mask) == 0
+                || (B.cat & A.mask) == 0 || joined))
+            collide_pair(&mf, A.P, B.P, clip);
+        if (mf.count > 0) {
+            /* the old contact of the same pair (the merge of the sorted lists) */
+            uint32_t key = shape_key(i, j);
+            int match = -1;
+            if (sorted) {
+                int lo = 0, hi = old_n;
+                while (lo < hi) {
+                    int mid = (lo + hi) >> 1;
+                    if ((uint32_t)lgeti(Q, Q.q.keys + mid) < key) lo = mid + 1;
+                    else hi = mid;
+                }
+                if (lo < old_n && (uint32_t)lgeti(Q, Q.q.keys + lo) == key) match = lo;
+            }
+            mani_store(Q.st, L.lane, t, mf, key, match);
+            lds_or(lrow(Q, Q.q.hits + (t >> 5)), 1u << (t & 31));
+        }
     }
 }
 
@@ -336,7 +350,7 @@ B3Q_FN int quad_append(const QLane& Q, int old_n, Soft cs, Soft ss, int* wg) {
     int cc = total < L.g.max_c ? total : L.g.max_c;
     bool sorted = lgeti(Q, Q.q.hits + hw) == 0;
     int acc = 0, word = 0, flags = 0;
-    for (int k = Q.worker; k < cc; k += kQuadWorkers) {
+    for (int k = Q.worker; k < cc; k += Q.workers) {
         uint32_t bits = (uint32_t)lgeti(Q, Q.q.hits + word);
         while (acc + __builtin_popcount(bits) <= k) {
             acc += __builtin_popcount(bits);
@@ -420,47 +434,100 @@ B3Q_FN void quad_joint_levels(const QLane& Q, int nj, int nb, int* wg) {
     atomicMax(wg + WG_JOINTS, nj);
 }
 
-/* The joints' delta-pose geometry to their LDS rows, joints first, first +
- * stride, ... */
-B3Q_FN void quad_joint_geometry(const QLane& Q, int nj, int first, int stride) {
-    const Lane& L = Q.L;
+B3Q_FN M3 rm3(const uint32_t* r, int k) { M3 m; m.cx = r3(r, k); m.cy = r3(r, k + 3); m.cz = r3(r, k + 6); return m; }
+/* A joint's constants (JC_*), as prepare_joints left them in the world and
+ * the joint record. */
+struct JConst { uint32_t ab; int info; b3d::Q qa, qb; V3 pa, pb, dc; float ma, mb; M3 ia, ib; };
+B3Q_FN JConst jconst_world(const Lane& L, int j) {
     const uint32_t* w = L.w;
-    for (int j = first; j < nj; j += stride) {
-        uint32_t ab = ldu(joint_rec(L, j), JS_AB);
-        int info = ldi(joint_rec(L, j), JS_INFO);
-        b3d::Q fqa = ldq(w, jw(L, j, J_FRAME_Q_A)), fqb = ldq(w, jw(L, j, J_FRAME_Q_B));
-        V3 fpa = ld3(w, jw(L, j, J_FRAME_P_A)), fpb = ld3(w, jw(L, j, J_FRAME_P_B));
-        V3 dcen = ld3(w, jw(L, j, J_DELTA_CENTER));
-        float ma = ldf(w, jw(L, j, J_INV_MASS_A)), mb = ldf(w, jw(L, j, J_INV_MASS_B));
-        M3 ia = ldm3(w, jw(L, j, J_INV_I_A)), ib = ldm3(w, jw(L, j, J_INV_I_B));
-        const uint32_t* da = delta_rec(L, (int)(ab & 0xffffu));
-        const uint32_t* db = delta_rec(L, (int)(ab >> 16));
-        JGeo o = joint_geo(info, rq4(da, BD_DQ), rq4(db, BD_DQ), r3(da, BD_DP), r3(db, BD_DP), fqa, fqb, fpa, fpb, dcen,
-            ma, mb, ia, ib);
+    return JConst{ldu(joint_rec(L, j), JS_AB), ldi(joint_rec(L, j), JS_INFO), ldq(w, jw(L, j, J_FRAME_Q_A)),
+        ldq(w, jw(L, j, J_FRAME_Q_B)), ld3(w, jw(L, j, J_FRAME_P_A)), ld3(w, jw(L, j, J_FRAME_P_B)),
+        ld3(w, jw(L, j, J_DELTA_CENTER)), ldf(w, jw(L, j, J_INV_MASS_A)), ldf(w, jw(L, j, J_INV_MASS_B)),
+        ldm3(w, jw(L, j, J_INV_I_A)), ldm3(w, jw(L, j, J_INV_I_B))};
+}
+B3Q_FN void jconst_store(uint32_t* c, const JConst& k) {
+    rsu(c, JC_AB, k.ab);
+    rsu(c, JC_INFO, (uint32_t)k.info);
+    rsq(c, JC_QA, k.qa);
+    rsq(c, JC_QB, k.qb);
+    rs3(c, JC_PA, k.pa);
+    rs3(c, JC_PB, k.pb);
+    rs3(c, JC_DC, k.dc);
+    rsf(c, JC_MA, k.ma);
+    rsf(c, JC_MB, k.mb);
+    rs3(c, JC_IA, k.ia.cx);
+    rs3(c, JC_IA + 3, k.ia.cy);
+    rs3(c, JC_IA + 6, k.ia.cz);
+    rs3(c, JC_IB, k.ib.cx);
+    rs3(c, JC_IB + 3, k.ib.cy);
+    rs3(c, JC_IB + 6, k.ib.cz);
+}
+B3Q_FN JConst jconst_load(const uint32_t* c) {
+    return JConst{ru(c, JC_AB), (int)ru(c, JC_INFO), rq4(c, JC_QA), rq4(c, JC_QB), r3(c, JC_PA), r3(c, JC_PB),
+        r3(c, JC_DC), rf(c, JC_MA), rf(c, JC_MB), rm3(c, JC_IA), rm3(c, JC_IB)};
+}
+
+/* The joints' delta-pose geometry (joint_geo) to their LDS rows.  The
+ * waves take one of three parts each, so that no lane runs all of it: waves
+ * 0, 3, .. the anchors, separation and twist (a weld: the angular error),
+ * 1, 4, .. the point rows' inverse matrix, 2, 5, .. the hinge rows and their
+ * matrix.  Waves `first` and up take part.  The first call of a step reads
+ * the constants from memory and leaves them in LDS for the others (from
+ * memory each time, eight hinges' geometry took 2.6 us a substep). */
+template <bool First>
+B3Q_FN void quad_joint_geometry(const QLane& Q, int nj, int first) {
+    const Lane& L = Q.L;
+    int wv = Q.wave - first, n = Q.waves - first;
+    if (wv < 0) return;
+    int parts = n < 3 ? n : 3, part = wv % parts;
+    int stride = 4 * ((n - part + parts - 1) / parts);
+    for (int j = (wv / parts) * 4 + Q.sub; j < nj; j += stride) {
+        uint32_t* crow = (uint32_t*)lrow(Q, Q.q.jconst + j * kJCWords);
+        JConst c = First ? jconst_world(L, j) : jconst_load(crow);
+        if (First && part == 0) jconst_store(crow, c);
+        const int info = c.info;
+        const b3d::Q fqa = c.qa, fqb = c.qb;
+        const V3 fpa = c.pa, fpb = c.pb, dcen = c.dc;
+        const float ma = c.ma, mb = c.mb;
+        const M3 ia = c.ia, ib = c.ib;
+        const uint32_t* da = delta_rec(L, (int)(c.ab & 0xffffu));
+        const uint32_t* db = delta_rec(L, (int)(c.ab >> 16));
+        b3d::Q dqa = rq4(da, BD_DQ), dqb = rq4(db, BD_DQ);
+        V3 dpa = r3(da, BD_DP), dpb = r3(db, BD_DP);
         float* g = lrow(Q, Q.q.jgeo + j * kJGWords);
-        auto put = [g](int k, float v) { g[k * kRow] = v; };
-        auto put3 = [put](int k, V3 v) { put(k, v.x); put(k + 1, v.y); put(k + 2, v.z); };
-        put3(JG_RA, o.ra);
-        put3(JG_RB, o.rb);
-        put3(JG_PSEP, o.psep);
-        put3(JG_PKI, o.pki.cx);
-        put3(JG_PKI + 3, o.pki.cy);
-        put3(JG_PKI + 6, o.pki.cz);
-        bool fixed = (info & JF_FIXED) != 0;
-        if (info & JF_WELD) {
-            if (!fixed) put3(JG_CV, o.cv);
-            continue;
+        auto put = [g](int quad, int k, float v) { g[(4 * quad + k) * kRow] = v; };
+        auto put3 = [put](int quad, V3 v) { put(quad, 0, v.x); put(quad, 1, v.y); put(quad, 2, v.z); };
+        /* the unused results of each part's call fall away */
+        bool fixed = (info & JF_FIXED) != 0, weld = (info & JF_WELD) != 0;
+        if (part == 0 || parts < 2) {
+            JGeo o = joint_geo(info, dqa, dqb, dpa, dpb, fqa, fqb, fpa, fpb, dcen, ma, mb, ia, ib);
+            put3(JG_RA_TW, o.ra);
+            put3(JG_RB_RELX, o.rb);
+            put3(JG_PSEP_RELY, o.psep);
+            if (weld) {
+                if (!fixed) put3(JG_PY_KXY, o.cv);
+            } else {
+                put(JG_RA_TW, 3, o.tw);
+                put(JG_RB_RELX, 3, o.relx);
+                put(JG_PSEP_RELY, 3, o.rely);
+            }
         }
-        put(JG_TW, o.tw);
-        put(JG_RELX, o.relx);
-        put(JG_RELY, o.rely);
-        if (fixed) continue;
-        put3(JG_PX, o.px);
-        put3(JG_PY, o.py);
-        put(JG_KXX, o.kxx);
-        put(JG_KXY, o.kxy);
-        put(JG_KYY, o.kyy);
-        put(JG_KINV, o.kinv);
+        if (part == 1 || parts < 2) {
+            M3 pki = inv3(point_k(ma, mb, ia, ib, rot(dqa, fpa), rot(dqb, fpb)));
+            put3(JG_K0_KYY, pki.cx);
+            put3(JG_K1_KINV, pki.cy);
+            put3(JG_K2, pki.cz);
+        }
+        if ((part == 2 || parts < 3) && part == parts - 1 && !weld && !fixed) {
+            JGeo o = joint_geo(info & ~(JF_SPRING | JF_MOTOR | JF_LIMIT), dqa, dqb, dpa, dpb, fqa, fqb, fpa, fpb, dcen,
+                ma, mb, ia, ib);
+            put3(JG_PX_KXX, o.px);
+            put3(JG_PY_KXY, o.py);
+            put(JG_PX_KXX, 3, o.kxx);
+            put(JG_PY_KXY, 3, o.kxy);
+            put(JG_K0_KYY, 3, o.kyy);
+            put(JG_K1_KINV, 3, o.kinv);
+        }
     }
 }
 
@@ -760,54 +827,46 @@ B3Q_FN void cq_writeback(const QLane& Q, const CQ& r) {
 
 /* ---- joint rows on quads ---- */
 
-/* A joint's row in a quad's registers.  Scalars are the same in all four
- * lanes.  A weld's fields share the hinge's: axis the accumulated angular
- * impulse, ia_ax, ib_ax, px the angular mass columns, py the angular error;
- * axial, maxt the linear and angular hertz, (target, ss.x, ss.y) the linear
- * and (ss.z, speed, lower) the angular spring. */
+/* A joint's row in a quad's registers: vectors with a scalar of the row in
+ * lane 3 (behind the slash), and two quads of scalars.
+ *   ia, ib   inverse inertia columns / ma, lower, upper and mb, softness
+ *            bias and mass scale
+ *   axis, ia_ax, ib_ax, px, py, ra, rb, psep, pki  as JRow's / (geometry)
+ *            twist, relx, rely with ra, rb, psep; kxx, kxy with px, py; kyy,
+ *            kinv with pki
+ *   s1       spring softness, then the softness' impulse scale
+ *   s2       axial mass, torque limit, target, speed
+ * A weld: axis its accumulated angular impulse, ia_ax, ib_ax, px its angular
+ * mass columns / angular spring, py the angular error, s1 the linear spring,
+ * s2 the linear and angular hertz. */
 struct JQ {
     int j, lev, info;      /* joint (-1: none), its two levels (quad_joint_levels), JF_* | kQDyn* */
     int va, vb;
-    float ma, mb;
-    QM ia, ib;
-    Soft soft;
-    float lin_imp, ra, rb, psep;
-    QM pki;
-    float axis, ia_ax, ib_ax, px, py;
-    float axial, maxt, target, speed, lower, upper;
-    QM ss;                 /* the spring's softness */
+    QM ia, ib, pki;
+    float lin_imp, ra, rb, psep, axis, ia_ax, ib_ax, px, py, s1, s2;
     float spring_imp, motor_imp, lower_imp, upper_imp, perp_x, perp_y;
-    float kxx, kxy, kyy, kinv, tw, relx, rely;
 };
 /* The row's delta-pose geometry (quad_joint_geometry). */
 B3Q_FN void jq_geometry(const QLane& Q, JQ* r) {
-    const float* g = lrow(Q, Q.q.jgeo + r->j * kJGWords);
-    const float* v = g + Q.sub * kRow;
-    r->ra = v[JG_RA * kRow];
-    r->rb = v[JG_RB * kRow];
-    r->psep = v[JG_PSEP * kRow];
-    r->pki = QM{v[JG_PKI * kRow], v[(JG_PKI + 3) * kRow], v[(JG_PKI + 6) * kRow]};
-    if (r->info & JF_WELD) {
-        r->py = v[JG_CV * kRow];
-        return;
-    }
-    r->px = v[JG_PX * kRow];
-    r->py = v[JG_PY * kRow];
-    r->kxx = g[JG_KXX * kRow];
-    r->kxy = g[JG_KXY * kRow];
-    r->kyy = g[JG_KYY * kRow];
-    r->kinv = g[JG_KINV * kRow];
-    r->tw = g[JG_TW * kRow];
-    r->relx = g[JG_RELX * kRow];
-    r->rely = g[JG_RELY * kRow];
+    const float* g = lrow(Q, Q.q.jgeo + r->j * kJGWords + Q.sub);
+    auto v = [g](int quad) { return g[4 * quad * kRow]; };
+    r->ra = v(JG_RA_TW);
+    r->rb = v(JG_RB_RELX);
+    r->psep = v(JG_PSEP_RELY);
+    r->pki = QM{v(JG_K0_KYY), v(JG_K1_KINV), v(JG_K2)};
+    r->py = v(JG_PY_KXY);
+    if (!(r->info & JF_WELD)) r->px = v(JG_PX_KXX);
 }
 B3Q_FN void jq_load(const QLane& Q, int j, JQ* r) {
     const Lane& L = Q.L;
     const uint32_t* w = L.w;
     const uint32_t* rec = joint_rec(L, j);
-    int k = Q.sub < 3 ? Q.sub : 2;     /* lane 3 reads what lane 2 does */
-    auto v = [w, k, &L, j](int f) { return ldf(w, jw(L, j, f + k)); };
+    int k = Q.sub;
+    bool l3 = k == 3;
+    /* the vector at word f, word g in lane 3 */
+    auto v = [w, k, l3, &L, j](int f, int g) { return ldf(w, jw(L, j, l3 ? g : f + k)); };
     auto s = [w, &L, j](int f) { return ldf(w, jw(L, j, f)); };
+    auto pick = [k](int a, int b, int c, int d) { return k == 0 ? a : (k == 1 ? b : (k == 2 ? c : d)); };
     uint32_t ab = ldu(rec, JS_AB);
     int a = (int)(ab & 0xffffu), b = (int)(ab >> 16);
     r->j = j;
@@ -815,38 +874,29 @@ B3Q_FN void jq_load(const QLane& Q, int j, JQ* r) {
     r->info = ldi(rec, JS_INFO) | (is_dyn_flag(L, a) ? kQDynA : 0) | (is_dyn_flag(L, b) ? kQDynB : 0);
     r->va = qvel_row(a);
     r->vb = qvel_row(b);
-    r->ma = s(J_INV_MASS_A);
-    r->mb = s(J_INV_MASS_B);
-    r->ia = QM{v(J_INV_I_A), v(J_INV_I_A + 3), v(J_INV_I_A + 6)};
-    r->ib = QM{v(J_INV_I_B), v(J_INV_I_B + 3), v(J_INV_I_B + 6)};
-    r->soft = ldsoft(w, jw(L, j, J_SOFTNESS));
-    r->lin_imp = v(J_LINEAR_IMPULSE);
-    r->kxx = r->kxy = r->kyy = r->kinv = r->tw = r->relx = r->rely = 0.0f;
-    r->spring_imp = r->motor_imp = r->lower_imp = r->upper_imp = r->perp_x = r->perp_y = r->upper = 0.0f;
+    r->lin_imp = v(J_LINEAR_IMPULSE, J_LINEAR_IMPULSE);
+    r->ia.x = v(J_INV_I_A, J_INV_MASS_A);
+    r->ib.x = v(J_INV_I_B, J_INV_MASS_B);
+    r->ia.y = v(J_INV_I_A + 3, J_LOWER_ANGLE);
+    r->ia.z = v(J_INV_I_A + 6, J_UPPER_ANGLE);
+    r->ib.y = v(J_INV_I_B + 3, J_SOFTNESS);
+    r->ib.z = v(J_INV_I_B + 6, J_SOFTNESS + 1);
     if (r->info & JF_WELD) {
-        r->axis = v(J_ANGULAR_IMPULSE);
-        r->ia_ax = v(J_ANGULAR_MASS);
-        r->ib_ax = v(J_ANGULAR_MASS + 3);
-        r->px = v(J_ANGULAR_MASS + 6);
-        r->axial = s(J_LINEAR_HERTZ);
-        r->maxt = s(J_ANGULAR_HERTZ);
-        r->target = s(J_LINEAR_SPRING);
-        r->ss.x = s(J_LINEAR_SPRING + 1);
-        r->ss.y = s(J_LINEAR_SPRING + 2);
-        r->ss.z = s(J_ANGULAR_SPRING);
-        r->speed = s(J_ANGULAR_SPRING + 1);
-        r->lower = s(J_ANGULAR_SPRING + 2);
+        r->axis = v(J_ANGULAR_IMPULSE, J_ANGULAR_IMPULSE);
+        r->ia_ax = v(J_ANGULAR_MASS, J_ANGULAR_SPRING);
+        r->ib_ax = v(J_ANGULAR_MASS + 3, J_ANGULAR_SPRING + 1);
+        r->px = v(J_ANGULAR_MASS + 6, J_ANGULAR_SPRING + 2);
+        r->s1 = s(pick(J_LINEAR_SPRING, J_LINEAR_SPRING + 1, J_LINEAR_SPRING + 2, J_LINEAR_SPRING));
+        r->s2 = s(k == 0 ? J_LINEAR_HERTZ : J_ANGULAR_HERTZ);
+        r->spring_imp = r->motor_imp = r->lower_imp = r->upper_imp = r->perp_x = r->perp_y = 0.0f;
     } else {
-        r->axis = v(J_ROTATION_AXIS);
-        r->ia_ax = ldf(rec, JS_IAX + k);
-        r->ib_ax = ldf(rec, JS_IBX + k);
-        r->axial = s(J_AXIAL_MASS);
-        r->maxt = s(J_MAX_MOTOR_TORQUE);
-        r->target = s(J_TARGET_ANGLE);
-        r->ss = QM{s(J_SPRING_SOFTNESS), s(J_SPRING_SOFTNESS + 1), s(J_SPRING_SOFTNESS + 2)};
-        r->speed = s(J_MOTOR_SPEED);
-        r->lower = s(J_LOWER_ANGLE);
-        r->upper = s(J_UPPER_ANGLE);
+        int k3 = l3 ? 2 : k;
+        r->axis = v(J_ROTATION_AXIS, J_ROTATION_AXIS);
+        r->ia_ax = ldf(rec, JS_IAX + k3);
+        r->ib_ax = ldf(rec, JS_IBX + k3);
+        r->px = 0.0f;
+        r->s1 = s(pick(J_SPRING_SOFTNESS, J_SPRING_SOFTNESS + 1, J_SPRING_SOFTNESS + 2, J_SOFTNESS + 2));
+        r->s2 = s(pick(J_AXIAL_MASS, J_MAX_MOTOR_TORQUE, J_TARGET_ANGLE, J_MOTOR_SPEED));
         r->spring_imp = s(J_SPRING_IMPULSE);
         r->motor_imp = s(J_MOTOR_IMPULSE);
         r->lower_imp = s(J_LOWER_IMPULSE);
@@ -855,6 +905,29 @@ B3Q_FN void jq_load(const QLane& Q, int j, JQ* r) {
         r->perp_y = s(J_PERP_IMPULSE + 1);
     }
     jq_geometry(Q, r);
+}
+
+/* The row's scalars in all four lanes.  A wave with one joint keeps them
+ * across the sweeps; with more it takes them out for each solve. */
+struct JScal { Soft soft; float ma, mb, tw, relx, rely, kxx, kxy, kyy, kinv, axial, maxt, target, speed, lower, upper; QM ss; };
+B3Q_FN void jq_scalars(const JQ& r, JScal* o) {
+    o->soft = Soft{qbc<3>(r.ib.y), qbc<3>(r.ib.z), qbc<3>(r.s1)};
+    o->ma = qbc<3>(r.ia.x);
+    o->mb = qbc<3>(r.ib.x);
+    o->lower = qbc<3>(r.ia.y);
+    o->upper = qbc<3>(r.ia.z);
+    o->tw = qbc<3>(r.ra);
+    o->relx = qbc<3>(r.rb);
+    o->rely = qbc<3>(r.psep);
+    o->kxx = qbc<3>(r.px);
+    o->kxy = qbc<3>(r.py);
+    o->kyy = qbc<3>(r.pki.x);
+    o->kinv = qbc<3>(r.pki.y);
+    o->axial = qbc<0>(r.s2);
+    o->maxt = qbc<1>(r.s2);
+    o->target = qbc<2>(r.s2);
+    o->speed = qbc<3>(r.s2);
+    o->ss = QM{qbc<0>(r.s1), qbc<1>(r.s1), qbc<2>(r.s1)};
 }
 
 /* The joint's warm start (b3_warm_start_joints, 06:204-239), at the start of
@@ -873,9 +946,9 @@ B3Q_FN void jq_warm(const QLane& Q, const JQ& r) {
         ang = ang + axial * r.axis;
     }
     QVel x = qvel_load(Q, r.va, r.vb);
-    x.va = x.va - r.ma * r.lin_imp;
+    x.va = x.va - qbc<3>(r.ia.x) * r.lin_imp;
     x.wa = x.wa - qmv(r.ia, qcross(r.ra, r.lin_imp) + ang);
-    x.vb = x.vb + r.mb * r.lin_imp;
+    x.vb = x.vb + qbc<3>(r.ib.x) * r.lin_imp;
     x.wb = x.wb + qmv(r.ib, qcross(r.rb, r.lin_imp) + ang);
     qvel_store(Q, r.va, r.vb, r.info, x);
 }
@@ -883,18 +956,18 @@ B3Q_FN void jq_warm(const QLane& Q, const JQ& r) {
 /* One joint's solve: b3_solve_revolute (06:436-642) or b3_solve_weld
  * (06:285-332), as solve_revolute and solve_weld. */
 template <bool Bias>
-B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
+B3Q_FN void jq_solve(const QLane& Q, JQ& r, const JScal& k, float h, float inv_h) {
     QVel x = qvel_load(Q, r.va, r.vb);
     const bool fixed = (r.info & JF_FIXED) != 0;
-    Soft psoft = r.soft;
+    Soft soft = k.soft;
     bool pbias = Bias;
     if (r.info & JF_WELD) {
         if (!fixed) {
             float bias = 0.0f, mscale = 1.0f, iscale = 0.0f;
-            if (Bias || r.maxt > 0.0f) {
-                bias = r.py * r.ss.z;
-                mscale = r.speed;
-                iscale = r.lower;
+            if (Bias || k.maxt > 0.0f) {
+                bias = r.py * qbc<3>(r.ia_ax);
+                mscale = qbc<3>(r.ib_ax);
+                iscale = qbc<3>(r.px);
             }
             float cdot = x.wb - x.wa;
             float impulse = qmv(QM{r.ia_ax, r.ib_ax, r.px}, cdot + bias) * -mscale - iscale * r.axis;
@@ -902,19 +975,18 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
             x.wa = x.wa - qmv(r.ia, impulse);
             x.wb = x.wb + qmv(r.ib, impulse);
         }
-        pbias = Bias || r.axial > 0.0f;
-        psoft.bias_rate = r.target;
-        psoft.mass_scale = r.ss.x;
-        psoft.impulse_scale = r.ss.y;
+        pbias = Bias || k.axial > 0.0f;
+        soft = Soft{k.ss.x, k.ss.y, k.ss.z};
     } else if (!fixed) {
+        const float tw = k.tw, axial = k.axial, maxt = k.maxt, speed = k.speed, lower = k.lower, upper = k.upper;
         if (r.info & JF_SPRING) {
-            float bias = r.ss.x * (r.tw - r.target);
+            float bias = k.ss.x * (tw - k.target);
             float cdot = qdot3(x.wb - x.wa, r.axis);
             float old = r.spring_imp;
-            float dimp = -r.ss.y * r.axial * (cdot + bias) - r.ss.z * old;
+            float dimp = -k.ss.y * axial * (cdot + bias) - k.ss.z * old;
             float nimp = old + dimp;
-            if (r.maxt > 0.0f) {
-                float maxp = r.maxt * h;
+            if (maxt > 0.0f) {
+                float maxp = maxt * h;
                 nimp = clampf(nimp, -maxp, maxp);
             }
             dimp = nimp - old;
@@ -925,17 +997,17 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
         if (r.info & JF_MOTOR) {
             bool blocked = false;
             if (r.info & JF_LIMIT) {
-                if (r.tw >= r.upper - 0.01f && r.speed > 0.0f) blocked = true;
-                if (r.tw <= r.lower + 0.01f && r.speed < 0.0f) blocked = true;
+                if (tw >= upper - 0.01f && speed > 0.0f) blocked = true;
+                if (tw <= lower + 0.01f && speed < 0.0f) blocked = true;
             }
             if (blocked) {
                 r.motor_imp = 0.0f;
             } else {
                 float old = r.motor_imp;
-                float cdot = qdot3(x.wb - x.wa, r.axis) - r.speed;
-                float dimp = -r.axial * cdot;
+                float cdot = qdot3(x.wb - x.wa, r.axis) - speed;
+                float dimp = -axial * cdot;
                 float nimp = old + dimp;
-                float maxp = r.maxt * h;
+                float maxp = maxt * h;
                 nimp = clampf(nimp, -maxp, maxp);
                 dimp = nimp - old;
                 r.motor_imp = nimp;
@@ -945,13 +1017,13 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
         }
         if (r.info & JF_LIMIT) {
             float old = r.lower_imp;
-            float lo = limit_impulse(r.tw - r.lower, qdot3(x.wb - x.wa, r.axis), inv_h, Bias, r.soft, r.axial, old);
+            float lo = limit_impulse(tw - lower, qdot3(x.wb - x.wa, r.axis), inv_h, Bias, soft, axial, old);
             r.lower_imp = lo;
             float dimp = lo - old;
             x.wa = x.wa - dimp * r.ia_ax;
             x.wb = x.wb + dimp * r.ib_ax;
             old = r.upper_imp;
-            float up = limit_impulse(r.upper - r.tw, qdot3(x.wa - x.wb, r.axis), inv_h, Bias, r.soft, r.axial, old);
+            float up = limit_impulse(upper - tw, qdot3(x.wa - x.wb, r.axis), inv_h, Bias, soft, axial, old);
             r.upper_imp = up;
             dimp = up - old;
             x.wa = x.wa + dimp * r.ia_ax;
@@ -962,10 +1034,10 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
         bias.y = 0.0f;
         float mscale = 1.0f, iscale = 0.0f;
         if (Bias) {
-            bias.x = r.soft.bias_rate * r.relx;
-            bias.y = r.soft.bias_rate * r.rely;
-            mscale = r.soft.mass_scale;
-            iscale = r.soft.impulse_scale;
+            bias.x = soft.bias_rate * k.relx;
+            bias.y = soft.bias_rate * k.rely;
+            mscale = soft.mass_scale;
+            iscale = soft.impulse_scale;
         }
         float wrel = x.wb - x.wa;
         V2 rhs;
@@ -974,9 +1046,9 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
         V2 sol;
         sol.x = 0.0f;
         sol.y = 0.0f;
-        if (r.kinv == r.kinv) {
-            sol.x = r.kinv * (r.kyy * rhs.x - r.kxy * rhs.y);
-            sol.y = r.kinv * (-r.kxy * rhs.x + r.kxx * rhs.y);
+        if (k.kinv == k.kinv) {
+            sol.x = k.kinv * (k.kyy * rhs.x - k.kxy * rhs.y);
+            sol.y = k.kinv * (-k.kxy * rhs.x + k.kxx * rhs.y);
         }
         V2 dimp;
         dimp.x = -mscale * sol.x - iscale * r.perp_x;
@@ -991,13 +1063,13 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, float h, float inv_h) {
     float cdot = (x.vb + qcross(x.wb, r.rb)) - (x.va + qcross(x.wa, r.ra));
     float bias = 0.0f, mscale = 1.0f, iscale = 0.0f;
     if (pbias) {
-        bias = r.psep * psoft.bias_rate;
-        mscale = psoft.mass_scale;
-        iscale = psoft.impulse_scale;
+        bias = r.psep * soft.bias_rate;
+        mscale = soft.mass_scale;
+        iscale = soft.impulse_scale;
     }
     float impulse = qmv(r.pki, cdot + bias) * -mscale - iscale * r.lin_imp;
     r.lin_imp = r.lin_imp + impulse;
-    qimpulse(&x, r.ma, r.ia, r.mb, r.ib, r.ra, r.rb, impulse);
+    qimpulse(&x, k.ma, r.ia, k.mb, r.ib, r.ra, r.rb, impulse);
     qvel_store(Q, r.va, r.vb, r.info, x);
 }
 
@@ -1043,7 +1115,7 @@ B3Q_FN void quad_level(const QLane& Q, CQ (&row)[CR], int cc, int lev, int* at, 
         r.sep = cq_separations(Q, r, cq_base(Q, r));
         solve(r);
         cq_store(Q, r);
-        *at += kQuadWaves;
+        *at += Q.waves;
     }
 }
 
@@ -1080,14 +1152,14 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
     int cc = 0;
     if (act) {
         cc = quad_append(Q, old_n, cs, ss, wg);
-        body_prepass(L, h, Q.worker, kQuadWorkers);
-        prepare_joints(L, h, Q.worker, kQuadWorkers);
+        body_prepass(L, h, Q.worker, Q.workers);
+        prepare_joints(L, h, Q.worker, Q.workers);
     }
     B3D_BARRIER();
     if (act) {
         if (Q.worker == 0) quad_levels(Q, cc, nb, wg);
         if (Q.worker == 4) quad_joint_levels(Q, nj, nb, wg);
-        if (Q.worker >= 8) quad_joint_geometry(Q, nj, Q.worker - 8, kQuadWorkers - 8);
+        quad_joint_geometry<true>(Q, nj, 2);   /* the waves that build no levels */
     }
     B3D_BARRIER();
     const int nlev = __builtin_amdgcn_readfirstlane(wg[WG_LEVELS]);
@@ -1098,7 +1170,7 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
     float base[CR];
 #pragma unroll
     for (int i = 0; i < CR; i++) {
-        int at = i * kQuadWaves + Q.wave;
+        int at = i * Q.waves + Q.wave;
         row[i].c = -1;
         row[i].lev = 0;
         if (at < cc) {
@@ -1109,12 +1181,12 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
     JQ joint[JR];
 #pragma unroll
     for (int i = 0; i < JR; i++) {
-        int j = i * kQuadWaves + Q.wave;
+        int j = i * Q.waves + Q.wave;
         joint[i].j = -1;
         joint[i].lev = 0;
         if (j < nj) jq_load(Q, j, &joint[i]);
     }
-    const int past = CR * kQuadWaves + Q.wave;   /* the wave's first contact not in registers */
+    const int past = CR * Q.waves + Q.wave;   /* the wave's first contact not in registers */
     auto levels = [&](auto solve) {
         int at = past;
         for (int lev = 1; lev <= nlev; lev++) {
@@ -1122,11 +1194,16 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
             B3D_BARRIER();
         }
     };
+    JScal scal;
+    if (JR == 1 && joint[0].j >= 0) jq_scalars(joint[0], &scal);
     auto joint_levels = [&](auto solve) {
         for (int lev = 1; lev <= njlev; lev++) {
 #pragma unroll
             for (int i = 0; i < JR; i++)
-                if ((joint[i].lev & 255) == lev || (joint[i].lev >> 8) == lev) solve(joint[i]);
+                if ((joint[i].lev & 255) == lev || (joint[i].lev >> 8) == lev) {
+                    if (JR > 1) jq_scalars(joint[i], &scal);
+                    solve(joint[i], scal);
+                }
             B3D_BARRIER();
         }
     };
@@ -1144,28 +1221,29 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
         B3D_BARRIER();
     }
     for (int s = 0; s < subs; s++) {
-        if (act) integrate_velocities(L, Q.worker, kQuadWorkers);
+        if (act) integrate_velocities(L, Q.worker, Q.workers);
         B3D_BARRIER();
         levels([&](CQ& r) { cq_solve<false>(Q, r, inv_h, contact_speed, cs, ss); });
-        joint_levels([&](JQ& r) { jq_solve<true>(Q, r, h, inv_h); });
-        if (act) integrate_positions(L, h, inv_dt, Q.worker, kQuadWorkers);
+        joint_levels([&](JQ& r, const JScal& k) { jq_solve<true>(Q, r, k, h, inv_h); });
+        if (act) integrate_positions(L, h, inv_dt, Q.worker, Q.workers);
         B3D_BARRIER();
         if (njmax > 0) {
-            quad_joint_geometry(Q, nj, Q.worker, kQuadWorkers);
+            quad_joint_geometry<false>(Q, nj, 0);
             B3D_BARRIER();
 #pragma unroll
             for (int i = 0; i < JR; i++)
                 if (joint[i].j >= 0) jq_geometry(Q, &joint[i]);
+            if (JR == 1 && joint[0].j >= 0) jq_scalars(joint[0], &scal);
         }
         separations();
         levels([&](CQ& r) { cq_solve<true>(Q, r, inv_h, contact_speed, cs, ss); });
-        joint_levels([&](JQ& r) { jq_solve<false>(Q, r, h, inv_h); });
+        joint_levels([&](JQ& r, const JScal& k) { jq_solve<false>(Q, r, k, h, inv_h); });
         if (rest) levels([&](CQ& r) { cq_restitution(Q, r, rest_threshold); });
     }
 #pragma unroll
     for (int i = 0; i < CR; i++)
         if (row[i].lev > 0) cq_writeback(Q, row[i]);
-    for (int at = past; at < cc; at += kQuadWaves) {
+    for (int at = past; at < cc; at += Q.waves) {
         CQ r;
         cq_load(Q, lgeti(Q, Q.q.order + at), &r);
         cq_writeback(Q, r);
@@ -1174,8 +1252,8 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
     for (int i = 0; i < JR; i++)
         if (joint[i].j >= 0) jq_writeback(Q, joint[i]);
     if (act) {
-        finalize(L, Q.worker, kQuadWorkers);
-        vel_store(L, Q.worker, kQuadWorkers);
+        finalize(L, Q.worker, Q.workers);
+        vel_store(L, Q.worker, Q.workers);
     }
 }
 
