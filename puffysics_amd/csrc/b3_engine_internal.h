@@ -64,6 +64,19 @@ bool b3i_quad_fit(const b3d::Geometry& g, int waves, size_t* scratch_tile_words)
 hipError_t b3i_quad_init();
 hipError_t b3i_step_quad(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
     const unsigned char* reset_mask, hipStream_t stream);
+/* The launch with gravity, its status in *err; false (nothing launched) when
+ * the engine's worlds do not step so. */
+bool b3i_step_quad_gravity(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
+    const unsigned char* reset_mask, B3GravityLaw law, const float* masses, hipStream_t stream, hipError_t* err);
+
+/* The step on quads of the caller's own worlds (b3_quad_worlds.hip): scratch
+ * words per 64 worlds, 0 when it does not take worlds of geometry g; its
+ * set-up on the current device; its launch on `count` worlds, world w at
+ * aos + w * stride + offset (words). */
+size_t b3i_quad_worlds_tile_words(const b3d::Geometry& g);
+hipError_t b3i_quad_worlds_init();
+hipError_t b3i_step_quad_worlds(uint32_t* aos, size_t stride, size_t offset, uint32_t* scratch,
+    const b3d::Geometry& g, int count, float dt, int substeps, const unsigned char* active, hipStream_t stream);
 
 /* The engine's device is the current one. */
 inline hipError_t on_device(const B3Engine* e) {

@@ -8,7 +8,8 @@
  * lane's substep loop, before each velocity update, on the lane's own world.
  *
  *   b3k_step_gravity   Plummer-softened pairwise gravity between each
- *                      world's bodies (nbody_rigid.cuh:15-66)
+ *                      world's bodies (nbody_rigid.cuh:15-66); batches that
+ *                      step on quads of lanes run it there (b3_quad.hip)
  */
 #include <hip/hip_runtime.h>
 
@@ -59,6 +60,9 @@ hipError_t b3_batch_step_gravity_gpu(B3Engine* e, float dt, int substeps, const 
     hipError_t err = on_device(e);
     if (err != hipSuccess) return err;
     if (dt == 0.0f) return reset_mask ? b3_batch_restore_gpu(e, reset_mask, stream) : hipSuccess;
+    if (!(e->options & B3_ENGINE_ONE_WAVE_PER_TILE)
+            && b3i_step_quad_gravity(e, dt, substeps, step_mask, reset_mask, law, masses, stream, &err))
+        return err;
     b3k_step_gravity<<<e->tiles, 64, e->lds_bytes, stream>>>(e->live, e->snap, e->scratch, e->g, e->count, dt,
         substeps, step_mask, reset_mask, e->options, law, masses);
     return hipGetLastError();

@@ -47,6 +47,7 @@ namespace b3d {
 
 constexpr int kLanes = B3D_LANES;
 constexpr int kRow = B3D_ROW;   /* stride of the LDS rows */
+constexpr int kWord = B3D_WORD; /* stride of a world's words and its per-lane scratch words */
 /* Velocity row of a body: linear, angular, flags.  With four lanes to a
  * world (B3D_QUAD) lane 0..2 of a quad reads a component and lane 3 a pad
  * word, so both vectors take four words and the flags live elsewhere. */
@@ -497,12 +498,12 @@ B3D_FN void restore_ranges(const Geometry& g, int snap_contacts, int lo[3], int 
     hi[2] = g.jo + g.max_j * kJointWords;
 }
 
-/* ---- word access (stride kLanes) ---- */
-B3D_FN float ldf(const uint32_t* p, int k) { return __builtin_bit_cast(float, p[k * kLanes]); }
-B3D_FN int ldi(const uint32_t* p, int k) { return (int)p[k * kLanes]; }
-B3D_FN uint32_t ldu(const uint32_t* p, int k) { return p[k * kLanes]; }
-B3D_FN void stf(uint32_t* p, int k, float v) { p[k * kLanes] = __builtin_bit_cast(uint32_t, v); }
-B3D_FN void sti(uint32_t* p, int k, int v) { p[k * kLanes] = (uint32_t)v; }
+/* ---- word access (stride kWord) ---- */
+B3D_FN float ldf(const uint32_t* p, int k) { return __builtin_bit_cast(float, p[k * kWord]); }
+B3D_FN int ldi(const uint32_t* p, int k) { return (int)p[k * kWord]; }
+B3D_FN uint32_t ldu(const uint32_t* p, int k) { return p[k * kWord]; }
+B3D_FN void stf(uint32_t* p, int k, float v) { p[k * kWord] = __builtin_bit_cast(uint32_t, v); }
+B3D_FN void sti(uint32_t* p, int k, int v) { p[k * kWord] = (uint32_t)v; }
 B3D_FN V3 ld3(const uint32_t* p, int k) { return v3(ldf(p, k), ldf(p, k + 1), ldf(p, k + 2)); }
 B3D_FN void st3(uint32_t* p, int k, V3 v) { stf(p, k, v.x); stf(p, k + 1, v.y); stf(p, k + 2, v.z); }
 B3D_FN Q ldq(const uint32_t* p, int k) { return q4(ldf(p, k), ldf(p, k + 1), ldf(p, k + 2), ldf(p, k + 3)); }
@@ -653,8 +654,8 @@ B3D_FN uint32_t* shape_rec(const Lane& L, int s) {
     if (B3D_QUAD) return L.sq + s * 4 * kShapeRows * kRow;
     return L.sq + (size_t)(L.g.q_shape + s * kShapeRows) * kRowWords + L.sslot;
 }
-B3D_FN uint32_t* old_rec(const Lane& L, int k) { return L.scr + (L.g.scr_old + k * kOldWords) * kLanes; }
-B3D_FN uint32_t* chead_rec(const Lane& L, int c) { return L.scr + (L.g.scr_sep + c * kContactScr) * kLanes; }
+B3D_FN uint32_t* old_rec(const Lane& L, int k) { return L.scr + (L.g.scr_old + k * kOldWords) * kWord; }
+B3D_FN uint32_t* chead_rec(const Lane& L, int c) { return L.scr + (L.g.scr_sep + c * kContactScr) * kWord; }
 /* Packed record of contact c and of its point p (see kCRows). */
 B3D_FN uint32_t* crec(const Lane& L, int c, int slot) {
     return L.sq + (size_t)(L.g.q_ct + c * kCRows) * kRowWords + slot * 4;
@@ -738,7 +739,7 @@ B3D_FN void rec_store_masses(uint32_t* r, int flags, float ma, M3 ia, float mb, 
         qsf(r, R_IB_ZYZ + 1, ib.cz.z);
     }
 }
-B3D_FN uint32_t* joint_rec(const Lane& L, int j) { return L.scr + (L.g.scr_joint + j * kJointScr) * kLanes; }
+B3D_FN uint32_t* joint_rec(const Lane& L, int j) { return L.scr + (L.g.scr_joint + j * kJointScr) * kWord; }
 /* Per-lane rows of LDS words (stride kLanes): a joint's LDS row (JL) or
  * impulse row (JI), word k at q[k * kLanes]. */
 B3D_FN float jlf(const float* q, int k) { return q[k * kLanes]; }

@@ -45,6 +45,12 @@
 #ifndef B3D_ROW
 #define B3D_ROW B3D_LANES
 #endif
+/* Stride between consecutive words of one world, and of its per-lane
+ * scratch: a tile's 64 lanes, or 1 where plain B3World structs are stepped
+ * in place. */
+#ifndef B3D_WORD
+#define B3D_WORD B3D_LANES
+#endif
 
 namespace b3d {
 

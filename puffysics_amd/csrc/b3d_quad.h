@@ -92,6 +92,7 @@ struct QuadLayout {
     int heads;
     int y;                              /* region Y: the bodies' rows */
     int bounds, masks, keys, clip, cw;  /* Y, contact generation; cw workers collide */
+    int law;                            /* rows of a force law, past everything else */
     int waves;                          /* of the workgroup */
     int words;                          /* in all, per world */
     size_t scratch_tile_words;          /* HBM, per tile: the per-lane words, then the contact records */
@@ -103,8 +104,9 @@ enum { QR_N, QR_T1, QR_CA, QR_CB, QR_IA, QR_IB = QR_IA + 3, QR_ROLL = QR_IB + 3,
 static_assert(QR_RB + 4 == kQRecQuads, "contact record quads");
 
 /* The layout of a capacity set for workgroups of `waves` waves with
- * lds_bytes of LDS; false when it does not fit. */
-B3D_FN bool quad_layout(const Geometry& g, int waves, size_t lds_bytes, QuadLayout* q) {
+ * lds_bytes of LDS, law_words of them per body for a force law; false when
+ * it does not fit. */
+B3D_FN bool quad_layout(const Geometry& g, int waves, size_t lds_bytes, int law_words, QuadLayout* q) {
     if (g.max_s > 64 || g.max_b > 255 || g.max_c > 1023 || g.max_j > 16) return false;
     q->waves = waves;
     int hw = hit_words(g);
@@ -126,7 +128,7 @@ B3D_FN bool quad_layout(const Geometry& g, int waves, size_t lds_bytes, QuadLayo
     q->masks = q->bounds + 6 * g.max_s;
     q->keys = q->masks + 2 * g.max_s;
     q->clip = q->keys + g.max_c;
-    int most = (int)(lds_bytes / 4 - kQuadWgWords) / kQuadCols, room = most - q->clip;
+    int most = (int)(lds_bytes / 4 - kQuadWgWords) / kQuadCols - law_words * g.max_b, room = most - q->clip;
     int rows = q->y + quad_body_rows(g);
     int cand = g.max_s * (g.max_s - 1) / 2;
     q->cw = room / kClipWords;
@@ -134,9 +136,10 @@ B3D_FN bool quad_layout(const Geometry& g, int waves, size_t lds_bytes, QuadLayo
     if (q->cw > cand) q->cw = cand < 1 ? 1 : cand;
     if (q->cw < 4 && q->cw < cand) return false;
     int gen = q->clip + q->cw * kClipWords;
-    q->words = gen > rows ? gen : rows;
+    q->law = gen > rows ? gen : rows;
+    q->words = q->law + law_words * g.max_b;
     q->scratch_tile_words = (size_t)g.scr_words * kLanes + (size_t)kLanes * g.max_c * kQRecWords;
-    return q->words <= most;
+    return q->law <= most;
 }
 
 /* One lane's view: its world (L, rows in LDS), its place in the quad and
@@ -1098,6 +1101,76 @@ B3Q_FN void jq_writeback(const QLane& Q, const JQ& r) {
     }
 }
 
+/* ---- force laws ---- */
+
+/* A law of the force hook (b3d_lane.h) on quads: per-body rows of kWords LDS
+ * words, staged once per step (stage), and each substep's velocity update of
+ * bodies first, first + stride, ... (update; every worker stages and updates
+ * the same bodies). */
+struct QuadNoLaw {
+    static constexpr int kWords = 0;
+};
+
+/* Plummer-softened gravity (GravityLaw, b3d_forces.h): body b's force is its
+ * own sum over the other bodies in index order, the pairs (k, b), k < b,
+ * subtracted and (b, j), j > b, added, which is the order in which the pair
+ * loop reaches it; each pair's force is thus computed by both bodies'
+ * workers, with the same operations.  Rows: center, mass, applied force,
+ * inverse mass, gravity scale. */
+struct QuadGravity {
+    static constexpr int kWords = 9;
+    float gravity, softening;
+    const float* masses;   /* the world's, or null */
+
+    static __device__ __attribute__((always_inline)) float* row(const QLane& Q, int b) {
+        return lrow(Q, Q.q.law + b * kWords);
+    }
+    __device__ __attribute__((always_inline)) void stage(const QLane& Q, int nb) const {
+        const Lane& L = Q.L;
+        for (int b = Q.worker; b < nb; b += Q.workers) {
+            V3 c = ld3(L.w, bw(L, b, B_CENTER)), f = ld3(L.w, bw(L, b, B_FORCE));
+            float im = ldf(L.w, bw(L, b, B_INV_MASS)), gs = ldf(L.w, bw(L, b, B_GRAVITY_SCALE));
+            int type = ldi(L.w, bw(L, b, B_TYPE));
+            float m = masses ? masses[b] : (type == kDynamic && im > 0.0f ? 1.0f / im : 0.0f);
+            float* r = row(Q, b);
+            const float v[kWords] = {c.x, c.y, c.z, m, f.x, f.y, f.z, im, im > 0.0f ? gs : 0.0f};
+#pragma unroll
+            for (int k = 0; k < kWords; k++) r[k * kRow] = v[k];
+        }
+    }
+    static __device__ __attribute__((always_inline)) V3 center(const QLane& Q, int b) {
+        const float* r = row(Q, b);
+        return add(v3(r[0], r[kRow], r[2 * kRow]), r3(delta_rec(Q.L, b), BD_DP));
+    }
+    __device__ __attribute__((always_inline)) void update(const QLane& Q, int nb, float h) const {
+        const Lane& L = Q.L;
+        float eps2 = softening * softening;
+        V3 g = ld3(L.w, H_GRAVITY);
+        for (int b = Q.worker; b < nb; b += Q.workers) {
+            if (!(ru(delta_rec(L, b), BD_KIND) & kKindDynamic)) continue;
+            const float* r = row(Q, b);
+            float mb = r[3 * kRow], im = r[7 * kRow], gs = r[8 * kRow];
+            V3 f = v3(r[4 * kRow], r[5 * kRow], r[6 * kRow]);
+            V3 cb = center(Q, b);
+            for (int k = 0; k < nb && mb != 0.0f; k++) {
+                float mk = row(Q, k)[3 * kRow];
+                if (k == b || mk == 0.0f) continue;
+                bool before = k < b;
+                V3 ck = center(Q, k);
+                V3 d = before ? sub(cb, ck) : sub(ck, cb);
+                float q = dot(d, d) + eps2;
+                float inv = 1.0f / sqrtf(q);
+                V3 p = scale(d, gravity * (before ? mk : mb) * (before ? mb : mk) * inv * inv * inv);
+                f = before ? sub(f, p) : add(f, p);
+            }
+            const uint32_t* s = body_rec(L, b);
+            V3 dv = add(scale(f, h * im), scale(g, h * gs));
+            set_vlin(L, b, madd(dv, rf(s, BS_LD), vlin(L, b)));
+            set_vang(L, b, madd(r3(s, BS_DW), rf(s, BS_AD), vang(L, b)));
+        }
+    }
+};
+
 /* ---- the step ---- */
 
 /* The wave's contacts of one level: those in registers whose level it is,
@@ -1124,8 +1197,8 @@ B3Q_FN void quad_level(const QLane& Q, CQ (&row)[CR], int cc, int lev, int* at, 
  * of worlds that do not step (L.active false) have no items.  `wg`: the
  * workgroup's words, zero at entry, as are the hit bits; a barrier has
  * passed since. */
-template <int CR, int JR>
-B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
+template <int CR, int JR, class Law>
+B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg, const Law& law) {
     Lane& L = Q.L;
     const bool act = L.active;
     int subs = substeps < 1 ? 1 : substeps;
@@ -1153,6 +1226,7 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
     if (act) {
         cc = quad_append(Q, old_n, cs, ss, wg);
         body_prepass(L, h, Q.worker, Q.workers);
+        if constexpr (Law::kWords > 0) law.stage(Q, nb);
         prepare_joints(L, h, Q.worker, Q.workers);
     }
     B3D_BARRIER();
@@ -1221,7 +1295,10 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
         B3D_BARRIER();
     }
     for (int s = 0; s < subs; s++) {
-        if (act) integrate_velocities(L, Q.worker, Q.workers);
+        if (act) {
+            if constexpr (Law::kWords > 0) law.update(Q, nb, h);
+            else integrate_velocities(L, Q.worker, Q.workers);
+        }
         B3D_BARRIER();
         levels([&](CQ& r) { cq_solve<false>(Q, r, inv_h, contact_speed, cs, ss); });
         joint_levels([&](JQ& r, const JScal& k) { jq_solve<true>(Q, r, k, h, inv_h); });
@@ -1255,6 +1332,34 @@ B3Q_FN void quad_step(QLane& Q, float dt, int substeps, int* wg) {
         finalize(L, Q.worker, Q.workers);
         vel_store(L, Q.worker, Q.workers);
     }
+}
+
+/* The view of one lane of a workgroup of `waves` waves: world `slot` of a
+ * tile, its words at w, the tile's scratch (scratch_tile_words) and stage. */
+B3Q_FN QLane quad_lane(uint32_t* w, uint32_t* tile_scratch, uint32_t* tile_stage, float* lds, const Geometry& g,
+        const QuadLayout& q, int slot, int waves, unsigned int opts) {
+    QLane Q;
+    Q.sub = (int)(threadIdx.x & 3u);
+    Q.wave = (int)(threadIdx.x >> 6);
+    Q.worker = Q.wave * 4 + Q.sub;
+    Q.waves = waves;
+    Q.workers = 4 * waves;
+    Q.q = q;
+    Q.lds = lds + kQuadWgWords + slot % kQuadCols;
+    Q.recs = tile_scratch + (size_t)g.scr_words * kLanes + (size_t)slot * g.max_c * kQRecWords;
+    Q.st = PairStage{};
+    Q.st.p = tile_stage + slot;
+    Q.L = lane_view(nullptr, nullptr, nullptr, g, 0, slot, opts);
+    Q.L.w = w;
+    Q.L.scr = tile_scratch + (size_t)slot * (kWord == kLanes ? 1 : g.scr_words);
+    Q.L.sq = reinterpret_cast<uint32_t*>(Q.lds);
+    Q.L.vel = Q.lds + q.y * kRow;
+    return Q;
+}
+/* Clears what quad_step expects cleared; a barrier follows. */
+B3Q_FN void quad_clear(const QLane& Q, int* wg) {
+    if (threadIdx.x < (unsigned)kQuadWgWords) wg[threadIdx.x] = 0;
+    for (int k = Q.worker; k <= hit_words(Q.L.g); k += Q.workers) lseti(Q, Q.q.hits + k, 0);
 }
 
 }  // namespace b3d

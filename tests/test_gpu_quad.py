@@ -119,3 +119,79 @@ def test_unsorted_old_contacts():
         eng.step(1.0 / 60.0, 3)
     assert (ref["contact_count"] > 1).any()
     _same(eng, ref, CUSTOM_SIG)
+
+
+def _step_worlds(worlds, sig, steps, dt, substeps, active=None, pad=0):
+    """`steps` calls of b3_batch_step_worlds_gpu on a device copy of the
+    worlds, `pad` bytes apart."""
+    from puffysics_amd import _native
+    from puffysics_amd.b3types import B3Batch
+    n, wb = len(worlds), worlds.dtype.itemsize
+    host = np.full((n, wb + pad), 0x5a, np.uint8)
+    host[:, :wb] = worlds.view(np.uint8).reshape(n, wb)
+    dev = torch.from_numpy(host).cuda()
+    act = None if active is None else torch.from_numpy(active).cuda()
+    for _ in range(steps):
+        rc = _native.engine_lib().b3_batch_step_worlds_gpu(
+            B3Batch(dev.data_ptr(), wb + pad, 0, n), sig, dt, substeps, None if act is None else act.data_ptr(),
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+    torch.cuda.synchronize()
+    out = dev.cpu().numpy()
+    assert (out[:, wb:] == 0x5a).all()
+    return np.ascontiguousarray(out[:, :wb]).view(worlds.dtype).reshape(n)
+
+
+# In place on quads: one world, a part of a workgroup, chunks of the array
+# (1,300 arm worlds are two); staged as tiles: more than 16 joints.
+@pytest.mark.parametrize("scene,count,steps,pad", [(1, 1, 30, 4), (5, 17, 20, 0), (5, 1300, 3, 12), (4, 300, 3, 0),
+                                                   (2, 1000, 3, 8)])
+def test_step_worlds_edges(scene, count, steps, pad):
+    sc = scenes.SCENES[scene]
+    worlds = scenes.build(scene, count)
+    oracle_run(scene, worlds, clone(worlds), 0, 25, threads=8)
+    ref = clone(worlds)
+    active = (np.arange(count) % 5 != 3).astype(np.uint8)
+    for _ in range(steps):
+        oracle_step_batch(ref, sc.sig, sc.dt, sc.substeps, active)
+    got = _step_worlds(worlds, sc.sig, steps, sc.dt, sc.substeps, active, pad)
+    diff = diff_words(got, ref, sc.sig)
+    from b3test import solver_field_words
+    allowed = solver_field_words(ref)              # not written back by this call
+    assert allowed[diff[:, 0], diff[:, 1]].all(), diff[:4].tolist()
+    idle = active == 0
+    raw = [x.view(np.uint32).reshape(count, -1)[idle] for x in (got, worlds)]   # with the structs' padding
+    assert (raw[0] == raw[1]).all()
+
+
+def test_step_worlds_staged():
+    sig = signature(27, 24, 32, 24)
+    worlds = _enlarge(scenes.build(3, 70), sig, 3)
+    ref = clone(worlds)
+    for _ in range(4):
+        oracle_step_batch(ref, sig, 1.0 / 120.0, 4)
+    got = _step_worlds(worlds, sig, 4, 1.0 / 120.0, 4)
+    assert len(diff_words(got, ref, sig)) == 0
+
+
+# Gravity: a worker sums one body's pairs, with the masses of the bodies and
+# with the caller's; four-wave workgroups past a quarter tile per CU; at one
+# lane a world past half a tile per CU.
+@pytest.mark.parametrize("scene,count,steps,caller", [(4, 20, 12, False), (2, 65, 12, True), (5, 33, 6, True),
+                                                      (2, 4100, 2, True), (2, 8200, 2, False)])
+def test_gravity(scene, count, steps, caller):
+    from b3test import oracle_step_gravity
+    sc = scenes.SCENES[scene]
+    worlds = scenes.build(scene, count)
+    masses = None
+    if caller:
+        masses = np.random.default_rng(2).uniform(0.0, 3.0, (count, sc.caps[0])).astype(np.float32)
+        masses[:, 2] = 0.0                         # a body that neither feels nor sources it
+        masses[::2, 0] = 5.0                       # the static ground as a source
+    ref = clone(worlds)
+    eng = _engine(worlds, sc.sig)
+    dev = None if masses is None else torch.from_numpy(masses).cuda()
+    for _ in range(steps):
+        oracle_step_gravity(ref, sc.sig, sc.dt, sc.substeps, 4.0, 0.15, masses)
+        eng.step_gravity(sc.dt, sc.substeps, 4.0, 0.15, dev)
+    _same(eng, ref, sc.sig)
