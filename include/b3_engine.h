@@ -190,15 +190,21 @@ hipError_t b3_batch_art_step_gpu(B3Engine* engine, float dt, int substeps, const
  * its scratch exceeds the array.  Enqueues on `stream`; calls no
  * allocating routine.
  *
+ * Worlds whose per-world state fits a workgroup's LDS (at most 64 shapes
+ * and 16 joints, and roughly 60 bodies or 400 contacts) are stepped where
+ * they are, and only their per-step scratch is in the array; others are
+ * staged there as tiles with their scratch beside them.
+ *
  * Limit: the array holds 64 MiB, reserved on each device the library runs
- * on until the process ends.  A tile of 64 worlds needs
- *   64 * (sizeof(B3World) + scratch per world) + 64
- * bytes of it; the per-step scratch per world is about the size of the
- * world (34.3 KB beside a 37.3 KB world of 17 bodies, 17 shapes, 64
- * contacts and 4 joints).  A call runs its batch in chunks of as many
- * tiles as the array holds (14 tiles, 896 worlds, of the first kind), one
- * launch of each kernel per chunk, in order on the stream; a large batch
- * therefore runs at a fraction of b3_batch_step_gpu's rate.
+ * on until the process ends.  64 worlds need
+ *   64 * (scratch per world)                          in place
+ *   64 * (sizeof(B3World) + scratch per world) + 64   staged
+ * bytes of it (the second must fit in any case); the per-step scratch per
+ * world is about 56 KB in place beside a 37.3 KB world of 17 bodies, 17
+ * shapes, 64 contacts and 4 joints.  A call runs its batch in chunks of as
+ * many 64 worlds as the array holds (18, 1,152 worlds, of that kind), one
+ * launch per chunk, in order on the stream; a large batch therefore runs at
+ * a fraction of b3_batch_step_gpu's rate.
  *
  * Calls share the array of their GPU.  Each call's stream waits for the
  * previous call's last kernel on that GPU (an event the library records

@@ -365,6 +365,7 @@ hipError_t noalloc_device(bool capturing, NoAllocDevice** out) {
         if ((err = hipGetSymbolAddress(&p, HIP_SYMBOL(b3_noalloc_scratch))) != hipSuccess) return err;
         if (!p) return hipErrorInvalidSymbol;
         if ((err = b3i_lds_limit((const void*)b3k_step<false>)) != hipSuccess) return err;
+        if ((err = b3i_quad_worlds_init()) != hipSuccess) return err;
         d.ptr = (uint32_t*)p;
     }
     if (!capturing && !d.last && (err = hipEventCreateWithFlags(&d.last, hipEventDisableTiming)) != hipSuccess)
@@ -728,10 +729,22 @@ hipError_t b3_batch_step_worlds_gpu(B3Batch worlds, unsigned long long config_si
      * call under capture cannot wait for work outside the graph: the caller
      * orders the graph's launches against other calls. */
     if (!capturing && (err = hipStreamWaitEvent(stream, nd->last, 0)) != hipSuccess) return err;
+    /* Worlds that fit step in place on quads, with only their scratch in
+     * the array; the others are staged as tiles (both sides: the comment at
+     * b3k_step_quad_worlds). */
+    size_t quad_words = b3i_quad_worlds_tile_words(g);
+    bool quad = quad_words != 0 && quad_words <= kNoAllocWords;
+    if (quad) chunk_tiles = kNoAllocWords / quad_words;
     int chunk = (int)(chunk_tiles * 64 < (size_t)worlds.count ? chunk_tiles * 64 : (size_t)worlds.count);
     uint32_t* aos = (uint32_t*)worlds.data;
     size_t stride = worlds.stride / 4, offset = worlds.world_offset / 4;
-    for (int first = 0; first < worlds.count; first += chunk) {
+    for (int first = 0; quad && first < worlds.count; first += chunk) {
+        int n = worlds.count - first < chunk ? worlds.count - first : chunk;
+        err = b3i_step_quad_worlds(aos + (size_t)first * stride, stride, offset, nd->ptr, g, n, dt, substeps,
+            active ? active + first : nullptr, stream);
+        if (err != hipSuccess) return err;
+    }
+    for (int first = 0; !quad && first < worlds.count; first += chunk) {
         int n = worlds.count - first < chunk ? worlds.count - first : chunk;
         int tiles = (n + 63) / 64;
         uint32_t* tile_words = nd->ptr;
