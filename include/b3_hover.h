@@ -4,15 +4,15 @@
  * The reference ships this task as a CUDA adapter whose single kernel runs
  * action, b3_step, reward / terminal, reset and observation per env
  * (examples/pufferlib/puffysics_hover/puffysics_hover.cu:21-79,
- * puffysics_hover.h:21-94, hover_task.h:45-99).  Here the physics runs in
- * the engine (b3_engine.h) and the task around it in three small kernels
- * on the same stream:
- *   action kernel      level = 0 / 1 / 2 from the action, force on the body
- *   b3_batch_step_gpu  every env
- *   reward kernel      tick, reward, terminal, episode return and log;
- *                      envs that are done draw their next start height
- *   b3_batch_restore_gpu of the done envs to the task's initial world
- *   observe kernel     the new start height of reset envs, observations
+ * puffysics_hover.h:21-94, hover_task.h:45-99).  So does this library, a
+ * 64-env tile to a wave of one launch, around the engine's own step code
+ * (b3_engine.h):
+ *   action     level = 0 / 1 / 2 from the action, force on the body
+ *   b3_step    every env
+ *   reward     tick, reward, terminal, episode return and log; envs that
+ *              are done draw their next start height
+ *   restore    of the done envs to the task's initial world
+ *   observe    the new start height of reset envs, observations
  * Results are the reference adapter's, bit for bit (tests/test_hover.py).
  *
  * The entry points mirror the adapter's puf_vec_create / puf_reset /

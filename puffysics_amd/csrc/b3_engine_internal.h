@@ -93,15 +93,13 @@ namespace b3d {
  * read 64 consecutive snapshot words and write them to their rows of the
  * tile.  A world's copy is cut into chunks of kRestoreChunk words; this
  * wave copies chunk k of every resetting world when k % nslices == slice,
- * so nslices waves share a tile's restores.  Only the worlds of the lanes
- * set in `lanes` are restored. */
+ * so nslices waves share a tile's restores.  restore_lanes: the worlds of
+ * the lanes set in `bits`; restore_tile: of those set in `lanes` whose reset
+ * byte is. */
 constexpr int kRestoreBatch = 8, kRestoreChunk = 64 * kRestoreBatch;
-__device__ inline void restore_tile(uint32_t* live, const uint32_t* snap, const Geometry& g, int count,
-        const unsigned char* reset, int tile, int slice, int nslices, uint64_t lanes = ~0ull) {
+__device__ inline void restore_lanes(uint32_t* live, const uint32_t* snap, const Geometry& g, int tile, int slice,
+        int nslices, uint64_t bits) {
     int lane = (int)(threadIdx.x & 63u);
-    int w = tile * 64 + lane;
-    int want = w < count && ((lanes >> lane) & 1u) && reset[w] != 0;
-    uint64_t bits = __ballot(want);
     uint32_t* lt = live + (size_t)tile * g.world_words * 64;
     while (bits) {
         int l = __builtin_ctzll(bits);
@@ -135,6 +133,14 @@ __device__ inline void restore_tile(uint32_t* live, const uint32_t* snap, const 
             }
         }
     }
+}
+
+__device__ inline void restore_tile(uint32_t* live, const uint32_t* snap, const Geometry& g, int count,
+        const unsigned char* reset, int tile, int slice, int nslices, uint64_t lanes = ~0ull) {
+    int lane = (int)(threadIdx.x & 63u);
+    int w = tile * 64 + lane;
+    int want = w < count && ((lanes >> lane) & 1u) && reset[w] != 0;
+    restore_lanes(live, snap, g, tile, slice, nslices, __ballot(want));
 }
 
 }  // namespace b3d
