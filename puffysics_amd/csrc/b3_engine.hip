@@ -564,7 +564,7 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
 hipError_t b3_engine_destroy(B3Engine* e) {
     if (!e) return hipSuccess;
     hipError_t first = hipSuccess;
-    void* bufs[6] = {e->live, e->snap, e->scratch, e->staging, e->art_ws, e->pair_stage};
+    void* bufs[7] = {e->live, e->snap, e->scratch, e->staging, e->art_ws, e->art_worlds, e->pair_stage};
     for (void* p : bufs) {
         if (!p) continue;
         hipError_t err = hipFree(p);

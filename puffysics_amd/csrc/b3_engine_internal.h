@@ -33,6 +33,8 @@ struct B3Engine {
     int quad_waves;          /* the step on quads of lanes (b3d_quad.h), a quarter tile to a workgroup of so
                                 many waves; 0: another step */
     bool joint_impulses_lds; /* the one-wave step keeps the joint impulses in LDS (b3d::ji_fit) */
+    uint32_t* art_worlds;    /* the worlds' words one after the other, for the articulated-contact step with
+                                one world to a wave (allocated with art_ws) */
 };
 
 /* Waves per tile when the narrowphase is shared (two per SIMD: the shared
@@ -55,6 +57,13 @@ hipError_t b3i_forces_init();
 /* The articulated-contact step (b3_art.hip): its workspace, then launches. */
 hipError_t b3i_art_init(B3Engine* e);
 hipError_t b3i_step_art(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
+    const unsigned char* reset_mask, hipStream_t stream);
+
+/* The same one world to a wave (b3_art_world.hip): whether worlds of
+ * geometry g fit in a CU's LDS; its set-up; its launch. */
+bool b3i_art_world_fit(const b3d::Geometry& g);
+hipError_t b3i_art_world_init();
+hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
     const unsigned char* reset_mask, hipStream_t stream);
 
 /* The step on quads (b3_quad.hip): whether it takes worlds of geometry g in

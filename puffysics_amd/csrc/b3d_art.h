@@ -70,6 +70,7 @@ struct ArtWs {
     float* p;   /* lane base; word k at p[k * kLanes] */
     int max_b;
     int n_links;
+    int n_tree; /* the first n_tree links are in trees; the others float alone */
     B3D_MFN int li(int link, int f) const { return link * kArtLinkWords + f; }
     B3D_MFN float gf(int link, int f) const { return p[li(link, f) * kLanes]; }
     B3D_MFN int gi(int link, int f) const { return __builtin_bit_cast(int, gf(link, f)); }
@@ -100,6 +101,28 @@ struct ArtWs {
 };
 constexpr int AT_DEG = 0, AT_ADJ_B = 1, AT_ADJ_J = 1 + kArtMaxDeg, AT_LINK = 1 + 2 * kArtMaxDeg, AT_SEEN = AT_LINK + 1,
               AT_QUEUE = AT_SEEN + 1, AT_PARENT_B = AT_QUEUE + 1, AT_PARENT_J = AT_PARENT_B + 1;
+
+/* B3D_ART_WAVE: the wave steps one world, every lane running the articulated
+ * passes with the same values; what is independent between links goes a link
+ * to a lane.  Otherwise a lane has its world to itself.  art_sync stands
+ * where a lane goes on to read workspace words that another lane wrote (one
+ * wave's LDS accesses complete in order, so only the compiler must keep
+ * them); loops that every lane runs in turn read their own writes. */
+#ifndef B3D_ART_WAVE
+#define B3D_ART_WAVE 0
+#endif
+#if B3D_ART_WAVE && defined(__HIP_DEVICE_COMPILE__)
+B3D_FN int art_lane() { return (int)(threadIdx.x & 63u); }
+B3D_FN int art_lanes() { return 64; }
+B3D_FN void art_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+#else
+B3D_FN int art_lane() { return 0; }
+B3D_FN int art_lanes() { return 1; }
+B3D_FN void art_sync() {}
+#endif
 
 B3D_FN S6 s6zero() { S6 s; s.w = zero3(); s.v = zero3(); return s; }
 B3D_FN M6 m6zero() { M6 m; m.ww = m3zero(); m.wv = m.ww; m.vw = m.ww; m.vv = m.ww; return m; }
@@ -229,11 +252,13 @@ B3D_FN void isolve_record(const ArtWs& A, int li, const M6& I) {
             return;
         }
         A.si(li, g + GJ_PIV + k, piv);
-        if (piv != k) {
+        /* the row swap as selects, so that M stays in registers */
+        for (int r = k + 1; r < 6; r++) {
+            bool s = piv == r;
             for (int c = k; c < 6; c++) {
-                float t = M[k][c];
-                M[k][c] = M[piv][c];
-                M[piv][c] = t;
+                float t = M[k][c], u = M[r][c];
+                M[k][c] = s ? u : t;
+                M[r][c] = s ? t : u;
             }
         }
         float inv = 1.0f / M[k][k];
@@ -256,11 +281,14 @@ B3D_FN bool isolve_replay(const ArtWs& A, int li, S6 rhs, S6* a) {
     }
     float b[6] = {rhs.w.x, rhs.w.y, rhs.w.z, rhs.v.x, rhs.v.y, rhs.v.z};
     for (int k = 0; k < 6; k++) {
+        /* the row swap as selects, so that b stays in registers */
         int piv = A.gi(li, g + GJ_PIV + k);
-        if (piv != k) {
-            float t = b[k];
-            b[k] = b[piv];
-            b[piv] = t;
+        float bk = b[k];
+        for (int r = k + 1; r < 6; r++) {
+            bool s = piv == r;
+            float t = b[r];
+            b[r] = s ? bk : t;
+            b[k] = s ? t : b[k];
         }
         b[k] *= A.gf(li, g + GJ_INV + k);
         for (int r = 0; r < 6; r++) {
@@ -284,6 +312,7 @@ B3D_FN bool art_build(const Lane& L, ArtWs& A) {
     int nb = body_count(L);
     int nj = clampi(ldi(w, H_JOINT_COUNT), 0, L.g.max_j);
     A.n_links = 0;
+    A.n_tree = 0;
     for (int i = 0; i < nb; i++) {
         A.tsi(i, AT_DEG, 0);
         A.tsi(i, AT_LINK, -1);
@@ -362,10 +391,12 @@ B3D_FN bool art_build(const Lane& L, ArtWs& A) {
             }
         }
     }
+    A.n_tree = A.n_links;
     for (int s = 0; s < nb; s++) {
         if (A.ti(s, AT_SEEN) || ldi(w, bw(L, s, B_TYPE)) != kDynamic) continue;
         if (A.n_links >= A.max_b) return false;
         int li = A.n_links++;
+        A.tsi(s, AT_LINK, li);
         A.si(li, AL_BODY, s);
         A.si(li, AL_FIXED, 0);
         A.si(li, AL_FLOATING, 1);
@@ -389,7 +420,7 @@ B3D_FN bool art_build(const Lane& L, ArtWs& A) {
  * delta poses are the step's, in the delta records. */
 B3D_FN void art_refresh(const Lane& L, const ArtWs& A) {
     const uint32_t* w = L.w;
-    for (int i = 0; i < A.n_links; i++) {
+    for (int i = art_lane(); i < A.n_links; i += art_lanes()) {
         int b = A.gi(i, AL_BODY);
         const uint32_t* d = delta_rec(L, b);
         Q rq = qnorm(qmul(rq4(d, BD_DQ), ldq(w, bw(L, b, B_ROTATION))));
@@ -406,8 +437,12 @@ B3D_FN void art_refresh(const Lane& L, const ArtWs& A) {
         A.s3(i, AL_SW, zero3());
         A.s3(i, AL_SV, zero3());
         A.s3(i, AL_R, zero3());
+    }
+    art_sync();
+    for (int i = art_lane(); i < A.n_tree; i += art_lanes()) {
         int p = A.gi(i, AL_PARENT);
         if (p < 0) continue;
+        V3 com = A.g3(i, AL_COM);
         V3 anchor = xf(A.g3(p, AL_POS), A.gq(p, AL_ROT), A.g3(i, AL_ANCHOR_A));
         V3 axis_local = rot(A.gq(i, AL_ROT_A), v3(0.0f, 0.0f, 1.0f));
         V3 u = norm(rot(A.gq(p, AL_ROT), axis_local));
@@ -452,13 +487,11 @@ B3D_FN S6 art_wrench(V3 r, V3 n, float x, int torque) {                 /* :675-
  * are the ones each call of the reference recomputes. */
 B3D_FN void art_pose_pass(const Lane& L, const ArtWs& A) {
     art_refresh(L, A);
-    for (int i = 0; i < A.n_links; i++) A.sI(i, AL_IA, art_inertia(A, i));
-    for (int i = A.n_links - 1; i >= 0; i--) {
+    for (int i = art_lane(); i < A.n_links; i += art_lanes()) A.sI(i, AL_IA, art_inertia(A, i));
+    art_sync();
+    for (int i = A.n_tree - 1; i >= 0; i--) {
         int p = A.gi(i, AL_PARENT);
-        if (p < 0) {
-            if (!A.gi(i, AL_FIXED) && A.gi(i, AL_FLOATING)) isolve_record(A, i, A.gI(i, AL_IA));
-            continue;
-        }
+        if (p < 0) continue;
         S6 S;
         S.w = A.g3(i, AL_SW);
         S.v = A.g3(i, AL_SV);
@@ -473,6 +506,9 @@ B3D_FN void art_pose_pass(const Lane& L, const ArtWs& A) {
         if (!A.gi(p, AL_FIXED))
             A.sI(p, AL_IA, iadd(A.gI(p, AL_IA), ishift(irank1(IA, U, Dinv), A.g3(i, AL_R))));
     }
+    for (int i = art_lane(); i < A.n_links; i += art_lanes())
+        if (A.gi(i, AL_PARENT) < 0 && !A.gi(i, AL_FIXED) && A.gi(i, AL_FLOATING)) isolve_record(A, i, A.gI(i, AL_IA));
+    art_sync();
 }
 
 /* y = J M^-1 J^T x for n rows: the impulse half of b3_art_delassus_apply
@@ -482,12 +518,13 @@ B3D_FN void art_pose_pass(const Lane& L, const ArtWs& A) {
  * the links' AL_A words. */
 B3D_FN void art_delassus(const Lane& L, const ArtWs& A, const ArtRow* rows, const float* x, float* y, int n) {
     (void)L;
-    for (int i = 0; i < A.n_links; i++) {
+    for (int i = art_lane(); i < A.n_links; i += art_lanes()) {
         S6 pa;
         pa.w = sub(zero3(), zero3());
         pa.v = pa.w;
         A.s6(i, AL_PA, pa);
     }
+    art_sync();
     for (int e = 0; e < n; e++) {
         const ArtRow& row = rows[e];
         if (row.link_a >= 0 && !A.gi(row.link_a, AL_FIXED)) {
@@ -506,7 +543,7 @@ B3D_FN void art_delassus(const Lane& L, const ArtWs& A, const ArtRow* rows, cons
         }
     }
     /* backward sweep, bias forces only (zero joint torques) */
-    for (int i = A.n_links - 1; i >= 0; i--) {
+    for (int i = A.n_tree - 1; i >= 0; i--) {
         int p = A.gi(i, AL_PARENT);
         if (p < 0) continue;
         S6 S;
@@ -527,20 +564,22 @@ B3D_FN void art_delassus(const Lane& L, const ArtWs& A, const ArtRow* rows, cons
             A.s6(p, AL_PA, pp);
         }
     }
-    /* forward sweep */
-    for (int i = 0; i < A.n_links; i++) {
-        int p = A.gi(i, AL_PARENT);
-        if (p < 0) {
-            S6 a = s6zero();
-            if (!A.gi(i, AL_FIXED) && A.gi(i, AL_FLOATING)) {
-                S6 pA = A.g6(i, AL_PA), rhs;
-                rhs.w = neg(pA.w);
-                rhs.v = neg(pA.v);
-                if (!isolve_replay(A, i, rhs, &a)) a = s6zero();
-            }
-            A.s6(i, AL_A, a);
-            continue;
+    /* forward sweep: the roots, then the trees' other links */
+    for (int i = art_lane(); i < A.n_links; i += art_lanes()) {
+        if (A.gi(i, AL_PARENT) >= 0) continue;
+        S6 a = s6zero();
+        if (!A.gi(i, AL_FIXED) && A.gi(i, AL_FLOATING)) {
+            S6 pA = A.g6(i, AL_PA), rhs;
+            rhs.w = neg(pA.w);
+            rhs.v = neg(pA.v);
+            if (!isolve_replay(A, i, rhs, &a)) a = s6zero();
         }
+        A.s6(i, AL_A, a);
+    }
+    art_sync();
+    for (int i = 0; i < A.n_tree; i++) {
+        int p = A.gi(i, AL_PARENT);
+        if (p < 0) continue;
         S6 ap = A.g6(p, AL_A), rhs;
         V3 r = A.g3(i, AL_R);
         rhs.w = ap.w;
@@ -585,11 +624,7 @@ B3D_FN void art_delassus(const Lane& L, const ArtWs& A, const ArtRow* rows, cons
     }
 }
 
-B3D_FN int art_link_of(const ArtWs& A, int body) {                      /* :751-758 */
-    for (int i = 0; i < A.n_links; i++)
-        if (A.gi(i, AL_BODY) == body) return i;
-    return -1;
-}
+B3D_FN int art_link_of(const ArtWs& A, int body) { return A.ti(body, AT_LINK); }   /* :751-758 */
 B3D_FN bool art_make_row(const ArtWs& A, int a, int b, V3 ra, V3 rb, V3 n, ArtRow* row) {   /* :769-779 */
     row->link_a = a >= 0 ? art_link_of(A, a) : -1;
     row->link_b = b >= 0 ? art_link_of(A, b) : -1;
@@ -609,13 +644,14 @@ B3D_FN float art_response(const Lane& L, const ArtWs& A, const ArtRow& row) {   
 B3D_FN void art_apply(const Lane& L, const ArtWs& A, const ArtRow& row, float lambda) {
     float x = -lambda, y = 0.0f;
     art_delassus(L, A, &row, &x, &y, 1);
-    for (int i = 0; i < A.n_links; i++) {
+    for (int i = art_lane(); i < A.n_links; i += art_lanes()) {
         if (A.gi(i, AL_FIXED)) continue;
         int b = A.gi(i, AL_BODY);
         S6 a = A.g6(i, AL_A);
         set_vlin(L, b, add(vlin(L, b), a.v));
         set_vang(L, b, add(vang(L, b), a.w));
     }
+    art_sync();
 }
 
 /* ---- the contact rows in the world (the reference's layout) ---- */
