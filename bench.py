@@ -181,9 +181,9 @@ def kernel_name(scene, count):
         return "b3k_step_quad<8, 2, %d>" % (1 if caps[3] <= 8 else 2)
     if 2 * tiles <= cus and caps[1] <= 32:
         return "b3k_step_quad<4, %s>" % ("3, 1" if caps[3] <= 4 else "2, 2" if caps[3] <= 8 else "1, 4")
-    if tiles > cus:
-        return "b3k_step<%s, false>" % ("true" if joint_impulses_fit(*caps) else "false")
     masks = 12 <= caps[1] <= 64
+    if tiles > (2 * cus if masks else cus):
+        return "b3k_step<%s, false>" % ("true" if joint_impulses_fit(*caps) else "false")
     return "b3k_step_shared<%s, %s>" % ("true" if masks else "false", "true" if joint_rows_fit(*caps) else "false")
 
 

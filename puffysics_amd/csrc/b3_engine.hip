@@ -506,7 +506,15 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
             if (4 * e->tiles <= cus && b3i_quad_fit(g, 8, &quad_scratch)) e->quad_waves = 8;
             else if (4 * e->tiles <= 2 * cus && b3i_quad_fit(g, 4, &quad_scratch)) e->quad_waves = 4;
         }
-        if (e->quad_waves || (e->tiles <= cus && shared_lds <= kCuLdsBytes && g.max_s > 2)) {
+        /* Shared tiles take a CU each; past one per CU they go in two turns.
+         * Worlds of many shapes (shared_masks) still gain over one wave per
+         * tile, whose narrowphase is serial, up to two tiles per CU, us one
+         * wave -> two turns: the arm at 16,448 worlds 993 -> 720, 32,768
+         * 1,058 -> 796, the bin 3,200 -> 1,750 and 3,535 -> 2,205.  The
+         * chains (830 -> 817, 880 -> 856) hardly do and the stacks lose
+         * (480 -> 512 at 32,768): they keep one wave. */
+        int shared_tiles = shared_masks(g) ? 2 * cus : cus;
+        if (e->quad_waves || (e->tiles <= shared_tiles && shared_lds <= kCuLdsBytes && g.max_s > 2)) {
             size_t max_cand = (size_t)g.max_s * (size_t)(g.max_s - 1) / 2;
             size_t stage_words = max_cand * kStageWords;
             if ((size_t)stage_sched_words(g) > stage_words) stage_words = (size_t)stage_sched_words(g);
