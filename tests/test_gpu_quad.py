@@ -121,6 +121,28 @@ def test_unsorted_old_contacts():
     _same(eng, ref, CUSTOM_SIG)
 
 
+# 0: the step on quads; 4: one wave per tile.
+@pytest.mark.parametrize("options", [0, 4])
+def test_joint_of_a_body_with_itself(options):
+    """Welds and hinges whose two ends are one body (the creation API takes
+    them): the warm start moves the body by end a and then, from there, by
+    end b."""
+    from puffysics_amd.creation import CUSTOM_SIG
+    worlds = feature_worlds(20)
+    for k in range(20):
+        for j in range(k % 2, int(worlds["joint_count"][k]), 2):
+            worlds["joints"]["body_a"][k, j] = worlds["joints"]["body_b"][k, j]
+    ref = clone(worlds)
+    eng = _engine(worlds, CUSTOM_SIG)
+    eng.set_options(1 | options)
+    for _ in range(6):
+        oracle_step_batch(ref, CUSTOM_SIG, 1.0 / 60.0, 4)
+        eng.step(1.0 / 60.0, 4)
+    own = ref["joints"]["body_a"] == ref["joints"]["body_b"]
+    assert (np.abs(ref["joints"]["linear_impulse"]["x"]) > 0)[own].any() and np.isfinite(ref["bodies"]["lin_vel"]["x"]).all()
+    _same(eng, ref, CUSTOM_SIG)
+
+
 def _step_worlds(worlds, sig, steps, dt, substeps, active=None, pad=0):
     """`steps` calls of b3_batch_step_worlds_gpu on a device copy of the
     worlds, `pad` bytes apart."""
