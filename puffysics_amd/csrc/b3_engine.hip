@@ -326,6 +326,29 @@ hipError_t put_worlds(B3Engine* e, const unsigned char* host, uint32_t* dst) {
     return hipDeviceSynchronize();
 }
 
+/* Device memory of the step: per tile `scratch_words` of per-step scratch
+ * and, where several waves step a tile together, its manifold stage
+ * (stage_tile_words, tile_parts).  The stage holds every candidate pair: 6.8
+ * MB a tile for the bin's 37 shapes, 20.6 MB for 64, and 512 tiles of those
+ * are 10.6 GB.  Such a step only saves time, so where the device has no room
+ * for it the batch steps one wave per tile, which needs no stage. */
+hipError_t alloc_step(B3Engine* e, size_t scratch_words) {
+    if (e->stage_tile_words) {
+        hipError_t err = hipMalloc((void**)&e->pair_stage,
+            (size_t)e->tiles * e->tile_parts * e->stage_tile_words * sizeof(uint32_t));
+        if (err == hipSuccess) err = hipMalloc((void**)&e->scratch, (size_t)e->tiles * scratch_words * 4);
+        if (err != hipErrorOutOfMemory) return err;
+        (void)hipGetLastError();
+        if (e->pair_stage && (err = hipFree(e->pair_stage)) != hipSuccess) return err;
+        e->pair_stage = nullptr;
+        e->scratch = nullptr;
+        e->quad_waves = 0;
+        e->tile_parts = 1;
+        scratch_words = (size_t)e->g.tile_scr_words;
+    }
+    return hipMalloc((void**)&e->scratch, (size_t)e->tiles * scratch_words * 4);
+}
+
 /* ---- the step without allocation ----
  * b3_batch_step_worlds_gpu steps device-resident B3World structs in place
  * through the kernels of b3_batch_step_gpu, staging them as tiles in a
@@ -536,18 +559,11 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
             else if (e->shared_masks && 4 * e->tiles <= cus) e->tile_parts = 4;
             else if (e->shared_masks && 2 * e->tiles <= cus) e->tile_parts = 2;
             else if (g.max_c > 4 * g.max_j && 2 * e->tiles <= cus) e->tile_parts = 2;
-            err = hipMalloc((void**)&e->pair_stage,
-                (size_t)e->tiles * e->tile_parts * e->stage_tile_words * sizeof(uint32_t));
-            if (err != hipSuccess) {
-                (void)b3_engine_destroy(e);
-                return err;
-            }
         }
         /* per-step scratch: one per workgroup of a tile */
         size_t scratch_words = (size_t)e->tile_parts * g.tile_scr_words;
         if (e->quad_waves && quad_scratch > scratch_words) scratch_words = quad_scratch;
-        err = hipMalloc((void**)&e->scratch, (size_t)e->tiles * scratch_words * 4);
-        if (err != hipSuccess) {
+        if ((err = alloc_step(e, scratch_words)) != hipSuccess) {
             (void)b3_engine_destroy(e);
             return err;
         }
