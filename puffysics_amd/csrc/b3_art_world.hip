@@ -2,13 +2,17 @@
  * b3_art_world.hip - b3_step with articulated contacts (b3_art.hip), one
  * world to a wave, for batches that leave most of the chip idle at 64.
  *
+ * Only the worlds whose contacts go through their joint trees are stepped
+ * here, from where b3k_step_art leaves them: a wave has nothing to share out
+ * in any other world, and 64 of those step together there.
+ *
  * The lane code is built here with one world to a tile (as the CPU step
  * is): a world's words, workspace and rows are contiguous.  A workgroup of
  * one wave copies its world out of the tiles, steps it and writes what a
  * step can change back.  The workspace and the velocities are in LDS; the
  * world stays in global memory, where its lines are in the L1 and L2 (in
  * LDS, 52 KB a world, three worlds fit a CU: 14.1 ms for 1,000 arm worlds,
- * 6.3 for 300).
+ * 6.3 for 300, where the whole step was here: 5.6 for 1,000).
  */
 #define B3D_LANES 1
 #define B3D_ART_WAVE 1
@@ -40,51 +44,47 @@ B3D_FN void put_words(const uint32_t* world, uint32_t* column, int lo, int hi) {
     for (int k = lo + (int)threadIdx.x; k < hi; k += 64) column[(size_t)k * 64] = world[k];
 }
 
-/* step_world_art on a wave: the parts the ordinary step shares run on lane
- * 0, the articulated passes on all lanes (B3D_ART_WAVE).  Bound by the chain
- * of ~1,000 impulse responses a step (every contact point, twice a substep),
- * each of which goes through every link: 32 ms for the 17 links of an arm
- * world with 64 worlds to a wave, whose lanes hold different links; 18 ms
- * with a world to itself on one lane; 4.8 with a link to a lane, the links
- * outside the trees then in one pass. */
+/* The rest of step_world_art on a wave, for a world that b3k_step_art has
+ * handed over: its contacts are found and prepared, and its trees build.  The
+ * parts the ordinary step shares run on lane 0, the articulated passes on all
+ * lanes (B3D_ART_WAVE).  Bound by the chain of ~1,000 impulse responses a
+ * step (every contact point, twice a substep), each of which goes through
+ * every link: 32 ms for the 17 links of an arm world with 64 worlds to a
+ * wave, whose lanes hold different links; 18 ms with a world to itself on one
+ * lane; 4.3 with a link to a lane, the links outside the trees then in one
+ * pass (1,000 worlds 4.9). */
 __device__ inline void step_world_art_wave(const Lane& L, float* ws, int* tree, float dt, int substeps) {
     bool one = threadIdx.x == 0;
     ArtParams P = art_params(L, dt, substeps);
     ArtWs A = art_ws_of(L, ws);
     if (one) {
-        art_open(L, P);
+        body_prepass(L, P.h);
         prepare_joints(L, P.h);
-        tree[0] = ldi(L.w, H_JOINT_COUNT) > 0 && ldi(L.w, H_CONTACT_COUNT) > 0 && art_build(L, A);
-        tree[1] = A.n_links;
-        tree[2] = A.n_tree;
+        art_build(L, A);
+        tree[0] = A.n_links;
+        tree[1] = A.n_tree;
     }
     __syncthreads();
-    bool art = tree[0] != 0;
-    A.n_links = tree[1];
-    A.n_tree = tree[2];
-    if (art) art_warm_start(L, A);
+    A.n_links = tree[0];
+    A.n_tree = tree[1];
+    art_warm_start(L, A);
     __syncthreads();
     if (one) {
-        if (!art) wrow_warm(L);
         warm_start_joints(L);
         joint_geometry(L);
     }
     for (int s = 0; s < P.subs; s++) {
-        if (one) {
-            integrate_velocities(L);
-            if (!art) wrow_solve(L, P.inv_h, P.contact_speed, 1);
-        }
+        if (one) integrate_velocities(L);
         __syncthreads();
-        if (art) art_solve_contacts(L, A, P.inv_h, P.contact_speed, 1);
+        art_solve_contacts(L, A, P.inv_h, P.contact_speed, 1);
         __syncthreads();
         if (one) {
             solve_joints(L, P.h, P.inv_h, 1);
             integrate_positions(L, P.h, P.inv_dt);
             delta_geometry(L);
-            if (!art) wrow_solve(L, P.inv_h, P.contact_speed, 0);
         }
         __syncthreads();
-        if (art) art_solve_contacts(L, A, P.inv_h, P.contact_speed, 0);
+        art_solve_contacts(L, A, P.inv_h, P.contact_speed, 0);
         __syncthreads();
         if (one) {
             solve_joints(L, P.h, P.inv_h, 0);
@@ -97,21 +97,16 @@ __device__ inline void step_world_art_wave(const Lane& L, float* ws, int* tree, 
     }
 }
 
-/* b3k_step_art<false>, one world to a workgroup; 256 VGPRs, so that two waves
- * share a SIMD (4,000 arm worlds 20.0 -> 11.4 ms). */
+/* The worlds that b3k_step_art<false> handed over, one to a workgroup; 256
+ * VGPRs, so that two waves share a SIMD (4,000 arm worlds 20.0 -> 11.4 ms). */
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void b3k_step_art_world(uint32_t* live,
-        const uint32_t* snap, uint32_t* worlds, uint32_t* scratch, Geometry g, int count, float dt, int substeps,
-        const unsigned char* step_mask, const unsigned char* reset_mask, unsigned int opts) {
+        uint32_t* worlds, uint32_t* scratch, Geometry g, int count, float dt, int substeps,
+        const unsigned char* handed, unsigned int opts) {
     extern __shared__ uint32_t lds[];
     int turn = (int)blockIdx.x / kXcds;
     int w = (turn / kGroup * kXcds + (int)blockIdx.x % kXcds) * kGroup + turn % kGroup;
-    if (w >= count) return;
+    if (w >= count || !handed[w]) return;
     int tile = w / 64, slot = w % 64;
-    if (reset_mask && reset_mask[w]) {
-        restore_lanes(live, snap, g, tile, 0, 1, 1ull << slot);
-        __syncthreads();
-    }
-    if (step_mask && !step_mask[w]) return;
     uint32_t* column = live + (size_t)tile * g.world_words * 64 + slot;
     uint32_t* world = worlds + (size_t)w * g.world_words;
     for (int k0 = (int)threadIdx.x; k0 < g.world_words; k0 += 64 * 16) {
@@ -137,14 +132,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 
 }  // namespace
 
-bool b3i_art_world_fit(const Geometry& g) { return lds_bytes_of(g) <= kCuLdsBytes; }
+int b3i_art_worlds_per_cu(const Geometry& g) {
+    size_t fit = kCuLdsBytes / lds_bytes_of(g);
+    return fit < 8 ? (int)fit : 8;
+}
 
 hipError_t b3i_art_world_init() {
     return b3i_lds_limit((const void*)b3k_step_art_world);
 }
 
-hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
-        const unsigned char* reset_mask, hipStream_t stream) {
+hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigned char* handed, hipStream_t stream) {
     /* the engine's geometry with this file's one-world scratch tiles: 64 of
      * them are the words of one of the engine's */
     Geometry g;
@@ -152,7 +149,7 @@ hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigne
     if (!geometry_of(e->sig, &g, &world_bytes)) return hipErrorInvalidValue;
     int groups = (e->count + kGroup - 1) / kGroup;
     int grid = (groups + kXcds - 1) / kXcds * kXcds * kGroup;
-    b3k_step_art_world<<<grid, 64, lds_bytes_of(g), stream>>>(e->live, e->snap, e->art_worlds, e->scratch, g, e->count,
-        dt, substeps, step_mask, reset_mask, e->options);
+    b3k_step_art_world<<<grid, 64, lds_bytes_of(g), stream>>>(e->live, e->art_worlds, e->scratch, g, e->count, dt,
+        substeps, handed, e->options);
     return hipGetLastError();
 }

@@ -33,8 +33,9 @@ struct B3Engine {
     int quad_waves;          /* the step on quads of lanes (b3d_quad.h), a quarter tile to a workgroup of so
                                 many waves; 0: another step */
     bool joint_impulses_lds; /* the one-wave step keeps the joint impulses in LDS (b3d::ji_fit) */
-    uint32_t* art_worlds;    /* the worlds' words one after the other, for the articulated-contact step with
-                                one world to a wave (allocated with art_ws) */
+    uint32_t* art_worlds;    /* the worlds' words one after the other, then a byte per world (handed over), for
+                                the articulated-contact step with one world to a wave (allocated with art_ws;
+                                null: 64 to a wave) */
 };
 
 /* Waves per tile when the narrowphase is shared (two per SIMD: the shared
@@ -59,12 +60,12 @@ hipError_t b3i_art_init(B3Engine* e);
 hipError_t b3i_step_art(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
     const unsigned char* reset_mask, hipStream_t stream);
 
-/* The same one world to a wave (b3_art_world.hip): whether worlds of
- * geometry g fit in a CU's LDS; its set-up; its launch. */
-bool b3i_art_world_fit(const b3d::Geometry& g);
+/* The same one world to a wave (b3_art_world.hip): how many such waves a CU
+ * holds for worlds of geometry g (0: their LDS does not fit); its set-up; its
+ * launch on the worlds whose `handed` byte is set. */
+int b3i_art_worlds_per_cu(const b3d::Geometry& g);
 hipError_t b3i_art_world_init();
-hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigned char* step_mask,
-    const unsigned char* reset_mask, hipStream_t stream);
+hipError_t b3i_step_art_world(B3Engine* e, float dt, int substeps, const unsigned char* handed, hipStream_t stream);
 
 /* The step on quads (b3_quad.hip): whether it takes worlds of geometry g in
  * workgroups of `waves` waves, with the scratch words it needs per tile; its set-up on the current

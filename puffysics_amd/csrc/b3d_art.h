@@ -1136,13 +1136,17 @@ B3D_FN void art_open(const Lane& L, const ArtParams& P) {
     wrow_prepare(L, P.cs, P.ss);
 }
 
+/* Whether the world's contacts go through its joint trees: it has joints and
+ * contacts, and the trees build (into A). */
+B3D_FN bool art_applies(const Lane& L, ArtWs& A) {
+    return ldi(L.w, H_JOINT_COUNT) > 0 && ldi(L.w, H_CONTACT_COUNT) > 0 && art_build(L, A);
+}
+
 /* The rest of b3_step with articulated contacts (09_step.inl:148-264 with
  * 08_contacts.inl:194-232, 422-437).  Joints, integration and finalize are
- * the ordinary step's.  `built` is 1 when the caller has already built the
- * lane's tree, 0 when it has not tried. */
-B3D_FN void art_indep_rest(const Lane& L, ArtWs& A, const ArtParams& P, int built) {
+ * the ordinary step's.  `art` is art_applies of the lane's world. */
+B3D_FN void art_indep_rest(const Lane& L, const ArtWs& A, const ArtParams& P, bool art) {
     prepare_joints(L, P.h);
-    bool art = ldi(L.w, H_JOINT_COUNT) > 0 && ldi(L.w, H_CONTACT_COUNT) > 0 && (built || art_build(L, A));
     if (art) art_warm_start(L, A);
     else wrow_warm(L);
     warm_start_joints(L);
@@ -1172,15 +1176,22 @@ B3D_FN ArtWs art_ws_of(const Lane& L, float* ws) {
 }
 
 /* One world's b3_step built with articulated contacts.  `ws` is the lane's
- * workspace. */
-B3D_FN void step_world_art(const Lane& L0, float* ws, float dt, int substeps) {
+ * workspace.  With `handed`, a world whose contacts go through its trees is
+ * left, its contacts found and prepared, for a wave of its own to go on with
+ * (b3_art_world.hip), and *handed says whether it was. */
+B3D_FN void step_world_art(const Lane& L0, float* ws, float dt, int substeps, unsigned char* handed = nullptr) {
     if (!(dt > 0.0f)) return;
     Lane L = L0;
     L.sslot = wave_slot(L);
     ArtParams P = art_params(L, dt, substeps);
     art_open(L, P);
     ArtWs A = art_ws_of(L, ws);
-    art_indep_rest(L, A, P, 0);
+    bool art = art_applies(L, A);
+    if (handed) {
+        *handed = art;
+        if (art) return;
+    }
+    art_indep_rest(L, A, P, art);
 }
 
 /* ---- the reduced-coordinate integrator (b3_art_step) ---- */
@@ -1564,7 +1575,7 @@ B3D_FN void step_world_art_reduced(const Lane& L0, float* ws, float dt, int subs
     art_open(L, P);
     ArtWs A = art_ws_of(L, ws);
     if (!(supported && ldi(L.w, H_JOINT_COUNT) > 0 && art_build(L, A))) {
-        art_indep_rest(L, A, P, 0);
+        art_indep_rest(L, A, P, art_applies(L, A));
         return;
     }
     /* b3_warm_start: this world's tree builds, so the articulated branch

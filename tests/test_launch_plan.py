@@ -55,3 +55,20 @@ def test_without_room_for_the_stage(scene, count, kernel):
     assert less["create"] == OUT_OF_MEMORY and less["left"] == 0
     gravity, = plan([dict(call, budget=tight["used"], step="gravity")])
     assert gravity["step"] == 0 and gravity["launches"][0][0] == "b3k_step_gravity"
+
+
+# The largest batch with a wave to a world is eight turns of the waves that 8
+# CUs hold: eight waves a CU for 17 bodies, five for 34, two for 68.
+@pytest.mark.parametrize("caps,limit", [((17, 17, 64, 4), 512), ((34, 34, 128, 8), 320), ((68, 68, 256, 16), 128)])
+def test_articulated_contacts(caps, limit):
+    """Up to the limit worlds are handed to a wave each; past it, and on a
+    device without room for the worlds' copy, all step 64 to a wave."""
+    call = {"sig": signature(*caps), "count": limit, "cus": 8, "options": 2}
+    most, past = plan([call, dict(call, count=limit + 1)])
+    assert [x[:2] for x in most["launches"]] == [["b3k_step_art<0>", (limit + 63) // 64],
+                                                 ["b3k_step_art_world", (limit + 127) // 128 * 128]]
+    assert [x[:2] for x in past["launches"]] == [["b3k_step_art<0>", (limit + 64) // 64]]
+    tight, reduced = plan([dict(call, budget=most["used"] - 1), dict(call, step="art_step")])
+    assert tight["options"] == 0 and tight["step"] == 0 and tight["left"] == 0
+    assert [x[:2] for x in tight["launches"]] == [["b3k_step_art<0>", (limit + 63) // 64]]
+    assert [x[:2] for x in reduced["launches"]] == [["b3k_step_art<1>", (limit + 63) // 64]]
