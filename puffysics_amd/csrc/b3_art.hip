@@ -54,9 +54,9 @@ __global__ __launch_bounds__(64) void b3k_step_art(uint32_t* live, const uint32_
  * holds.  A turn takes about as long as its longest world, so the time grows
  * by turns; 64 to a wave, every lane waits for every other's rows, but 1,024
  * tiles are one turn.  Measured at the rule's edge, ms a vector step, one ->
- * 64 to a wave: the arm's 17 bodies (eight waves a CU) 38.9 at 16,384 worlds,
- * 51.0 at 17,000; twice the bodies (five) 215 at 10,240, 420 at 10,304; four
- * times (two) 899 at 4,096, 2,163 at 4,160.  Worlds that do not go through
+ * 64 to a wave: the arm's 17 bodies (eight waves a CU) 38.7 at 16,384 worlds,
+ * 49.2 at 17,000; twice the bodies (five) 216 at 10,240, 409 at 10,304; four
+ * times (two) 903 at 4,096, 2,099 at 4,160.  Worlds that do not go through
  * trees never leave the 64: at 16,384 chains that touch nothing take 0.84,
  * stacks 0.47, bins 4.2 (a wave each, they took 9.7, 4.2 and 38.8). */
 constexpr int kArtWorldTurns = 8;
