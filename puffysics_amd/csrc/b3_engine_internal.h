@@ -88,6 +88,10 @@ hipError_t b3i_quad_worlds_init();
 hipError_t b3i_step_quad_worlds(uint32_t* aos, size_t stride, size_t offset, uint32_t* scratch,
     const b3d::Geometry& g, int count, float dt, int substeps, const unsigned char* active, hipStream_t stream);
 
+/* The identity of the engine's build (b3_build.cpp).  Weak: an engine
+ * library may be of a build that has none. */
+extern "C" __attribute__((weak)) unsigned long long b3i_build_id(void);
+
 /* The engine's device is the current one. */
 inline hipError_t on_device(const B3Engine* e) {
     int dev = -1;

@@ -32,6 +32,7 @@ struct B3HoverEnvs {
     int n;
     B3HoverConfig config;
     B3Engine* engine;
+    bool same_build;     /* the engine library's, so that its structures can be read */
     uint32_t* tiles;
     size_t world_words;
     float *obs, *actions, *rewards, *terminals;  /* the caller's */
@@ -282,6 +283,7 @@ hipError_t b3_hover_create(B3HoverEnvs** out, int n, B3HoverConfig cfg, uint32_t
     if (!h) return hipErrorOutOfMemory;
     h->n = n;
     h->config = cfg;
+    h->same_build = b3i_build_id && b3i_build_id() == B3_BUILD_ID;
     h->obs = obs;
     h->actions = actions;
     h->rewards = rewards;
@@ -345,9 +347,9 @@ hipError_t b3_hover_reset(B3HoverEnvs* h, hipStream_t stream) {
 hipError_t b3_hover_step(B3HoverEnvs* h, hipStream_t stream) {
     if (!h) return hipErrorInvalidValue;
     B3Engine* e = h->engine;
-    /* one launch, unless the engine was told to step otherwise
-     * (articulated contacts) */
-    if (!(e->options & B3_ENGINE_ART_CONTACTS) && e->joint_impulses_lds) {
+    /* one launch, unless the engine is of another build or was told to step
+     * otherwise (articulated contacts) */
+    if (h->same_build && !(e->options & B3_ENGINE_ART_CONTACTS) && e->joint_impulses_lds) {
         hipError_t err = on_device(e);
         if (err != hipSuccess) return err;
         hk_step<<<e->tiles, 64, e->lds_bytes, stream>>>(e->live, e->snap, e->scratch, e->g, h->n, h->config, buffers(h),

@@ -1,5 +1,5 @@
 """What the engine allocates and launches, on a machine without a GPU: run as
-`python hipstand.py < calls.json`, a process of its own in which the stand-in
+`python hipstand.py LIBRARY < calls.json`, a process of its own in which the stand-in
 for the HIP runtime (tests/emu/hipstand.c) takes the libraries' HIP calls.
 `plan(calls)` runs it and returns one result per call."""
 import json
@@ -12,12 +12,12 @@ TESTS = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(TESTS)
 
 
-def plan(calls):
+def plan(calls, stand="libhipstand.so"):
     """Each call: {"sig", "count", "cus"} and optionally "budget" (bytes of
     device memory), "options", "step" ("step", "gravity", "art_step" or
     "hover").  Each result: {"create", "options", "step"} codes, "used" and
     "peak" bytes and the step's "launches" [name, grid, block, LDS bytes]."""
-    run = subprocess.run([sys.executable, os.path.abspath(__file__)], input=json.dumps(calls), capture_output=True,
+    run = subprocess.run([sys.executable, os.path.abspath(__file__), stand], input=json.dumps(calls), capture_output=True,
                          text=True, timeout=120)
     assert run.returncode == 0, run.stderr
     return json.loads(run.stdout)
@@ -36,7 +36,7 @@ def _main():
     sys.modules["torch"] = None            # its own HIP runtime stays out of this process
     sys.path.insert(0, ROOT)
     import ctypes as C
-    stand = C.CDLL(os.path.join(TESTS, "emu", "libhipstand.so"), mode=C.RTLD_GLOBAL)
+    stand = C.CDLL(os.path.join(TESTS, "emu", sys.argv[1]), mode=C.RTLD_GLOBAL)
     stand.hipstand_budget.argtypes = [C.c_size_t]
     stand.hipstand_used.restype = C.c_size_t
     stand.hipstand_launch.restype = C.c_char_p

@@ -72,3 +72,17 @@ def test_articulated_contacts(caps, limit):
     assert tight["options"] == 0 and tight["step"] == 0 and tight["left"] == 0
     assert [x[:2] for x in tight["launches"]] == [["b3k_step_art<0>", (limit + 63) // 64]]
     assert [x[:2] for x in reduced["launches"]] == [["b3k_step_art<1>", (limit + 63) // 64]]
+
+
+@pytest.mark.parametrize("stand,options,kernels", [
+    ("libhipstand.so", 0, ["hk_step"]),
+    ("libhipstand.so", 2, ["hk_action", "b3k_step_art<0>", "b3k_step_art_world", "hk_reward", "b3k_restore",
+                           "hk_observe"]),
+    ("libhipstand_other.so", 0, ["hk_action", "b3k_step<1,1>", "hk_reward", "b3k_restore", "hk_observe"])])
+def test_hover_with_an_engine_of_another_build(stand, options, kernels):
+    """The hover library steps in one launch only with the engine that it was
+    built with, whose structures it reads; with another, and with articulated
+    contacts, through the engine's public calls."""
+    one, = plan([{"count": 130, "step": "hover", "options": options}], stand)
+    assert (one["create"], one["options"], one["step"], one["left"]) == (0, 0, 0, 0)
+    assert [x[0] for x in one["launches"]] == kernels
