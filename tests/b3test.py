@@ -241,6 +241,20 @@ def diff_words(a, b, sig):
     return np.argwhere(d)
 
 
+def on_shared_tiles(worlds, sig):
+    """The worlds in their capacity set with 17 joints, which is more than the
+    step on quads takes, and its signature: batches of up to one tile per CU
+    then step on shared tiles (b3k_step_shared) at any size."""
+    from puffysics_amd.b3types import empty_worlds, signature
+    wide = signature(*(len(worlds[f][0]) for f in ("bodies", "shapes", "contacts")), 17)
+    out = empty_worlds(wide, len(worlds))
+    for f in worlds.dtype.names:
+        if f != "joints":
+            out[f] = worlds[f]
+    out["joints"][:, :worlds["joints"].shape[1]] = worlds["joints"]
+    return out, wide
+
+
 # ---- the contacts' prepared solver fields (written only with B3_ENGINE_KEEP_SOLVER_FIELDS) ----
 
 SOLVER_FIELDS = ("inv_mass_a", "inv_mass_b", "inv_i_a", "inv_i_b", "softness", "center_a", "center_b",

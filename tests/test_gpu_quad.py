@@ -30,10 +30,11 @@ def _same(eng, ref, sig):
 
 # One world, the edges of a workgroup's 16 worlds and of a 64-world tile;
 # then batches on both sides of a quarter and of half a tile per CU (64 and
-# 128 tiles on 256 CUs).
+# 128 tiles on 256 CUs), and chains on the most shared tiles of one turn.
 @pytest.mark.parametrize("scene,count,steps", [
     (1, 1, 40), (1, 17, 40), (2, 15, 30), (2, 65, 30), (3, 16, 20), (3, 33, 20), (4, 1, 60), (4, 31, 25), (5, 63, 25),
-    (5, 49, 25), (2, 4096, 4), (2, 4097, 4), (3, 4100, 3), (4, 4100, 2), (5, 4100, 4), (3, 8192, 3), (5, 8200, 3), (2, 8200, 3)])
+    (5, 49, 25), (2, 4096, 4), (2, 4097, 4), (3, 4100, 3), (4, 4100, 2), (5, 4100, 4), (3, 8192, 3), (5, 8200, 3), (2, 8200, 3),
+    (3, 8200, 3), (3, 16384, 2)])
 def test_batch_edges(scene, count, steps):
     worlds = scenes.build(scene, count)
     ref = clone(worlds)

@@ -129,8 +129,8 @@ def test_no_alloc_step_skips_corrupt_worlds():
 
 
 def test_no_alloc_step_runs_a_large_batch_in_chunks():
-    """2,000 arm worlds with a step mask are three chunks of the 64 MiB array
-    (896 + 896 + 208 worlds): equal to the engine's step on the same
+    """2,000 arm worlds with a step mask are two chunks of the 64 MiB array
+    (1,152 + 848 worlds): equal to the engine's step on the same
     worlds."""
     lib = _lib()
     scene, count = 5, 2000
