@@ -168,8 +168,9 @@ def joint_impulses_fit(max_b, max_s, max_c, max_j):
 def kernel_name(scene, count):
     """The step kernel a batch launches (b3_engine_create): b3k_step<JI, true>
     for worlds of at most two shapes; else b3k_step_quad<W, CR, JR> up to a
-    quarter (W = 8) or half a tile (4) per CU, b3k_step_shared<Masks, JL>
-    when the tiles fit one per CU, b3k_step<JI, false> when they do not."""
+    quarter (W = 8) or half a tile (4) per CU, b3k_step_shared<Masks, JL> when
+    the tiles fit one per CU (two, for worlds of 12 to 64 shapes),
+    b3k_step<JI, false> when they do not."""
     import torch
     from puffysics_amd import scenes
     tiles = (count + 63) // 64
@@ -364,7 +365,7 @@ def run_workload(scene, count, steps, warmup, repeats, event_every, digest, cpu_
     mean_stepped = stepped / steps
     bytes_env = float(bytes_sum) / stepped
     k_ms = kernel_ms[med]
-    kernel = "b3k_step_art<false>" if art else kernel_name(scene, count)
+    kernel = "b3k_step_art<false>, b3k_step_art_world" if art else kernel_name(scene, count)
     hbm_gbs = bytes_launch / (k_ms * 1e-3) / 1e9
     flops_env, counted = counted_flops(scene, start, steps)
     tflops = flops_env * mean_stepped / (k_ms * 1e-3) / 1e12
@@ -521,8 +522,8 @@ def _short(name):
 
 
 def _step_kernel(names):
-    """The workload's step kernel: the launched kernel named b3k_step<JI> or
-    b3k_step_shared<...>."""
+    """The workload's step kernel: the launched kernel named b3k_step<...>,
+    b3k_step_shared<...> or b3k_step_quad<...>."""
     cands = [n for n in names if _short(n).startswith(("b3k_step<", "b3k_step_shared<", "b3k_step_quad<"))]
     if len(set(cands)) != 1:
         raise SystemExit("expected one step kernel, found %s" % sorted(set(cands)))

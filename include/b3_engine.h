@@ -122,8 +122,11 @@ hipError_t b3_engine_device_view(const B3Engine* engine, void** tiles, size_t* w
  * worlds step as usual.  The contacts' solver fields are then always
  * written back.  Turning it on allocates a workspace of
  * 4 * count * ((171 + 22) * max_bodies + 209) bytes (the one exception to
- * b3_engine_create being the only allocating call); it is freed by
- * b3_engine_destroy.  This mode costs far more per contact than the
+ * b3_engine_create being the only allocating call) and, where there is room
+ * for it, a copy of the worlds of count * (sizeof(B3World) + 1) bytes for
+ * batches whose articulated worlds take a wave each (up to 64 worlds a CU of
+ * 17 bodies, fewer of more; larger batches step 64 worlds to a wave).  Both
+ * are freed by b3_engine_destroy.  This mode costs far more per contact than the
  * default, as in the reference.  The force-law entry points return
  * hipErrorNotSupported while it is on. */
 #define B3_ENGINE_ART_CONTACTS 2u
@@ -131,8 +134,10 @@ hipError_t b3_engine_device_view(const B3Engine* engine, void** tiles, size_t* w
  * choice).  A batch of at most a quarter (half) of a 64-world tile per CU
  * normally runs with four workgroups per tile, each of eight (four) waves
  * that give every world four lanes each (a contact or joint solve to four
- * lanes, everything independent within a world spread over all of them).  A batch of at most one
- * tile per CU runs with eight waves per tile, one lane of each to a world:
+ * lanes, everything independent within a world spread over all of them),
+ * where a world's rows fit (at most 16 joints and 64 shapes).  Other batches
+ * of at most one tile per CU, of worlds of 12 to 64 shapes of at most two,
+ * run with eight waves per tile, one lane of each to a world:
  * they share the narrowphase (its pairs are independent; four to seven
  * waves collide, as many as have LDS rows for their clip polygons), the
  * contact sweeps and warm start (contacts on disjoint dynamic bodies, level
@@ -142,7 +147,10 @@ hipError_t b3_engine_device_view(const B3Engine* engine, void** tiles, size_t* w
  * contact-bound worlds split each tile over `parts` = 2 or 4 such workgroups
  * when the CUs allow.  Both allocate at creation a staging buffer of 4 *
  * tiles * parts * 64 * (1 + max(40 * max_shapes * (max_shapes - 1) / 2, 2 *
- * max_contacts)) bytes (parts 1 for the first).  Worlds of at most two
+ * max_contacts)) bytes (parts 1 for the first), the first also 416 *
+ * max_contacts bytes of scratch per world: at 37 shapes 6.8 MB a tile, 3.5
+ * GB for 32,768 worlds.  Where the device has no room for them, the batch
+ * steps one wave per tile.  Worlds of at most two
  * shapes (one candidate pair) always step one wave per tile.  This option
  * launches one wave per tile as for larger batches.  Results are identical
  * either way. */
@@ -191,7 +199,8 @@ hipError_t b3_batch_art_step_gpu(B3Engine* engine, float dt, int substeps, const
  * allocating routine.
  *
  * Worlds whose per-world state fits a workgroup's LDS (at most 64 shapes
- * and 16 joints, and roughly 60 bodies or 400 contacts) are stepped where
+ * and 16 joints, and at most 91 bodies or 483 contacts where the world has
+ * little else) are stepped where
  * they are, and only their per-step scratch is in the array; others are
  * staged there as tiles with their scratch beside them.
  *

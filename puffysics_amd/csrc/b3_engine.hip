@@ -1,9 +1,10 @@
 /*
  * b3_engine.hip - MI355X kernels and C ABI of the batched stepping engine.
  *
- * Launch geometry: every batch is split into tiles of 64 worlds, one
- * wave64 workgroup per tile, so each lane owns one world.  The grid is the
- * tile count (1024 workgroups at 65,536 worlds).  Worlds are stored as
+ * Launch geometry: every batch is split into tiles of 64 worlds.  Large
+ * batches step one wave64 workgroup per tile, so each lane owns one world and
+ * the grid is the tile count (1024 workgroups at 65,536 worlds); smaller ones
+ * give a tile several waves or workgroups (b3_engine_create).  Worlds are stored as
  * word-transposed tiles (b3d_lane.h), which makes every per-field access of
  * a wave a single 256-byte row.
  *
@@ -23,7 +24,8 @@
  *                              0's row kept for the step, for worlds of at
  *                              most two shapes)
  *   b3k_step_shared<Masks, JL> the same for batches of at most one tile per
- *                              CU, with the contact writes, preparation,
+ *                              CU (worlds of many shapes: two) that do not
+ *                              step on quads of lanes (b3_quad.hip), with the contact writes, preparation,
  *                              contact sweeps and body and joint work split
  *                              over eight waves per tile and the
  *                              narrowphase over the four to seven of them
@@ -484,8 +486,6 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
             (void)b3_engine_destroy(e);
             return err;
         }
-        /* A batch of at most one tile per CU shares each tile's step among
-         * kTileWaves waves (b3k_step_shared). */
         int cus = 0;
         /* wave 0's rows and the helpers' clip rows, then the old contact
          * keys, the overlap masks and the hit bits of the candidates */
@@ -515,15 +515,17 @@ hipError_t b3_engine_create(B3Engine** out, B3Batch worlds, unsigned long long c
          * CU: up to there each world of three shapes or more steps on a quad
          * of lanes of each of eight waves (b3d_quad.h), and up to half a tile
          * per CU, two workgroups to a CU, of four waves (where their LDS
-         * fits: not the bin).  Measured, the shared step -> quads, us: at
-         * 4,096 worlds (64 tiles) stacks 207 -> 91, chains 395 -> 153, bin
+         * fits: not the bin).  Measured, the step kernel, shared -> quads,
+         * us: at 4,096 worlds (64 tiles) stacks 207 -> 91, chains 395 -> 153, bin
          * 686 -> 395, the arm 320 -> 131 (at 300 worlds 313 -> 117); at
          * 8,192 stacks 211 -> 132, chains 405 -> 210, the arm 336 -> 225.
          * With more workgroups than the CUs hold at once the shared step
          * wins: at 16,384 worlds stacks 234 against 243, the arm 398
-         * against 442 (chains 430 against 408).  Of two-shape worlds those
-         * with a contact gain (hover 34.9 -> 26.3 at 4,096) and those without
-         * lose to the barriers (a free sphere's step and task 23.9 -> 28.1). */
+         * against 442 (chains 430 against 408).  Of two-shape worlds, one
+         * wave per tile -> quads, those with a contact gain at 4,096 (hover
+         * 33.5 -> 25.6; at 8,192 34.1 -> 36.4) and those without lose to the
+         * barriers (a free sphere 13.0 -> 14.6, 13.3 -> 18.7); the capacities
+         * do not tell them apart. */
         e->quad_waves = 0;
         if (g.max_s > 2) {
             if (4 * e->tiles <= cus && b3i_quad_fit(g, 8, &quad_scratch)) e->quad_waves = 8;
@@ -754,8 +756,12 @@ hipError_t b3_batch_step_worlds_gpu(B3Batch worlds, unsigned long long config_si
      * orders the graph's launches against other calls. */
     if (!capturing && (err = hipStreamWaitEvent(stream, nd->last, 0)) != hipSuccess) return err;
     /* Worlds that fit step in place on quads, with only their scratch in
-     * the array; the others are staged as tiles (both sides: the comment at
-     * b3k_step_quad_worlds). */
+     * the array; the others are staged as tiles, one lane a world.  In place
+     * is faster at every size measured, us a call staged -> in place at 64 /
+     * 2,000 / 30,000 worlds: hover 57 -> 29, 64 -> 29, 256 -> 207; stacks 377
+     * -> 93, 432 -> 91, 3,902 -> 874; chains 783 -> 148, 1,669 -> 152, 15,560
+     * -> 1,544; at 64 / 2,000 / 8,000 the arm 871 -> 120, 2,786 -> 266, 8,504
+     * -> 962, the bin 2,959 -> 329, 15,941 -> 2,614, 57,257 -> 9,591. */
     size_t quad_words = b3i_quad_worlds_tile_words(g);
     bool quad = quad_words != 0 && quad_words <= kNoAllocWords;
     if (quad) chunk_tiles = kNoAllocWords / quad_words;

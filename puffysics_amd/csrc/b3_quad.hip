@@ -19,8 +19,10 @@ namespace {
  * 160 levels of joint solves at 1.83 us (a solve's ~400 instructions and
  * ~90 row loads at ~5 cycles each, a wave alone on its SIMD); on quads with
  * the rows in registers 153 us.  W: waves of the workgroup; CR, JR: contacts
- * and joints of a world that a wave keeps in registers (more contacts than
- * two or three spill: with four, the chains took 197 us). */
+ * and joints of a world that a wave keeps in registers (with four contacts
+ * the chains took 197 us).  Of the 256 VGPRs that two waves per SIMD allow
+ * <8, 2, 1> spills none, <8, 2, 2> and <4, 2, 2> 18, <4, 3, 1> 49 and
+ * <4, 1, 4> 61, to private memory. */
 template <int W, int CR, int JR, class Law>
 __device__ __attribute__((always_inline)) inline void step_quad(uint32_t* live, const uint32_t* snap, uint32_t* scratch,
         uint32_t* stage, size_t stage_tile_words, const Geometry& g, const QuadLayout& q, int count, float dt,
