@@ -545,9 +545,10 @@ def _counter_means(rows, picks):
 
 def code_object_resources(kernel):
     """Registers and static memory of a kernel (its short name) from the
-    AMDGPU metadata notes of the gfx950 code object in the in-tree
-    puffysics_amd/libb3engine.so (llvm-readelf --notes of the object that
-    clang-offload-bundler takes out of the library's .hip_fatbin section);
+    AMDGPU metadata notes of the gfx950 code objects in the in-tree
+    puffysics_amd/libb3engine.so (llvm-readelf --notes of the objects that
+    clang-offload-bundler takes out of the library's .hip_fatbin section, a
+    bundle per source file);
     None when the tools or the kernel are missing.  .vgpr_count counts the
     AGPRs too."""
     import subprocess
@@ -558,11 +559,18 @@ def code_object_resources(kernel):
         with tempfile.TemporaryDirectory() as tmp:
             fat, co = os.path.join(tmp, "fat.bin"), os.path.join(tmp, "co.elf")
             subprocess.run(["objcopy", "-O", "binary", "--only-section=.hip_fatbin", lib, fat], check=True)
-            subprocess.run([os.path.join(llvm, "clang-offload-bundler"), "--unbundle", "--type=o",
-                            "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", "--input=" + fat, "--output=" + co],
-                           check=True)
-            notes = subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", co], check=True,
-                                   capture_output=True, text=True).stdout
+            magic = b"__CLANG_OFFLOAD_BUNDLE__"
+            with open(fat, "rb") as f:
+                bundles = f.read().split(magic)[1:]
+            notes = ""
+            for bundle in bundles:
+                with open(fat, "wb") as f:
+                    f.write(magic + bundle)
+                subprocess.run([os.path.join(llvm, "clang-offload-bundler"), "--unbundle", "--type=o",
+                                "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", "--input=" + fat, "--output=" + co],
+                               check=True)
+                notes += subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", co], check=True,
+                                        capture_output=True, text=True).stdout
     except (OSError, subprocess.CalledProcessError):
         return None
     blocks, cur = [], None
