@@ -3311,6 +3311,8 @@ B3D_FN int joint_levels_scan(const Lane& L, int nj, int nb, int place) {
         int la = da ? jsch_get(L, jsch_last(L, a)) : 0;
         int lb = db ? jsch_get(L, jsch_last(L, b)) : 0;
         int lev = (la > lb ? la : lb) + 1;
+        /* no dynamic body keeps the two solves of its row apart */
+        if (!da && !db) lev = 1 + t / nj;
         if (da) jsch_set(L, jsch_last(L, a), lev);
         if (db) jsch_set(L, jsch_last(L, b), lev);
         int at = jsch_get(L, jsch_p(L, lev));

@@ -350,6 +350,8 @@ B3Q_FN void quad_joint_levels(const QLane& Q, int nj, int nb, int* wg) {
             int la = da ? lgeti(Q, Q.q.jlast + a) : 0;
             int lb = db ? lgeti(Q, Q.q.jlast + b) : 0;
             int lev = (la > lb ? la : lb) + 1;
+            /* no dynamic body keeps the two solves of its row apart */
+            if (!da && !db) lev = 1 + it;
             if (da) lseti(Q, Q.q.jlast + a, lev);
             if (db) lseti(Q, Q.q.jlast + b, lev);
             lseti(Q, Q.q.jlev + j, it == 0 ? lev : lgeti(Q, Q.q.jlev + j) | (lev << 8));

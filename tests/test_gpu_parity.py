@@ -267,6 +267,55 @@ def test_feature_worlds_with_hinges_bit_exact(count, shared):
     assert np.abs(ref["joints"]["motor_impulse"]).max() > 0
 
 
+@pytest.mark.parametrize("kernel", ["quads", "shared-17-joints", "shared-130-tiles", "one_wave"])
+def test_joints_without_a_dynamic_body(kernel):
+    """Joints between static and kinematic bodies that still hold impulses
+    (from when a body was dynamic): each of a pass's solves takes its part
+    of them off, one after the other."""
+    from b3test import feature_worlds, on_shared_tiles, oracle_step_batch
+    from puffysics_amd.b3types import B3_KINEMATIC
+    from puffysics_amd.creation import CUSTOM_SIG
+    from puffysics_amd.engine import B3_ENGINE_KEEP_SOLVER_FIELDS, B3_ENGINE_ONE_WAVE_PER_TILE, B3Engine
+    some, count = 100, 8260 if kernel == "shared-130-tiles" else 100
+    worlds, sig = feature_worlds(some), CUSTOM_SIG
+    rng = np.random.default_rng(9)
+    for f in ("linear_impulse", "angular_impulse"):
+        for a in "xyz":
+            worlds["joints"][f][a] = rng.normal(0.0, 0.3, worlds["joints"][f][a].shape)
+    for f in ("spring_impulse", "motor_impulse", "lower_impulse", "upper_impulse"):
+        worlds["joints"][f] = rng.uniform(0.0, 0.3, worlds["joints"][f].shape)
+    for k in range(some):
+        for j in range(int(worlds["joint_count"][k])):
+            for f in ("body_a", "body_b"):
+                if (j + k) % 2 == 0:
+                    b = worlds["joints"][f][k, j]
+                    if worlds["bodies"]["type"][k, b] == 2:
+                        worlds["bodies"]["type"][k, b] = B3_KINEMATIC
+                        worlds["bodies"]["flags"][k, b] &= 0xffffefff
+    if kernel == "shared-17-joints":
+        worlds, sig = on_shared_tiles(worlds, sig)
+    pick = np.arange(count) % some
+    ref = clone(worlds)
+    eng = B3Engine(worlds[pick], sig)
+    eng.set_options(B3_ENGINE_KEEP_SOLVER_FIELDS | (B3_ENGINE_ONE_WAVE_PER_TILE if kernel == "one_wave" else 0))
+    for _ in range(4):
+        oracle_step_batch(ref, sig, 1.0 / 60.0, 4)
+        eng.step(1.0 / 60.0, 4)
+    torch.cuda.synchronize()
+    got = eng.download()
+    eng.close()
+    inert = np.zeros(ref["joints"].shape, bool)
+    for k in range(some):
+        for j in range(int(ref["joint_count"][k])):
+            ab = [ref["joints"][f][k, j] for f in ("body_a", "body_b")]
+            inert[k, j] = not (ref["bodies"]["type"][k, ab] == 2).any()
+    assert (np.abs(ref["joints"]["linear_impulse"]["x"][inert]) > 0).sum() > 20
+    for k in range(0, count, some):
+        part = got[k:k + some]
+        bad = diff_words(part, ref[:len(part)], sig)
+        assert len(bad) == 0, describe(bad, part, ref, worlds)
+
+
 def test_default_options_differ_only_in_solver_fields():
     """Without B3_ENGINE_KEEP_SOLVER_FIELDS the worlds evolve identically;
     only the prepared solver fields of the live contacts are not written."""
