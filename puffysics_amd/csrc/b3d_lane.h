@@ -2015,16 +2015,24 @@ B3D_FN void sched_build(const Lane& L) {
 #pragma unroll
         for (int k = 0; k < kSchedChunk; k++)
             if (c0 + k < cc) hds[k] = chead_load(L, c0 + k);
+        /* what a solve writes goes by the bodies' flags, whatever their type */
+        int da[kSchedChunk], db[kSchedChunk];
+#pragma unroll
+        for (int k = 0; k < kSchedChunk; k++) {
+            if (c0 + k >= cc) continue;
+            da[k] = is_dyn_flag(L, hds[k].a);
+            db[k] = is_dyn_flag(L, hds[k].b);
+        }
 #pragma unroll
         for (int k = 0; k < kSchedChunk; k++) {
             int c = c0 + k;
             if (c >= cc) continue;
             const CHead& hd = hds[k];
-            int la = (hd.flags & CF_DYN_A) ? sch_get(L, sch_last(L, hd.a)) : 0;
-            int lb = (hd.flags & CF_DYN_B) ? sch_get(L, sch_last(L, hd.b)) : 0;
+            int la = da[k] ? sch_get(L, sch_last(L, hd.a)) : 0;
+            int lb = db[k] ? sch_get(L, sch_last(L, hd.b)) : 0;
             int lev = (la > lb ? la : lb) + 1;
-            if (hd.flags & CF_DYN_A) sch_set(L, sch_last(L, hd.a), lev);
-            if (hd.flags & CF_DYN_B) sch_set(L, sch_last(L, hd.b), lev);
+            if (da[k]) sch_set(L, sch_last(L, hd.a), lev);
+            if (db[k]) sch_set(L, sch_last(L, hd.b), lev);
             sch_set(L, sch_level(L, c), lev | (hd.pc << 16));
             sch_set(L, sch_p(L, lev), sch_get(L, sch_p(L, lev)) + 1);
             if (lev > nlev) nlev = lev;

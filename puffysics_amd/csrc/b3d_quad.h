@@ -306,16 +306,24 @@ B3Q_FN void quad_levels(const QLane& Q, int cc, int nb, int* wg) {
 #pragma unroll
         for (int k = 0; k < kSchedChunk; k++)
             if (c0 + k < cc) hd[k] = lgeti(Q, Q.q.heads + c0 + k);
+        /* what a solve writes goes by the bodies' flags, whatever their type */
+        int da[kSchedChunk], db[kSchedChunk];
+#pragma unroll
+        for (int k = 0; k < kSchedChunk; k++) {
+            if (c0 + k >= cc) continue;
+            da[k] = is_dyn_flag(Q.L, hd[k] & 255);
+            db[k] = is_dyn_flag(Q.L, (hd[k] >> 8) & 255);
+        }
 #pragma unroll
         for (int k = 0; k < kSchedChunk; k++) {
             int c = c0 + k;
             if (c >= cc) continue;
-            int a = hd[k] & 255, b = (hd[k] >> 8) & 255, fl = hd[k] >> 20;
-            int la = (fl & CF_DYN_A) ? lgeti(Q, Q.q.last + a) : 0;
-            int lb = (fl & CF_DYN_B) ? lgeti(Q, Q.q.last + b) : 0;
+            int a = hd[k] & 255, b = (hd[k] >> 8) & 255;
+            int la = da[k] ? lgeti(Q, Q.q.last + a) : 0;
+            int lb = db[k] ? lgeti(Q, Q.q.last + b) : 0;
             int lev = (la > lb ? la : lb) + 1;
-            if (fl & CF_DYN_A) lseti(Q, Q.q.last + a, lev);
-            if (fl & CF_DYN_B) lseti(Q, Q.q.last + b, lev);
+            if (da[k]) lseti(Q, Q.q.last + a, lev);
+            if (db[k]) lseti(Q, Q.q.last + b, lev);
             lseti(Q, Q.q.level + c, lev);
             lseti(Q, Q.q.pos + lev, lgeti(Q, Q.q.pos + lev) + 1);
             if (lev > nlev) nlev = lev;

@@ -316,6 +316,49 @@ def test_joints_without_a_dynamic_body(kernel):
         assert len(bad) == 0, describe(bad, part, ref, worlds)
 
 
+@pytest.mark.parametrize("kernel", ["quads", "shared-17-joints", "shared-130-tiles", "one_wave"])
+def test_bodies_whose_flag_and_type_disagree(kernel):
+    """Bodies switched to kinematic by their type alone, whose velocities a
+    solve still writes (that goes by the flag): contacts on one such body
+    keep their order, which shows in a negative zero and in the NaN of a
+    neighbour of infinite speed."""
+    from b3test import feature_worlds, on_shared_tiles, oracle_step_batch
+    from puffysics_amd.b3types import B3_KINEMATIC
+    from puffysics_amd.creation import CUSTOM_SIG
+    from puffysics_amd.engine import B3_ENGINE_KEEP_SOLVER_FIELDS, B3_ENGINE_ONE_WAVE_PER_TILE, B3Engine
+    some, count = 100, 8260 if kernel == "shared-130-tiles" else 100
+    worlds, sig = feature_worlds(some, hinges=False), CUSTOM_SIG
+    for _ in range(20):
+        oracle_step_batch(worlds, sig, 1.0 / 60.0, 4)
+    b = worlds["bodies"]
+    for k in range(some):
+        for i in range(1 + k % 3, int(worlds["body_count"][k]), 3):
+            b["type"][k, i] = B3_KINEMATIC
+            for f in ("lin_vel", "ang_vel"):
+                for a in "xyz":
+                    b[f][a][k, i] = -0.0
+        if k % 2:
+            b["lin_vel"]["y"][k, 1 + (k + 1) % 3] = -np.inf
+    if kernel == "shared-17-joints":
+        worlds, sig = on_shared_tiles(worlds, sig)
+    pick = np.arange(count) % some
+    ref = clone(worlds)
+    eng = B3Engine(worlds[pick], sig)
+    eng.set_options(B3_ENGINE_KEEP_SOLVER_FIELDS | (B3_ENGINE_ONE_WAVE_PER_TILE if kernel == "one_wave" else 0))
+    for _ in range(2):
+        oracle_step_batch(ref, sig, 1.0 / 60.0, 4)
+        eng.step(1.0 / 60.0, 4)
+    torch.cuda.synchronize()
+    got = eng.download()
+    eng.close()
+    flagged = (ref["bodies"]["type"] == B3_KINEMATIC) & (ref["bodies"]["flags"] & 0x1000 != 0)
+    assert np.isnan(ref["bodies"]["lin_vel"]["x"][flagged]).sum() > 10
+    for k in range(0, count, some):
+        part = got[k:k + some]
+        bad = diff_words(part, ref[:len(part)], sig)
+        assert len(bad) == 0, describe(bad, part, ref, worlds)
+
+
 def test_default_options_differ_only_in_solver_fields():
     """Without B3_ENGINE_KEEP_SOLVER_FIELDS the worlds evolve identically;
     only the prepared solver fields of the live contacts are not written."""
