@@ -276,12 +276,14 @@ constexpr int PR_RA = 0, PR_NMASS = 3, PR_RB = 4, PR_LEVER = 7, kPRows = 2;
  * rotation's x, y, the point anchors and separation, the weld's angular
  * error; the inverse of the point rows' 3x3 mass matrix (JS_PKI) and the
  * perpendicular rows' 2x2 mass matrix with its reciprocal determinant
- * (JS_KXX, JS_KXY, JS_KYY, JS_KINV; NaN when singular).  Last, fixed for
+ * (JS_KXX, JS_KXY, JS_KYY, JS_KINV; kSingular when singular).  Last, fixed for
  * the step: the hinge axis through each body's inverse inertia (JS_IAX,
  * JS_IBX). */
 constexpr int JS_KEY = 0, JS_AB = 1, JS_INFO = 2, JS_TW = 3, JS_RELX = 4, JS_RELY = 5, JS_PX = 6, JS_PY = 9,
               JS_RA = 12, JS_RB = 15, JS_PSEP = 18, JS_CV = 21, JS_PKI = 24, JS_KXX = 33, JS_KXY = 34, JS_KYY = 35,
               JS_KINV = 36, JS_IAX = 37, JS_IBX = 40, kJointScr = 43;
+/* not the reciprocal of any determinant above the limit, nor of a NaN */
+constexpr float kSingular = -1.0f;
 constexpr int JF_WELD = 1, JF_FIXED = 2, JF_SPRING = 4, JF_MOTOR = 8, JF_LIMIT = 16, JF_DYN_A = 32, JF_DYN_B = 64;
 
 constexpr int kStatic = 0, kKinematic = 1, kDynamic = 2;
@@ -2355,7 +2357,7 @@ B3D_FN JGeo joint_geo(int info, Q dqa, Q dqb, V3 dpa, V3 dpb, Q fqa, Q fqb, V3 f
         o.kyy = dot(o.py, mv(isum, o.py));
         o.kxy = dot(o.px, mv(isum, o.py));
         float det = o.kxx * o.kyy - o.kxy * o.kxy;
-        o.kinv = det <= 1.0e-12f ? __builtin_nanf("") : 1.0f / det;
+        o.kinv = det <= 1.0e-12f ? kSingular : 1.0f / det;
     }
     return o;
 }
@@ -3027,7 +3029,7 @@ struct JRow {
     /* revolute */
     V3 axis, px, py;
     V3 ia_ax, ib_ax;        /* inverse inertias times the axis */
-    float kxx, kxy, kyy, kinv;   /* perpendicular rows' matrix, 1 / det or NaN */
+    float kxx, kxy, kyy, kinv;   /* perpendicular rows' matrix, 1 / det or kSingular */
     float axial_mass, max_torque, speed, target, lower, upper;
     Soft spring_soft;
     float tw, relx, rely;
@@ -3598,7 +3600,7 @@ B3D_FN void solve_revolute(const Lane& L, int j, const JRow& r, float h, float i
         V2 sol;
         sol.x = 0.0f;
         sol.y = 0.0f;
-        if (r.kinv == r.kinv) {
+        if (r.kinv != kSingular) {
             sol.x = r.kinv * (r.kyy * rhs.x - r.kxy * rhs.y);
             sol.y = r.kinv * (-r.kxy * rhs.x + r.kxx * rhs.y);
         }

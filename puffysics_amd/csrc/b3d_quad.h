@@ -989,7 +989,7 @@ B3Q_FN void jq_solve(const QLane& Q, JQ& r, const JScal& k, float h, float inv_h
         V2 sol;
         sol.x = 0.0f;
         sol.y = 0.0f;
-        if (k.kinv == k.kinv) {
+        if (k.kinv != kSingular) {
             sol.x = k.kinv * (k.kyy * rhs.x - k.kxy * rhs.y);
             sol.y = k.kinv * (-k.kxy * rhs.x + k.kxx * rhs.y);
         }

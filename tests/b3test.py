@@ -362,6 +362,21 @@ def feature_worlds(count, seed=7, hinges=True):
     return w
 
 
+def nan_hinge_worlds(count):
+    """The coverage worlds after some steps, a hinged body of every other one
+    at a NaN orientation: its hinge's rows have a NaN determinant, which is
+    not a singular one."""
+    from puffysics_amd.creation import CUSTOM_SIG
+    w = feature_worlds(count)
+    for _ in range(10):
+        oracle_step_batch(w, CUSTOM_SIG, 1.0 / 60.0, 4)
+    for k in range(0, count, 2):
+        for j in range(int(w["joint_count"][k])):
+            if w["joints"]["type"][k, j] == 1 and (j + k // 2) % 2:
+                w["bodies"]["rotation"]["v"]["y"][k, w["joints"]["body_b"][k, j]] = np.nan
+    return w
+
+
 def passive_hinge_worlds(count, seed=5):
     """Worlds of capacity set 16/16/32/8 for the articulated-contact path:
     a ground box, a static post with a chain of three links on passive

@@ -316,6 +316,29 @@ def test_joints_without_a_dynamic_body(kernel):
         assert len(bad) == 0, describe(bad, part, ref, worlds)
 
 
+@pytest.mark.parametrize("kernel", ["quads", "shared", "one_wave"])
+def test_nan_hinges(kernel):
+    """A NaN body's NaN reaches its hinge's impulses as in the oracle."""
+    from b3test import nan_hinge_worlds, on_shared_tiles, oracle_step_batch
+    from puffysics_amd.creation import CUSTOM_SIG
+    from puffysics_amd.engine import B3_ENGINE_KEEP_SOLVER_FIELDS, B3_ENGINE_ONE_WAVE_PER_TILE, B3Engine
+    worlds, sig = nan_hinge_worlds(70), CUSTOM_SIG
+    if kernel == "shared":
+        worlds, sig = on_shared_tiles(worlds, sig)
+    ref = clone(worlds)
+    eng = B3Engine(worlds, sig)
+    eng.set_options(B3_ENGINE_KEEP_SOLVER_FIELDS | (B3_ENGINE_ONE_WAVE_PER_TILE if kernel == "one_wave" else 0))
+    for _ in range(2):
+        oracle_step_batch(ref, sig, 1.0 / 60.0, 4)
+        eng.step(1.0 / 60.0, 4)
+    torch.cuda.synchronize()
+    got = eng.download()
+    eng.close()
+    assert np.isnan(ref["joints"]["perp_impulse"]["x"]).sum() > 4
+    bad = diff_words(got, ref, sig)
+    assert len(bad) == 0, describe(bad, got, ref, worlds)
+
+
 @pytest.mark.parametrize("kernel", ["quads", "shared-17-joints", "shared-130-tiles", "one_wave"])
 def test_bodies_whose_flag_and_type_disagree(kernel):
     """Bodies switched to kinematic by their type alone, whose velocities a

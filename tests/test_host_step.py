@@ -71,6 +71,20 @@ def test_host_step_feature_worlds():
     assert (ref["contacts_dropped"] > 0).any() and np.abs(ref["joints"]["motor_impulse"]).max() > 0
 
 
+def test_host_step_nan_hinges():
+    """A NaN body's NaN reaches its hinge's impulses as in the oracle."""
+    from b3test import nan_hinge_worlds
+    from puffysics_amd.creation import CUSTOM_SIG
+    worlds = nan_hinge_worlds(24)
+    ref = clone(worlds)
+    for _ in range(2):
+        oracle_step_batch(ref, CUSTOM_SIG, 1.0 / 60.0, 4)
+        assert _lib().b3_host_batch_step(batch_of(worlds), CUSTOM_SIG, 1.0 / 60.0, 4, None) == 1
+    assert np.isnan(ref["joints"]["perp_impulse"]["x"]).sum() > 4
+    bad = diff_words(worlds, ref, CUSTOM_SIG)
+    assert len(bad) == 0, bad[:10].tolist()
+
+
 def test_host_batch_step_strided_and_invalid_arguments():
     """Worlds embedded in larger records (stride, world_offset) step in place
     with the rest of each record untouched; invalid batches, dt, substeps or
