@@ -97,8 +97,9 @@ __device__ inline void step_world_art_wave(const Lane& L, float* ws, int* tree, 
     }
 }
 
-/* The worlds that b3k_step_art<false> handed over, one to a workgroup; 256
- * VGPRs, so that two waves share a SIMD (4,000 arm worlds 20.0 -> 11.4 ms). */
+/* The worlds that b3k_step_art<false> handed over, one to a workgroup; at
+ * most 256 VGPRs, so that two waves share a SIMD (4,000 arm worlds 20.0 ->
+ * 11.4 ms). */
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void b3k_step_art_world(uint32_t* live,
         uint32_t* worlds, uint32_t* scratch, Geometry g, int count, float dt, int substeps,
         const unsigned char* handed, unsigned int opts) {
