@@ -883,15 +883,17 @@ B3Q_FN void jq_warm(const QLane& Q, const JQ& r) {
     QVel x = qvel_load(Q, r.va, r.vb);
     x.va = x.va - qbc<3>(r.ia.x) * r.lin_imp;
     x.wa = x.wa - qmv(r.ia, qcross(r.ra, r.lin_imp) + ang);
+    float dv = qbc<3>(r.ib.x) * r.lin_imp, dw = qmv(r.ib, qcross(r.rb, r.lin_imp) + ang);
+    x.vb = x.vb + dv;
+    x.wb = x.wb + dw;
     /* a joint of a body with itself: end b moves the body from where end a
      * left it (the solves take both ends from the same state, 06:204-239
-     * against 06:436-642) */
-    if (r.va == r.vb) {
-        x.vb = x.va;
-        x.wb = x.wa;
+     * against 06:436-642).  A wave without one skips it: as selects it cost
+     * the chains 1 us of 151. */
+    if (__ballot(r.va == r.vb) && r.va == r.vb) {
+        x.vb = x.va + dv;
+        x.wb = x.wa + dw;
     }
-    x.vb = x.vb + qbc<3>(r.ib.x) * r.lin_imp;
-    x.wb = x.wb + qmv(r.ib, qcross(r.rb, r.lin_imp) + ang);
     qvel_store(Q, r.va, r.vb, r.info, x);
 }
 
